@@ -65,7 +65,7 @@ __device__ inline void ah_force(double x1, double y1, double z1, double gm1, con
 	if constexpr(kFast)
 	{
 		r2 = fmax(r2, kMinDistance);
-		coeff = div_rn(gm1 * s.w, r2 * sqrt_rn(r2));
+		coeff = pair_quot_rn((8.0 * gm1) * s.w, r2);
 	}
 	else
 	{

@@ -1,9 +1,8 @@
 // nbh_direct.hip -- direct all-pairs accelerations on gfx950.
 //
-// FP64 kernel: two targets per work-item, sources staged in LDS tiles, the
-// source loop runs in index order and each pair is evaluated with exactly the
-// operations of nbody_data::force followed by the division by m1 of
-// nbody_engine_simple::fcompute (nbody/nbody_data.cpp:35-44,
+// FP64 kernels: every target sums its sources in index order, and each pair is
+// evaluated with exactly the operations of nbody_data::force followed by the
+// division by m1 of nbody_engine_simple::fcompute (nbody/nbody_data.cpp:35-44,
 // nbody/nbody_engine_simple.cpp:152-171).  This file is compiled with
 // -ffp-contract=off, so the FP64 result equals the CPU restatement bit for bit
 // (IEEE sqrt and division are correctly rounded on both sides).
@@ -43,73 +42,103 @@ constexpr double kMinDistance = 1e-8;   // nbody/nbtype.h:79
 constexpr int kLawSimple = 0;
 constexpr int kLawBlock = 1;
 
-template <int kLaw, bool kFast>
-__device__ inline void pair64(double x1, double y1, double z1, double gm1, const double4& s, double& tx, double& ty,
-                              double& tz)
+// One term in the general sequences, for operands outside their range.
+template <int kLaw>
+__device__ inline void term64(double x1, double y1, double z1, double gm1, const double4& s, double& ux, double& uy,
+                              double& uz)
 {
 	const double dx = x1 - s.x;
 	const double dy = y1 - s.y;
 	const double dz = z1 - s.z;
 	double r2 = dx * dx + dy * dy + dz * dz;
-	double coeff;
-	if constexpr(kFast)
+	if(r2 < kMinDistance)
 	{
-		r2 = fmax(r2, kMinDistance);     // r2 is finite here: the same as the branch below
-		coeff = kLaw == kLawSimple ? div_rn(gm1 * s.w, r2 * sqrt_rn(r2)) : div_rn(s.w, sqrt_rn(r2) * r2);
+		r2 = kMinDistance;
 	}
-	else
-	{
-		if(r2 < kMinDistance)
-		{
-			r2 = kMinDistance;
-		}
-		coeff = kLaw == kLawSimple ? (gm1 * s.w) / (r2 * sqrt(r2)) : s.w / (sqrt(r2) * r2);
-	}
-	if constexpr(kLaw == kLawSimple)
-	{
-		tx += dx * coeff;
-		ty += dy * coeff;
-		tz += dz * coeff;
-	}
-	else
-	{
-		tx -= dx * coeff;
-		ty -= dy * coeff;
-		tz -= dz * coeff;
-	}
+	const double coeff = kLaw == kLawSimple ? (gm1 * s.w) / (r2 * sqrt(r2)) : s.w / (sqrt(r2) * r2);
+	ux = dx * coeff;
+	uy = dy * coeff;
+	uz = dz * coeff;
 }
 
-// kF64Tgt targets per work-item (i0 + k * blockDim.x), sources staged in LDS as
-// double4 (x, y, z, m) tiles of blockDim.x and read back as wave-wide
-// broadcasts, each reused for every target of the work-item.  The source loop
-// runs in index order.  The simple law skips the self pair in the reference;
-// here, on the fast path, it is summed: dx = dy = dz = +0 there, so its term is
-// -0 and adding -0 leaves every value (+0 included) unchanged.  The block law
-// sums it in the reference too (its term subtracts +0).  Two targets per
-// work-item when that still leaves two waves per SIMD (n >= 2^18 on 256 CUs),
-// else one, so that smaller n still spreads over every SIMD.
-template <int kLaw, int kF64Tgt>
+// N terms between targets (x1, y1, z1, gm8 = 8 gm1) and sources s, operands in
+// range, written step by step so that their chains interleave.
+template <int kLaw, int N>
+__device__ inline void terms64(const double (&x1)[N], const double (&y1)[N], const double (&z1)[N],
+                               const double (&gm8)[N], const double4 (&s)[N], double (&ux)[N], double (&uy)[N],
+                               double (&uz)[N])
+{
+	double r2[N], t[N], a8[N], q[N];
+#pragma unroll
+	for(int k = 0; k < N; ++k) { ux[k] = x1[k] - s[k].x; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { uy[k] = y1[k] - s[k].y; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { uz[k] = z1[k] - s[k].z; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { r2[k] = ux[k] * ux[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { t[k] = uy[k] * uy[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { r2[k] = r2[k] + t[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { t[k] = uz[k] * uz[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { r2[k] = r2[k] + t[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { a8[k] = kLaw == kLawSimple ? gm8[k] * s[k].w : 8.0 * s[k].w; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { r2[k] = fmax(r2[k], kMinDistance); }   // finite here: the same as the branch above
+	pair_quot_rn<N>(a8, r2, q);
+#pragma unroll
+	for(int k = 0; k < N; ++k) { ux[k] = ux[k] * q[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { uy[k] = uy[k] * q[k]; }
+#pragma unroll
+	for(int k = 0; k < N; ++k) { uz[k] = uz[k] * q[k]; }
+}
+
+template <int kLaw>
+__device__ inline void add_term(double& t, double u)
+{
+	t = kLaw == kLawSimple ? t + u : t - u;
+}
+
+// One target per work-item, sources staged in LDS as double4 (x, y, z, m) tiles
+// of blockDim.x and read back as wave-wide broadcasts, four at a time.  The
+// source loop runs in index order.  The simple law skips the self pair in the
+// reference; here, on the fast path, it is summed: dx = dy = dz = +0 there, so its
+// term is -0 and adding -0 leaves every value (+0 included) unchanged.  The block
+// law sums it in the reference too (its term subtracts +0).  FP64 issue bound:
+// 2^18 bodies in 77-85 ms, 34 FP64 operations and a v_rsq_f64 per pair at their
+// issue rate (with two targets per work-item and the chains one after the other,
+// 86-90 ms).
+template <int kLaw>
 __global__ void __launch_bounds__(1024)
 k_direct_fp64(const double* __restrict__ y, const double* __restrict__ mass, double* __restrict__ f, size_t n)
 {
+	constexpr int kN = 4;
 	extern __shared__ double4 src[];
 	const int bs = blockDim.x;
-	const size_t i0 = static_cast<size_t>(blockIdx.x) * (kF64Tgt * bs) + threadIdx.x;
-	double x1[kF64Tgt], y1[kF64Tgt], z1[kF64Tgt], m1[kF64Tgt], gm1[kF64Tgt];
-	double tx[kF64Tgt], ty[kF64Tgt], tz[kF64Tgt];
-	bool safe = true;
-	for(int k = 0; k < kF64Tgt; ++k)
+	const size_t i = static_cast<size_t>(blockIdx.x) * bs + threadIdx.x;
+	const bool active = i < n;
+	const double x1 = active ? y[i] : 0.0;
+	const double y1 = active ? y[n + i] : 0.0;
+	const double z1 = active ? y[2 * n + i] : 0.0;
+	const double m1 = active ? mass[i] : 1.0;
+	const double gm1 = -1.0 * m1;                 // (-GravityConst * mass1), G = 1
+	const double gm8 = 8.0 * gm1;
+	double tx = 0.0, ty = 0.0, tz = 0.0;
+	const bool safe = coord_in_range(x1) && coord_in_range(y1) && coord_in_range(z1) &&
+	                  (kLaw == kLawBlock || mass_in_range(m1));
+	double xn[kN], yn[kN], zn[kN], gn[kN];
+#pragma unroll
+	for(int k = 0; k < kN; ++k)
 	{
-		const size_t i = i0 + static_cast<size_t>(k) * bs;
-		const bool active = i < n;
-		x1[k] = active ? y[i] : 0.0;
-		y1[k] = active ? y[n + i] : 0.0;
-		z1[k] = active ? y[2 * n + i] : 0.0;
-		m1[k] = active ? mass[i] : 1.0;
-		gm1[k] = -1.0 * m1[k];            // (-GravityConst * mass1), G = 1
-		tx[k] = ty[k] = tz[k] = 0.0;
-		safe = safe && coord_in_range(x1[k]) && coord_in_range(y1[k]) && coord_in_range(z1[k]) &&
-		       (!active || kLaw == kLawBlock || mass_in_range(m1[k]));
+		xn[k] = x1;
+		yn[k] = y1;
+		zn[k] = z1;
+		gn[k] = gm8;
 	}
 	for(size_t base = 0; base < n; base += bs)
 	{
@@ -125,43 +154,394 @@ k_direct_fp64(const double* __restrict__ y, const double* __restrict__ mass, dou
 		src[threadIdx.x] = s;
 		const bool fast = __syncthreads_and(ok && safe) != 0;
 		const int cnt = n - base < static_cast<size_t>(bs) ? static_cast<int>(n - base) : bs;
+		int jj = 0;
 		if(fast)
 		{
-			for(int jj = 0; jj < cnt; ++jj)
+			for(; jj + kN <= cnt; jj += kN)
 			{
-				const double4 sj = src[jj];
-				for(int k = 0; k < kF64Tgt; ++k)
+				double4 sn[kN];
+				double ux[kN], uy[kN], uz[kN];
+#pragma unroll
+				for(int k = 0; k < kN; ++k) { sn[k] = src[jj + k]; }
+				terms64<kLaw, kN>(xn, yn, zn, gn, sn, ux, uy, uz);
+#pragma unroll
+				for(int k = 0; k < kN; ++k)
 				{
-					pair64<kLaw, true>(x1[k], y1[k], z1[k], gm1[k], sj, tx[k], ty[k], tz[k]);
+					add_term<kLaw>(tx, ux[k]);
+					add_term<kLaw>(ty, uy[k]);
+					add_term<kLaw>(tz, uz[k]);
+				}
+			}
+		}
+		for(; jj < cnt; ++jj)
+		{
+			if(kLaw == kLawBlock || base + jj != i)
+			{
+				double ux, uy, uz;
+				term64<kLaw>(x1, y1, z1, gm1, src[jj], ux, uy, uz);
+				add_term<kLaw>(tx, ux);
+				add_term<kLaw>(ty, uy);
+				add_term<kLaw>(tz, uz);
+			}
+		}
+	}
+	if(active)
+	{
+		f[i] = y[3 * n + i];
+		f[n + i] = y[4 * n + i];
+		f[2 * n + i] = y[5 * n + i];
+		f[3 * n + i] = kLaw == kLawSimple ? tx / m1 : tx;
+		f[4 * n + i] = kLaw == kLawSimple ? ty / m1 : ty;
+		f[5 * n + i] = kLaw == kLawSimple ? tz / m1 : tz;
+	}
+}
+
+// The same sums for bodies too few to give every CU more than one work-group:
+// there a target's chain of additions is what takes the time, and this form
+// leaves nothing else in it.  Four waves compute the terms of 16 targets for a
+// tile of 64 sources (lane = 4 sources x 16 targets, four pairs in flight) into
+// LDS; a fifth adds the previous tile's terms in source order, lane = (component,
+// target), reading 16 terms ahead, and stages and range-checks the next tile.
+// 1024 bodies take 12.7 us and 4096 44 us (99 and 392 us with a target per lane,
+// 18 and 61 us in turns, below, whose sums change hands); with more than one
+// work-group per CU its LDS traffic makes it the slower one (5000 bodies: 81 us
+// against 75).
+constexpr int kSplitTgt = 16;
+constexpr int kSplitSrc = 64;
+constexpr int kSplitWaves = 4;                              // waves that compute terms
+constexpr int kSplitPer = kSplitSrc / (4 * kSplitWaves);    // pairs per lane and tile
+constexpr int kSplitThreads = 64 * (kSplitWaves + 1);
+// one component's terms of a tile, [source][target], and half an LDS row so that
+// the adding wave's components start in different banks
+constexpr int kSplitComp = kSplitSrc * kSplitTgt + kSplitTgt;
+
+template <int kLaw>
+__global__ void __launch_bounds__(kSplitThreads)
+k_direct_fp64_split(const double* __restrict__ y, const double* __restrict__ mass, double* __restrict__ f, size_t n)
+{
+	__shared__ double4 src[2][kSplitSrc];
+	__shared__ double term[2][3 * kSplitComp];
+	__shared__ int in_range[2];
+	const int lane = threadIdx.x & 63;
+	const int wave = threadIdx.x >> 6;
+	const int t = lane & (kSplitTgt - 1);
+	const int g = lane / kSplitTgt;             // source within a group of four, or component
+	const size_t i = static_cast<size_t>(blockIdx.x) * kSplitTgt + t;
+	const bool active = i < n;
+	const size_t tiles = (n + kSplitSrc - 1) / kSplitSrc;
+	const double m1 = active ? mass[i] : 1.0;
+	if(wave == kSplitWaves)
+	{
+		__builtin_amdgcn_s_setprio(3);          // its additions are the one serial chain of the group
+		// sources beyond n: a body in range whose terms are never added
+		auto load = [&](size_t tile) {
+			const size_t j = tile * kSplitSrc + lane;
+			return j < n ? make_double4(y[j], y[n + j], y[2 * n + j], mass[j]) : make_double4(0.0, 0.0, 0.0, 1.0);
+		};
+		auto stage = [&](int b, const double4& s) {
+			const bool ok = coord_in_range(s.x) && coord_in_range(s.y) && coord_in_range(s.z) && mass_in_range(s.w);
+			const bool all = __ballot(!ok) == 0;
+			src[b][lane] = s;
+			if(lane == 0) { in_range[b] = all; }
+		};
+		const int comp = g < 3 ? g : 2;         // the last quarter of the wave repeats z and is not stored
+		double acc = 0.0;
+		stage(0, load(0));
+		double4 next = load(1);
+		__syncthreads();
+		for(size_t k = 0; k <= tiles; ++k)
+		{
+			if(k + 1 < tiles)
+			{
+				stage(static_cast<int>((k + 1) & 1), next);
+				next = load(k + 2);
+			}
+			if(k > 0)
+			{
+				const double* u = &term[(k - 1) & 1][comp * kSplitComp + t];
+				const size_t base = (k - 1) * kSplitSrc;
+				if(n - base >= static_cast<size_t>(kSplitSrc))
+				{
+					// the next 16 terms are read while the last 16 are added: left alone,
+					// the scheduler reads two ahead and every addition waits for LDS
+					constexpr int kAhead = 16;
+					double v[2][kAhead];
+#pragma unroll
+					for(int s = 0; s < kAhead; ++s) { v[0][s] = u[s * kSplitTgt]; }
+#pragma unroll
+					for(int c = 0; c < kSplitSrc / kAhead; ++c)
+					{
+						__builtin_amdgcn_sched_barrier(0);
+						if(c + 1 < kSplitSrc / kAhead)
+						{
+#pragma unroll
+							for(int s = 0; s < kAhead; ++s)
+							{
+								v[(c + 1) & 1][s] = u[((c + 1) * kAhead + s) * kSplitTgt];
+							}
+						}
+						__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+						for(int s = 0; s < kAhead; ++s) { add_term<kLaw>(acc, v[c & 1][s]); }
+					}
+				}
+				else
+				{
+					const int cnt = static_cast<int>(n - base);
+					for(int s = 0; s < cnt; ++s) { add_term<kLaw>(acc, u[s * kSplitTgt]); }
+				}
+			}
+			__syncthreads();
+		}
+		if(active && g < 3)
+		{
+			f[g * n + i] = y[(3 + g) * n + i];
+			f[(3 + g) * n + i] = kLaw == kLawSimple ? acc / m1 : acc;
+		}
+		return;
+	}
+	const double x1 = active ? y[i] : 0.0;
+	const double y1 = active ? y[n + i] : 0.0;
+	const double z1 = active ? y[2 * n + i] : 0.0;
+	const double gm1 = -1.0 * m1;               // (-GravityConst * mass1), G = 1
+	const double gm8 = 8.0 * gm1;
+	const bool safe = coord_in_range(x1) && coord_in_range(y1) && coord_in_range(z1) &&
+	                  (kLaw == kLawBlock || mass_in_range(m1));
+	const bool all_safe = __ballot(!safe) == 0;
+	const int s0 = wave * (kSplitSrc / kSplitWaves) + g;
+	__syncthreads();
+	for(size_t k = 0; k <= tiles; ++k)
+	{
+		if(k < tiles)
+		{
+			const int b = static_cast<int>(k & 1);
+			double* u = &term[b][t];
+			if(all_safe && in_range[b] != 0)
+			{
+				// all reads, then all terms, then all writes: chains do not interleave
+				// across LDS accesses
+				double xn[kSplitPer], yn[kSplitPer], zn[kSplitPer], gn[kSplitPer];
+				double ux[kSplitPer], uy[kSplitPer], uz[kSplitPer];
+				double4 sn[kSplitPer];
+#pragma unroll
+				for(int p = 0; p < kSplitPer; ++p)
+				{
+					xn[p] = x1;
+					yn[p] = y1;
+					zn[p] = z1;
+					gn[p] = gm8;
+					sn[p] = src[b][s0 + 4 * p];
+				}
+				terms64<kLaw, kSplitPer>(xn, yn, zn, gn, sn, ux, uy, uz);
+#pragma unroll
+				for(int p = 0; p < kSplitPer; ++p)
+				{
+					const int s = (s0 + 4 * p) * kSplitTgt;
+					u[s] = ux[p];
+					u[kSplitComp + s] = uy[p];
+					u[2 * kSplitComp + s] = uz[p];
+				}
+			}
+			else
+			{
+				for(int p = 0; p < kSplitPer; ++p)
+				{
+					const int s = s0 + 4 * p;
+					double ux = -0.0, uy = -0.0, uz = -0.0;      // the self pair the simple law skips: v + -0 is v
+					if(kLaw == kLawBlock || k * kSplitSrc + s != i)
+					{
+						term64<kLaw>(x1, y1, z1, gm1, src[b][s], ux, uy, uz);
+					}
+					u[s * kSplitTgt] = ux;
+					u[kSplitComp + s * kSplitTgt] = uy;
+					u[2 * kSplitComp + s * kSplitTgt] = uz;
+				}
+			}
+		}
+		__syncthreads();
+	}
+}
+
+// The same sums with the pair terms of one target spread over several waves.
+// The reference's bits need every target's terms added in index order, but only
+// the additions are ordered.  The four waves of a work-group share 32 targets
+// and take the chunks of sources in turn: a wave computes its chunk's terms into
+// registers (lane = target x set of consecutive sources, four pairs in flight),
+// then waits for the running sums, adds its terms in source order and hands the
+// sums to the next wave.  The waves fall into step one hand-over apart, so that
+// the additions of one overlap the pairs of the others.  Eight waves then share
+// the 64 targets that one wave has below: 16384 bodies take 367 us (1578 us a
+// target per lane), 20011 667 us (1924), 65536 5.5 ms (6.3); about 80 ns per pair
+// of a wave with the chip full, where issue alone takes 71.  32 targets and 16
+// pairs per lane measured best: 64 targets 432, 823 and 5.3; 8 pairs 431, 752 and
+// 6.0; 12 pairs (three work-groups per CU instead of two) 406, 681 and 5.7.
+constexpr int kTurnWaves = 4;
+constexpr int kTurnThreads = 64 * kTurnWaves;
+constexpr int kTurnTgt = 32;
+constexpr int kTurnSet = 64 / kTurnTgt;           // sets of sources per wave
+constexpr int kTurnPer = 16;                      // pairs per lane and chunk
+constexpr int kTurnSrc = kTurnSet * kTurnPer;     // sources per chunk
+
+// The value of lane l mod 32 in every lane.
+__device__ inline double low_half(double v)
+{
+	const unsigned lo = static_cast<unsigned>(__double2loint(v));
+	const unsigned hi = static_cast<unsigned>(__double2hiint(v));
+	const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+	const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+	return __hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0]));
+}
+
+template <int kLaw>
+__global__ void __launch_bounds__(kTurnThreads)
+k_direct_fp64_turns(const double* __restrict__ y, const double* __restrict__ mass, double* __restrict__ f, size_t n)
+{
+	constexpr int kIlp = 4;
+	__shared__ double4 src[kTurnWaves][kTurnSrc];    // each wave's own
+	__shared__ double sum[3][kTurnTgt];
+	__shared__ unsigned turn;                    // chunk whose terms are to be added next
+	const int lane = threadIdx.x & 63;
+	const unsigned wave = threadIdx.x >> 6;
+	const int t = lane & (kTurnTgt - 1);
+	const int set = lane / kTurnTgt;
+	const size_t i = static_cast<size_t>(blockIdx.x) * kTurnTgt + t;
+	const bool active = i < n;
+	const double x1 = active ? y[i] : 0.0;
+	const double y1 = active ? y[n + i] : 0.0;
+	const double z1 = active ? y[2 * n + i] : 0.0;
+	const double m1 = active ? mass[i] : 1.0;
+	const double gm1 = -1.0 * m1;                // (-GravityConst * mass1), G = 1
+	const double gm8 = 8.0 * gm1;
+	const bool safe = coord_in_range(x1) && coord_in_range(y1) && coord_in_range(z1) &&
+	                  (kLaw == kLawBlock || mass_in_range(m1));
+	const bool all_safe = __ballot(!safe) == 0;
+	if(threadIdx.x < kTurnTgt)
+	{
+		sum[0][threadIdx.x] = 0.0;
+		sum[1][threadIdx.x] = 0.0;
+		sum[2][threadIdx.x] = 0.0;
+	}
+	if(threadIdx.x == 0) { turn = 0; }
+	__syncthreads();
+	// sources beyond n: a body in range whose terms are not added
+	auto load = [&](size_t chunk) {
+		const size_t j = chunk * kTurnSrc + lane;
+		return lane < kTurnSrc && j < n ? make_double4(y[j], y[n + j], y[2 * n + j], mass[j]) :
+		                              make_double4(0.0, 0.0, 0.0, 1.0);
+	};
+	const unsigned chunks = static_cast<unsigned>((n + kTurnSrc - 1) / kTurnSrc);
+	double4 next = load(wave);
+	for(unsigned c = wave; c < chunks; c += kTurnWaves)
+	{
+		const bool ok = coord_in_range(next.x) && coord_in_range(next.y) && coord_in_range(next.z) &&
+		                mass_in_range(next.w);
+		const bool fast = __ballot(!ok) == 0 && all_safe;
+		if(lane < kTurnSrc) { src[wave][lane] = next; }
+		next = load(static_cast<size_t>(c) + kTurnWaves);
+		__builtin_amdgcn_wave_barrier();
+		const double4* own = &src[wave][set * kTurnPer];
+		double ux[kTurnPer], uy[kTurnPer], uz[kTurnPer];
+		if(fast)
+		{
+			double xn[kIlp], yn[kIlp], zn[kIlp], gn[kIlp], vx[kIlp], vy[kIlp], vz[kIlp];
+			double4 sn[kIlp];
+#pragma unroll
+			for(int k = 0; k < kIlp; ++k)
+			{
+				xn[k] = x1;
+				yn[k] = y1;
+				zn[k] = z1;
+				gn[k] = gm8;
+			}
+#pragma unroll
+			for(int p = 0; p < kTurnPer; p += kIlp)
+			{
+#pragma unroll
+				for(int k = 0; k < kIlp; ++k) { sn[k] = own[p + k]; }
+				terms64<kLaw, kIlp>(xn, yn, zn, gn, sn, vx, vy, vz);
+#pragma unroll
+				for(int k = 0; k < kIlp; ++k)
+				{
+					ux[p + k] = vx[k];
+					uy[p + k] = vy[k];
+					uz[p + k] = vz[k];
 				}
 			}
 		}
 		else
 		{
-			for(int jj = 0; jj < cnt; ++jj)
+#pragma unroll
+			for(int p = 0; p < kTurnPer; ++p)
 			{
-				const double4 sj = src[jj];
-				for(int k = 0; k < kF64Tgt; ++k)
+				ux[p] = uy[p] = uz[p] = -0.0;          // the self pair the simple law skips: v + -0 is v
+				if(kLaw == kLawBlock || static_cast<size_t>(c) * kTurnSrc + set * kTurnPer + p != i)
 				{
-					if(kLaw == kLawBlock || base + jj != i0 + static_cast<size_t>(k) * bs)
+					term64<kLaw>(x1, y1, z1, gm1, own[p], ux[p], uy[p], uz[p]);
+				}
+			}
+		}
+		__builtin_amdgcn_wave_barrier();
+		// every wave's turn comes: the wave whose turn it is waits for nothing
+		while(__hip_atomic_load(&turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != c)
+		{
+		}
+		__builtin_amdgcn_s_setprio(3);
+		double tx = sum[0][t], ty = sum[1][t], tz = sum[2][t];
+		const size_t base = static_cast<size_t>(c) * kTurnSrc;
+		const int cnt = n - base < static_cast<size_t>(kTurnSrc) ? static_cast<int>(n - base) : kTurnSrc;
+#pragma unroll
+		for(int h = 0; h < kTurnSet; ++h)
+		{
+			// set h adds its terms to the sums of set h - 1; the other sets' sums are not used
+			if(h > 0)
+			{
+				tx = low_half(tx);
+				ty = low_half(ty);
+				tz = low_half(tz);
+			}
+			if(cnt == kTurnSrc)
+			{
+#pragma unroll
+				for(int p = 0; p < kTurnPer; ++p)
+				{
+					add_term<kLaw>(tx, ux[p]);
+					add_term<kLaw>(ty, uy[p]);
+					add_term<kLaw>(tz, uz[p]);
+				}
+			}
+			else
+			{
+#pragma unroll
+				for(int p = 0; p < kTurnPer; ++p)
+				{
+					if(h * kTurnPer + p < cnt)
 					{
-						pair64<kLaw, false>(x1[k], y1[k], z1[k], gm1[k], sj, tx[k], ty[k], tz[k]);
+						add_term<kLaw>(tx, ux[p]);
+						add_term<kLaw>(ty, uy[p]);
+						add_term<kLaw>(tz, uz[p]);
 					}
 				}
 			}
 		}
-	}
-	for(int k = 0; k < kF64Tgt; ++k)
-	{
-		const size_t i = i0 + static_cast<size_t>(k) * bs;
-		if(i < n)
+		if(c + 1 < chunks)
+		{
+			if(set == kTurnSet - 1)
+			{
+				sum[0][t] = tx;
+				sum[1][t] = ty;
+				sum[2][t] = tz;
+			}
+			__hip_atomic_store(&turn, c + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+			__builtin_amdgcn_s_setprio(0);
+		}
+		else if(active && set == kTurnSet - 1)
 		{
 			f[i] = y[3 * n + i];
 			f[n + i] = y[4 * n + i];
 			f[2 * n + i] = y[5 * n + i];
-			f[3 * n + i] = kLaw == kLawSimple ? tx[k] / m1[k] : tx[k];
-			f[4 * n + i] = kLaw == kLawSimple ? ty[k] / m1[k] : ty[k];
-			f[5 * n + i] = kLaw == kLawSimple ? tz[k] / m1[k] : tz[k];
+			f[3 * n + i] = kLaw == kLawSimple ? tx / m1 : tx;
+			f[4 * n + i] = kLaw == kLawSimple ? ty / m1 : ty;
+			f[5 * n + i] = kLaw == kLawSimple ? tz / m1 : tz;
 		}
 	}
 }
@@ -645,33 +1025,30 @@ extern "C" nbh_status nbh_fcompute_direct(nbh_ctx* ctx, const double* y, const d
 		int bs = block_size == 0 ? 256 : block_size;
 		NBH_CHECK(bs >= 64 && bs <= 1024 && bs % 64 == 0,
 		          "block_size %d: must be a multiple of 64 in [64, 1024]", block_size);
-		// two targets per work-item when the grid still holds two waves per SIMD
-		const size_t simds = static_cast<size_t>(ctx->cu_count > 0 ? ctx->cu_count : 256) * 4;
-		const int tgt = n >= 2 * 64 * 2 * simds ? 2 : 1;
-		unsigned grid = static_cast<unsigned>((n + tgt * bs - 1) / (tgt * bs));
-		nbh::scoped_timer timer(ctx, precision == NBH_FP64 ? "direct_fp64" : "direct_fp64_block");
-		const size_t lds = bs * sizeof(double4);
-		if(precision == NBH_FP64)
+		const bool simple = precision == NBH_FP64;
+		nbh::scoped_timer timer(ctx, simple ? "direct_fp64" : "direct_fp64_block");
+		// split terms while every work-group gets a CU of its own; a target per lane
+		// once that gives every SIMD four waves (turns and a target per lane: 21.7 and
+		// 20.6 ms at 2^17, 33.2 and 36.9 at 150000, 57.7 and 63.3 at 200000, 95.8 and
+		// 84.8 at 2^18); turns between
+		const size_t cus = static_cast<size_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
+		if(n <= kSplitTgt * cus)
 		{
-			if(tgt == 2)
-			{
-				hipLaunchKernelGGL((k_direct_fp64<kLawSimple, 2>), dim3(grid), dim3(bs), lds, ctx->stream, y, mass, f, n);
-			}
-			else
-			{
-				hipLaunchKernelGGL((k_direct_fp64<kLawSimple, 1>), dim3(grid), dim3(bs), lds, ctx->stream, y, mass, f, n);
-			}
+			hipLaunchKernelGGL(simple ? k_direct_fp64_split<kLawSimple> : k_direct_fp64_split<kLawBlock>,
+			                   dim3(static_cast<unsigned>((n + kSplitTgt - 1) / kSplitTgt)), dim3(kSplitThreads), 0,
+			                   ctx->stream, y, mass, f, n);
+		}
+		else if(n < 4 * 4 * 64 * cus)
+		{
+			hipLaunchKernelGGL(simple ? k_direct_fp64_turns<kLawSimple> : k_direct_fp64_turns<kLawBlock>,
+			                   dim3(static_cast<unsigned>((n + kTurnTgt - 1) / kTurnTgt)), dim3(kTurnThreads), 0,
+			                   ctx->stream, y, mass, f, n);
 		}
 		else
 		{
-			if(tgt == 2)
-			{
-				hipLaunchKernelGGL((k_direct_fp64<kLawBlock, 2>), dim3(grid), dim3(bs), lds, ctx->stream, y, mass, f, n);
-			}
-			else
-			{
-				hipLaunchKernelGGL((k_direct_fp64<kLawBlock, 1>), dim3(grid), dim3(bs), lds, ctx->stream, y, mass, f, n);
-			}
+			hipLaunchKernelGGL(simple ? k_direct_fp64<kLawSimple> : k_direct_fp64<kLawBlock>,
+			                   dim3(static_cast<unsigned>((n + bs - 1) / bs)), dim3(bs), bs * sizeof(double4), ctx->stream,
+			                   y, mass, f, n);
 		}
 		NBH_LAUNCHED();
 		return NBH_OK;

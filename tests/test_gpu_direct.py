@@ -15,7 +15,7 @@ from nbody_amd import native, nbody_data
 
 pytestmark = pytest.mark.gpu
 
-NBH_FP64, NBH_FP32, NBH_FP32_CORR = 0, 1, 2
+NBH_FP64, NBH_FP32, NBH_FP32_CORR, NBH_FP64_BLOCK = 0, 1, 2, 3
 
 # Bounds on the relative error |a32 - a64| / |a64| of the FP32-tile kernel.
 # Sources enter as FP32 offsets from the work-group's first target and the
@@ -55,6 +55,41 @@ def test_fp64_bit_exact(ctx, n, bs):
     f = _run(ctx, y, m, NBH_FP64, bs)
     f0 = oracle_lib.fcompute_simple(y, m)
     assert np.array_equal(f, f0)
+
+
+def _edge_state(n):
+    """A ball in which some tiles hold operands outside the bare sequences' range."""
+    y, m = _state("ball", n, 5 + n)
+    if n > 70:
+        m[n // 3] = 1e-70
+        y[n - 2] = 2e6
+        y[[0, n, 2 * n]] = y[[n // 2, n + n // 2, 2 * n + n // 2]]      # a coincident pair
+    return y, m
+
+
+# edges of the FP64 direct sums: 16 targets and 64 sources (terms through LDS, up to
+# one work-group per CU: 4096 bodies on 256 CUs), 32 targets and 32 sources (turns)
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 127, 129, 4095, 4096, 4097, 4128, 4161, 6001])
+@pytest.mark.parametrize("law", [NBH_FP64, NBH_FP64_BLOCK])
+def test_fp64_bit_exact_at_tile_edges(ctx, n, law):
+    y, m = _edge_state(n)
+    f = _run(ctx, y, m, law)
+    f0 = oracle_lib.fcompute_simple(y, m, threads=0) if law == NBH_FP64 else oracle_lib.fcompute_block(y, m)
+    assert np.array_equal(f, f0)
+
+
+@pytest.mark.parametrize("n", [131071, 262143, 262144])
+def test_fp64_large_matches_sampled_targets(ctx, n):
+    """On both sides of the last switch (2^18 bodies on 256 CUs) against the
+    per-target sums of nbh_direct_sample, which keeps the same order."""
+    y, m = _state("plummer", n, 9)
+    idx = np.unique(np.concatenate([np.arange(0, n, 4099), [n - 2, n - 1]])).astype(np.uint32)
+    dy, dm, df, di, da = ctx.put(y), ctx.put(m), ctx.alloc(6 * n), ctx.put_raw(idx), ctx.alloc(3 * len(idx))
+    native.check(ctx.lib.nbh_fcompute_direct(ctx.h, dy.ptr, dm.ptr, df.ptr, n, NBH_FP64, 0), "fcompute")
+    native.check(ctx.lib.nbh_direct_sample(ctx.h, dy.ptr, dm.ptr, n, di.ptr, len(idx), da.ptr), "direct_sample")
+    f = df.read()
+    assert np.array_equal(f[3 * n:].reshape(3, n)[:, idx].T, da.read().reshape(-1, 3))
+    assert np.array_equal(f[:3 * n], y[3 * n:])
 
 
 def test_fp64_clamp_and_coincident(ctx):
