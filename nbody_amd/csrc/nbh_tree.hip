@@ -26,12 +26,12 @@
 #include <cstring>
 
 #include "nbh_common.h"
+#include "nbh_f64.h"
 #include "nbh_mlp_dev.h"
 
 namespace {
 
 constexpr int kRoot = 1;               // NBODY_HEAP_ROOT_INDEX
-constexpr int kMaxStack = 64;          // MAX_STACK_SIZE of the reference traversal
 constexpr int kSortThreads = 256;
 constexpr int kSortItems = 16;
 constexpr int kSortTile = kSortThreads * kSortItems;   // 4096 keys per work-group
@@ -1307,9 +1307,9 @@ __device__ inline void count_add(unsigned long long* counters, unsigned long lon
 	}
 }
 
-// FP64 monopole term of nbody_data::force: tot += (v1 - cm) * (-(m1 M) / r^3)
-__device__ inline void add_force64(double x1, double y1, double z1, double gm1, const double4& nd, double M,
-                                   double& tx, double& ty, double& tz)
+// FP64 monopole term of nbody_data::force: u = (v1 - cm) * (-(m1 M) / r^3)
+__device__ inline void term64(double x1, double y1, double z1, double gm1, const double4& nd, double M, double& ux,
+                              double& uy, double& uz)
 {
 	double dx = x1 - nd.x;
 	double dy = y1 - nd.y;
@@ -1317,9 +1317,9 @@ __device__ inline void add_force64(double x1, double y1, double z1, double gm1, 
 	double r2 = dx * dx + dy * dy + dz * dz;
 	if(r2 < 1e-8) { r2 = 1e-8; }
 	double coeff = (gm1 * M) / (r2 * sqrt(r2));
-	tx += dx * coeff;
-	ty += dy * coeff;
-	tz += dz * coeff;
+	ux = dx * coeff;
+	uy = dy * coeff;
+	uz = dz * coeff;
 }
 
 __device__ inline void write_f(const double* __restrict__ y, const double* __restrict__ mass, double* __restrict__ f,
@@ -1334,92 +1334,396 @@ __device__ inline void write_f(const double* __restrict__ y, const double* __res
 	f[5 * n + b] = tz / m1;
 }
 
-// nbody_space_heap_stackless::traverse (nbody_space_heap_stackless.cpp:3-26)
-__global__ void __launch_bounds__(256)
-k_bh_stackless64(const double4* __restrict__ xyzr, const double* __restrict__ nmass,
-                 const int32_t* __restrict__ body_n, const double* __restrict__ y, const double* __restrict__ mass,
-                 double* __restrict__ f, int n, unsigned long long* __restrict__ counters)
+// The FP64 walks: nbody_space_heap::traverse (nbody_space_heap.cpp:64-97) and
+// nbody_space_heap_stackless::traverse (nbody_space_heap_stackless.cpp:3-26) visit
+// a body's nodes in the same order (left subtree first) and add the accepted ones
+// in that order, so one kernel serves both layouts bit for bit.
+//
+// One wave walks for 32 neighbouring leaves at once: it visits every node that any
+// of its bodies visits (13% more nodes than one body alone at 2^17 bodies, ratio
+// 2), and a 32-bit mask says whose node it is.  What is left of the walk is a stack
+// of elements (node, bodies that take it, bodies that open it) in walk order, the
+// next one on top.  A step moves the elements at the top that nobody opens to a
+// list, then opens up to kWalkOpen nodes at once and puts what each leaves --
+// itself for its takers, its children -- in its place, in order.  One lane per
+// child decides from the bodies' box whether all of them or none pass its test
+// (four children in five); the others are tested body by body, two at a time (one
+// per half of the wave), four tests interleaved.  64
+// listed nodes at a time are evaluated: the halves take eight consecutive entries
+// each, two terms in flight (with four waves per SIMD that covers the 16 clocks of
+// a dependent FP64 operation), and then add them in list order, one half after the other; a body whose
+// mask bit is clear adds a zero.
+//
+// A body per lane, each on its own way through the tree, spent its time on gathers,
+// divergent branches and the general quotient and root: 252 us at 1024 bodies, 1.56
+// ms at 16384, 3.8 at 65536, 7.6 at 2^17 and 313 at 2^20 (ratio 2) against 90 us,
+// 0.44, 1.49, 3.9 and 72 ms.  At 2^17 bodies the VALU is then busy 62% of the time,
+// three quarters of that with the terms.  Without the box test it took 5.0 ms;
+// four terms in flight at two or three waves per SIMD 4.1 and 4.8 (spills), four
+// entries per half 4.0.
+constexpr int kWalkTgt = 32;
+constexpr int kWalkEntries = 64;
+constexpr int kWalkPer = 8;
+constexpr int kWalkIlp = 2;
+constexpr int kWalkOpen = 32;
+// Stack elements.  Opening one node at a time leaves at most three elements per
+// level (31 levels at most): that many stay in reserve, and what is above them
+// limits how many nodes open together.
+constexpr int kWalkStack64 = 400;   // with the list, 9.4 KB of LDS: 16 waves per CU
+constexpr int kWalkReserve = 3 * 33;
+
+// The value of lane l mod 32 (upper: l mod 32 + 32) in every lane.
+template <bool kUpper>
+__device__ inline double half_wave(double v)
 {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	const int tree_size = 2 * n;
-	unsigned long long inter = 0, vis = 0;
-	if(t < n)
-	{
-		const int tn = n + t;
-		const double4 me = xyzr[tn];
-		const double m1 = nmass[tn];
-		const double gm1 = -1.0 * m1;
-		double tx = 0.0, ty = 0.0, tz = 0.0;
-		int curr = kRoot;
-		do
-		{
-			const double4 nd = xyzr[curr];
-			const double dx = me.x - nd.x;
-			const double dy = me.y - nd.y;
-			const double dz = me.z - nd.z;
-			const double d2 = dx * dx + dy * dy + dz * dz;
-			++vis;
-			if(d2 > nd.w)
-			{
-				add_force64(me.x, me.y, me.z, gm1, nd, nmass[curr], tx, ty, tz);
-				++inter;
-				curr = next_down(curr);
-			}
-			else
-			{
-				curr = next_up(curr, tree_size);
-			}
-		}
-		while(curr != kRoot);
-		write_f(y, mass, f, n, body_n[tn], tx, ty, tz);
-	}
-	count_add(counters, inter, vis);
+	const unsigned lo = static_cast<unsigned>(__double2loint(v));
+	const unsigned hi = static_cast<unsigned>(__double2hiint(v));
+	const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+	const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+	return __hiloint2double(static_cast<int>(h[kUpper ? 1 : 0]), static_cast<int>(l[kUpper ? 1 : 0]));
 }
 
-// nbody_space_heap::traverse (nbody_space_heap.cpp:64-97): explicit stack, the
-// right child pushed first so the left subtree is walked first.
-__global__ void __launch_bounds__(256)
-k_bh_stack64(const double4* __restrict__ xyzr, const double* __restrict__ nmass,
-             const int32_t* __restrict__ body_n, const double* __restrict__ y, const double* __restrict__ mass,
-             double* __restrict__ f, int n, unsigned long long* __restrict__ counters)
+struct walk64_lds {
+	double4 rec[kWalkEntries];      // x, y, z, mass of the listed nodes, or records of undecided children
+	unsigned mask[kWalkEntries];
+	int list_node[2 * kWalkEntries];
+	unsigned list_mask[2 * kWalkEntries];
+	int node[kWalkStack64];
+	unsigned take[kWalkStack64];
+	unsigned open[kWalkStack64];
+	int open_node[kWalkOpen];
+	unsigned open_mask[kWalkOpen];
+	unsigned passed[2 * kWalkOpen + 8];     // bodies whose test an undecided child passes
+	uint2 child[2 * kWalkOpen];             // bodies that take / open a child
+};
+
+// The terms of entries e0 .. e0 + 2 kWalkPer - 1 of the list, added in order to the
+// sums that half kFrom of the wave holds; the other half holds them afterwards.
+template <bool kFrom>
+__device__ inline void walk64_chunk(const walk64_lds& w, int e0, int lane, const double4& me, double gm8, double& tx,
+                                    double& ty, double& tz)
 {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	const int tree_size = 2 * n;
-	unsigned long long inter = 0, vis = 0;
-	if(t < n)
+	const int t = lane & (kWalkTgt - 1);
+	const int own = e0 + ((lane >= kWalkTgt) != kFrom ? kWalkPer : 0);
+	double ux[kWalkPer], uy[kWalkPer], uz[kWalkPer];
+#pragma unroll
+	for(int p = 0; p < kWalkPer; p += kWalkIlp)
 	{
-		const int tn = n + t;
-		const double4 me = xyzr[tn];
-		const double m1 = nmass[tn];
-		const double gm1 = -1.0 * m1;
-		double tx = 0.0, ty = 0.0, tz = 0.0;
-		int stack[kMaxStack];
-		int sp = 0;
-		stack[sp++] = kRoot;
-		while(sp != 0)
+		double r2[kWalkIlp], s[kWalkIlp], q[kWalkIlp];
+		bool mine[kWalkIlp];
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k)
 		{
-			const int curr = stack[--sp];
-			const double4 nd = xyzr[curr];
-			const double dx = me.x - nd.x;
-			const double dy = me.y - nd.y;
-			const double dz = me.z - nd.z;
-			const double d2 = dx * dx + dy * dy + dz * dz;
-			++vis;
-			if(d2 > nd.w)
+			const double4 nd = w.rec[own + p + k];
+			mine[k] = (w.mask[own + p + k] >> t) & 1u;
+			ux[p + k] = me.x - nd.x;
+			uy[p + k] = me.y - nd.y;
+			uz[p + k] = me.z - nd.z;
+			s[k] = gm8 * nd.w;
+		}
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k) { r2[k] = ux[p + k] * ux[p + k]; }
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k) { q[k] = uy[p + k] * uy[p + k]; }
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k) { r2[k] = r2[k] + q[k]; }
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k) { q[k] = uz[p + k] * uz[p + k]; }
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k) { r2[k] = r2[k] + q[k]; }
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k) { r2[k] = fmax(r2[k], 1e-8); }    // finite here: the same as term64's branch
+		pair_quot_rn<kWalkIlp>(s, r2, q);
+#pragma unroll
+		for(int k = 0; k < kWalkIlp; ++k)
+		{
+			// a sum that starts at +0 is never -0, so adding a zero of either sign keeps it
+			q[k] = mine[k] ? q[k] : 0.0;
+			ux[p + k] = ux[p + k] * q[k];
+			uy[p + k] = uy[p + k] * q[k];
+			uz[p + k] = uz[p + k] * q[k];
+		}
+	}
+#pragma unroll
+	for(int h = 0; h < 2; ++h)
+	{
+		if(h == 1)
+		{
+			tx = half_wave<kFrom>(tx);
+			ty = half_wave<kFrom>(ty);
+			tz = half_wave<kFrom>(tz);
+		}
+#pragma unroll
+		for(int p = 0; p < kWalkPer; ++p)
+		{
+			tx += ux[p];
+			ty += uy[p];
+			tz += uz[p];
+		}
+	}
+}
+
+__global__ void __launch_bounds__(64, 4)
+k_bh_walk64(const double4* __restrict__ xyzr, const double* __restrict__ nmass, const int32_t* __restrict__ body_n,
+            const double* __restrict__ y, const double* __restrict__ mass, double* __restrict__ f, int n,
+            unsigned long long* __restrict__ counters)
+{
+	__shared__ walk64_lds w;
+	const int lane = threadIdx.x;
+	const int t = lane & (kWalkTgt - 1);
+	const int upper = lane / kWalkTgt;
+	// neighbouring groups on one XCD (work-groups go round robin over eight), so
+	// that its L2 serves the nodes they share
+	const unsigned groups = gridDim.x;
+	const unsigned group = groups % 8 == 0 ? (blockIdx.x % 8) * (groups / 8) + blockIdx.x / 8 : blockIdx.x;
+	const int first = static_cast<int>(group) * kWalkTgt;
+	const bool active = first + t < n;
+	const int tn = n + (active ? first + t : first);
+	const double4 me = xyzr[tn];
+	const double gm1 = -1.0 * nmass[tn];
+	const double gm8 = 8.0 * gm1;
+	const bool all_safe =
+	    __ballot(!(coord_in_range(me.x) && coord_in_range(me.y) && coord_in_range(me.z) && mass_in_range(gm1))) == 0;
+	// box of the bodies (lanes without one repeat the first); it says nothing of a
+	// body that is not a number
+	const bool box_holds = __ballot(!(me.x == me.x && me.y == me.y && me.z == me.z)) == 0;
+	double3 lo = make_double3(me.x, me.y, me.z), hi = lo;
+	for(int off = 16; off > 0; off >>= 1)
+	{
+		lo.x = fmin(lo.x, __shfl_xor(lo.x, off, 64));
+		lo.y = fmin(lo.y, __shfl_xor(lo.y, off, 64));
+		lo.z = fmin(lo.z, __shfl_xor(lo.z, off, 64));
+		hi.x = fmax(hi.x, __shfl_xor(hi.x, off, 64));
+		hi.y = fmax(hi.y, __shfl_xor(hi.y, off, 64));
+		hi.z = fmax(hi.z, __shfl_xor(hi.z, off, 64));
+	}
+	double tx = 0.0, ty = 0.0, tz = 0.0;
+	unsigned long long inter = 0, vis = 0;      // per lane
+	int count = 0, sp = 0;
+	const unsigned long long lt_mask = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+	auto below = [&](unsigned long long b) { return __popcll(b & lt_mask); };
+	auto passes = [&](const double4& nd) {
+		const double dx = me.x - nd.x;
+		const double dy = me.y - nd.y;
+		const double dz = me.z - nd.z;
+		return __ballot(dx * dx + dy * dy + dz * dz > nd.w);
+	};
+	// the first `e` <= 64 listed nodes; the list keeps the others
+	auto evaluate = [&](int e) {
+		__builtin_amdgcn_wave_barrier();
+		const int node = lane < e ? w.list_node[lane] : kRoot;
+		const unsigned mask = lane < e ? w.list_mask[lane] : 0u;
+		const double4 c = xyzr[node];
+		const double m = nmass[node];
+		const bool ok = coord_in_range(c.x) && coord_in_range(c.y) && coord_in_range(c.z) && mass_in_range(m);
+		const bool fast = __ballot(!ok) == 0 && all_safe;
+		w.rec[lane] = make_double4(c.x, c.y, c.z, m);
+		w.mask[lane] = mask;
+		if(kWalkEntries + lane < count)
+		{
+			w.list_node[lane] = w.list_node[kWalkEntries + lane];
+			w.list_mask[lane] = w.list_mask[kWalkEntries + lane];
+		}
+		__builtin_amdgcn_wave_barrier();
+		if(fast)
+		{
+			for(int k = 0; k < e; k += 4 * kWalkPer)
 			{
-				add_force64(me.x, me.y, me.z, gm1, nd, nmass[curr], tx, ty, tz);
-				++inter;
-			}
-			else
-			{
-				const int left = curr << 1;
-				const int rght = left + 1;
-				if(rght < tree_size && sp < kMaxStack) { stack[sp++] = rght; }
-				if(left < tree_size && sp < kMaxStack) { stack[sp++] = left; }
+				walk64_chunk<false>(w, k, lane, me, gm8, tx, ty, tz);
+				walk64_chunk<true>(w, k + 2 * kWalkPer, lane, me, gm8, tx, ty, tz);
 			}
 		}
-		write_f(y, mass, f, n, body_n[tn], tx, ty, tz);
+		else
+		{
+			// the general sequences, one entry at a time
+#pragma unroll 1
+			for(int k = 0; k < e; ++k)
+			{
+				if((w.mask[k] >> t) & 1u)
+				{
+					const double4 nd = w.rec[k];
+					double ux, uy, uz;
+					term64(me.x, me.y, me.z, gm1, nd, nd.w, ux, uy, uz);
+					tx += ux;
+					ty += uy;
+					tz += uz;
+				}
+			}
+		}
+		__builtin_amdgcn_wave_barrier();
+		count -= e;
+	};
+
+	{
+		const unsigned all = static_cast<unsigned>(__ballot(active));
+		const unsigned take = static_cast<unsigned>(passes(xyzr[kRoot])) & all;
+		if(lane == 0)
+		{
+			w.node[0] = kRoot;
+			w.take[0] = take;
+			w.open[0] = kRoot < n ? all & ~take : 0u;
+			vis = __popc(all);
+			inter = __popc(take);
+		}
+		sp = 1;
 	}
+	for(;;)
+	{
+		if(count >= kWalkEntries || sp == 0)
+		{
+			if(count == 0) { break; }
+			evaluate(count < kWalkEntries ? count : kWalkEntries);
+			continue;
+		}
+		__builtin_amdgcn_wave_barrier();
+		// the top of the stack in walk order, lane 0 first
+		const bool have = lane < sp;
+		const int at = have ? sp - 1 - lane : 0;
+		const int node = w.node[at];
+		const unsigned take = w.take[at];
+		const bool opened = have && w.open[at] != 0;
+		const unsigned long long opens = __ballot(opened);
+		const int seen = sp < 64 ? sp : 64;
+		// elements before the first opened one go to the list
+		const int lead = opens == 0 ? seen : __builtin_ctzll(opens);
+		if(lane < lead)
+		{
+			w.list_node[count + lane] = node;
+			w.list_mask[count + lane] = take;
+		}
+		count += lead;
+		if(opens != 0)
+		{
+			int most = (kWalkStack64 - kWalkReserve - sp) / 2;
+			most = most > kWalkOpen ? kWalkOpen : most < 1 ? 1 : most;
+			const int rank = below(opens);
+			const bool mine = opened && rank < most;
+			const int total = __popcll(opens);
+			const int used = total < most ? total : most;
+			// the window ends before the first opened element that is left for later
+			const unsigned long long later = __ballot(opened && rank >= most);
+			const int window = later == 0 ? seen : __builtin_ctzll(later);
+			if(mine)
+			{
+				w.open_node[rank] = node;
+				w.open_mask[rank] = w.open[at];
+			}
+			__builtin_amdgcn_wave_barrier();
+			const bool born = lane < 2 * used;
+			const int child = born ? 2 * w.open_node[lane >> 1] + (lane & 1) : kRoot;
+			const unsigned parents = born ? w.open_mask[lane >> 1] : 0u;
+			const double4 c = xyzr[child];
+			// the nearest and the farthest point of the bodies' box, against the test
+			// d2 > crit: rounding moves either side by less than 1e-14 of it, and 1e-300
+			// stands above what underflow can take
+			double near2 = 0.0, far2 = 0.0;
+			{
+				const double ax = lo.x - c.x, bx = c.x - hi.x;
+				const double ay = lo.y - c.y, by = c.y - hi.y;
+				const double az = lo.z - c.z, bz = c.z - hi.z;
+				const double ex = fmax(fmax(ax, bx), 0.0), ey = fmax(fmax(ay, by), 0.0), ez = fmax(fmax(az, bz), 0.0);
+				const double fx = fmax(fabs(ax), fabs(bx)), fy = fmax(fabs(ay), fabs(by)), fz = fmax(fabs(az), fabs(bz));
+				near2 = fma(ez, ez, fma(ey, ey, ex * ex));
+				far2 = fma(fz, fz, fma(fy, fy, fx * fx));
+			}
+			const bool all_pass = box_holds && far2 == far2 && fma(near2, 1.0 - 1e-12, -1e-300) > c.w;
+			const bool none_pass = box_holds && fma(far2, 1.0 + 1e-12, 1e-300) < c.w;
+			const bool undecided = born && !all_pass && !none_pass;
+			const unsigned long long und = __ballot(undecided);
+			unsigned pass = all_pass ? ~0u : 0u;
+			if(und != 0)
+			{
+				const int place = below(und);
+				const int tests = (__popcll(und) + 1) / 2;      // two children each
+				if(undecided) { w.rec[place] = c; }
+				__builtin_amdgcn_wave_barrier();
+				for(int p0 = 0; p0 < tests; p0 += 4)
+				{
+					double r[4], d[4], dy[4], dz[4];
+#pragma unroll
+					for(int k = 0; k < 4; ++k)
+					{
+						// records beyond the undecided ones are old ones; their results are not read
+						const double4 nd = w.rec[(2 * (p0 + k) + upper) & (kWalkEntries - 1)];
+						r[k] = nd.w;
+						d[k] = me.x - nd.x;
+						dy[k] = me.y - nd.y;
+						dz[k] = me.z - nd.z;
+					}
+#pragma unroll
+					for(int k = 0; k < 4; ++k) { d[k] = d[k] * d[k]; }
+#pragma unroll
+					for(int k = 0; k < 4; ++k) { dy[k] = dy[k] * dy[k]; }
+#pragma unroll
+					for(int k = 0; k < 4; ++k) { d[k] = d[k] + dy[k]; }
+#pragma unroll
+					for(int k = 0; k < 4; ++k) { dz[k] = dz[k] * dz[k]; }
+#pragma unroll
+					for(int k = 0; k < 4; ++k) { d[k] = d[k] + dz[k]; }
+					unsigned long long b[4];
+#pragma unroll
+					for(int k = 0; k < 4; ++k) { b[k] = __ballot(d[k] > r[k]); }
+					if(lane < 8)
+					{
+						const unsigned long long m = (lane & 4) ? ((lane & 2) ? b[3] : b[2]) : ((lane & 2) ? b[1] : b[0]);
+						w.passed[2 * p0 + lane] = static_cast<unsigned>(lane & 1 ? m >> 32 : m);
+					}
+				}
+				__builtin_amdgcn_wave_barrier();
+				if(undecided) { pass = w.passed[place]; }
+			}
+			if(born)
+			{
+				const unsigned taken = pass & parents;
+				w.child[lane] = make_uint2(taken, child < n ? parents & ~taken : 0u);
+				vis += __popc(parents);
+				inter += __popc(taken);
+			}
+			__builtin_amdgcn_wave_barrier();
+			// what every element of the window leaves
+			const bool stays = have && lane >= lead && lane < window && !opened;
+			uint2 l = make_uint2(0u, 0u), r = make_uint2(0u, 0u);
+			if(mine)
+			{
+				l = w.child[2 * rank];
+				r = w.child[2 * rank + 1];
+			}
+			const bool self = stays || (mine && take != 0);
+			const bool left = (l.x | l.y) != 0;
+			const bool right = (r.x | r.y) != 0;
+			const unsigned long long bs = __ballot(self), bl = __ballot(left), br = __ballot(right);
+			int pos = sp - window + __popcll(bs) + __popcll(bl) + __popcll(br);
+			sp = pos;
+			pos -= 1 + below(bs) + below(bl) + below(br);
+			__builtin_amdgcn_wave_barrier();
+			if(self)
+			{
+				w.node[pos] = node;
+				w.take[pos] = take;
+				w.open[pos] = 0;
+				--pos;
+			}
+			if(left)
+			{
+				w.node[pos] = 2 * node;
+				w.take[pos] = l.x;
+				w.open[pos] = l.y;
+				--pos;
+			}
+			if(right)
+			{
+				w.node[pos] = 2 * node + 1;
+				w.take[pos] = r.x;
+				w.open[pos] = r.y;
+			}
+		}
+		else
+		{
+			sp -= lead;
+		}
+	}
+	// the last chunk leaves the sums in the lower half
+	if(active && upper == 0) { write_f(y, mass, f, n, body_n[tn], tx, ty, tz); }
 	count_add(counters, inter, vis);
 }
 
@@ -3518,15 +3822,10 @@ nbh_status nbh_bh_fcompute(nbh_ctx* ctx, const nbh_tree* t, const double* y, con
 		hipLaunchKernelGGL(k_bh_stackless32, grid, dim3(256), 0, ctx->stream, t->xyzr, t->mass, t->body_n, y, mass,
 		                   f, n, t->counters);
 	}
-	else if(layout == NBH_LAYOUT_HEAP)
-	{
-		hipLaunchKernelGGL(k_bh_stack64, grid, dim3(256), 0, ctx->stream, t->xyzr, t->mass, t->body_n, y, mass, f,
-		                   n, t->counters);
-	}
 	else
 	{
-		hipLaunchKernelGGL(k_bh_stackless64, grid, dim3(256), 0, ctx->stream, t->xyzr, t->mass, t->body_n, y, mass,
-		                   f, n, t->counters);
+		hipLaunchKernelGGL(k_bh_walk64, dim3((n + kWalkTgt - 1) / kWalkTgt), dim3(64), 0, ctx->stream, t->xyzr, t->mass,
+		                   t->body_n, y, mass, f, n, t->counters);
 	}
 	NBH_LAUNCHED();
 	return NBH_OK;

@@ -142,6 +142,41 @@ def test_traverse_fp64_bit_exact(ctx, ratio, layout):
     t.close()
 
 
+@pytest.mark.parametrize("ratio", [0.5, 2.0, 10.0])
+@pytest.mark.parametrize("n", [1, 2, 16, 32, 64, 256, 4096, 32768])
+def test_traverse_fp64_edges_bit_exact(ctx, n, ratio):
+    """Fewer bodies than a walk's 32, one walk and several; stacks wider than the
+    walk opens at once (ratio 10); coincident bodies, a body far outside and masses
+    outside the bare quotient's range."""
+    y, m = _state("plummer", n, 40 + n)
+    if n >= 16:
+        y[[3, n + 3, 2 * n + 3]] = y[[7, n + 7, 2 * n + 7]]
+        y[5] = 3e6
+        m[n // 2] = 1e-70
+    dy, dm = ctx.put(y), ctx.put(m)
+    t = GpuTree(ctx, n)
+    t.build(dy, dm, ratio)
+    h = oracle_lib.Heap(n)
+    h.build(y, m, ratio)
+    f0 = h.fcompute(y, m, LAYOUT["heap"], 1)
+    assert np.array_equal(t.fcompute(dy, dm, LAYOUT["heap"]), f0)
+    assert np.array_equal(t.fcompute(dy, dm, LAYOUT["heap_stackless"]), f0)
+    t.close()
+
+
+def test_traverse_fp64_coincident_bodies(ctx):
+    """No node is ever taken: every body's walk reaches every leaf, and f is 0."""
+    n = 128
+    y = np.concatenate([np.full(3 * n, 0.25), np.arange(3.0 * n)])
+    dy, dm = ctx.put(y), ctx.put(np.full(n, 1.0 / n))
+    t = GpuTree(ctx, n)
+    t.build(dy, dm, 2.0)
+    f = t.fcompute(dy, dm, LAYOUT["heap_stackless"])
+    assert np.array_equal(f, np.concatenate([y[3 * n:], np.zeros(3 * n)]))
+    assert t.counters() == (0, n * (2 * n - 1))
+    t.close()
+
+
 def test_traverse_fp32_close_to_fp64(ctx):
     n = 1 << 15
     y, m = _state("plummer", n, 4)
