@@ -921,12 +921,12 @@ k_morton_keys(const double* __restrict__ y, size_t n, const double* __restrict__
 // Launch shape and scratch layout of the FP32 path for n bodies: the sources
 // are split so that the grid holds ~8 work-groups per CU; the scratch holds
 // the split partial sums, the Morton-ordered records, the sort keys / values
-// (two halves each), sort counts, scan chunk sums, bounding-box partials and
-// the box, each at a 256-byte boundary.
+// (two halves each), the sort's scratch, bounding-box partials and the box, each
+// at a 256-byte boundary.
 struct fp32_layout {
 	size_t gx, nsplit, jchunk;
 	unsigned gbox;
-	size_t off_sorted, off_keys, off_vals, off_counts, off_scan, off_bpart, off_box, bytes;
+	size_t off_sorted, off_keys, off_vals, off_counts, off_bpart, off_box, bytes;
 };
 
 fp32_layout fp32_plan(const nbh_ctx* ctx, size_t n)
@@ -948,8 +948,7 @@ fp32_layout fp32_plan(const nbh_ctx* ctx, size_t n)
 	l.off_keys = l.off_sorted + align(n * sizeof(double4));
 	l.off_vals = l.off_keys + align(2 * n * sizeof(uint64_t));
 	l.off_counts = l.off_vals + align(2 * n * sizeof(uint32_t));
-	l.off_scan = l.off_counts + align(nbh::sort_counts_size(n) * sizeof(uint32_t));
-	l.off_bpart = l.off_scan + align(nbh::sort_scan_size() * sizeof(uint32_t));
+	l.off_bpart = l.off_counts + align(nbh::sort_counts_size(n) * sizeof(uint32_t));
 	l.off_box = l.off_bpart + align(6 * static_cast<size_t>(l.gbox) * sizeof(double));
 	l.bytes = l.off_box + align(6 * sizeof(double));
 	return l;
@@ -966,7 +965,6 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	uint64_t* keys = reinterpret_cast<uint64_t*>(base + l.off_keys);
 	uint32_t* vals = reinterpret_cast<uint32_t*>(base + l.off_vals);
 	uint32_t* counts = reinterpret_cast<uint32_t*>(base + l.off_counts);
-	uint32_t* scanp = reinterpret_cast<uint32_t*>(base + l.off_scan);
 	double* bpart = reinterpret_cast<double*>(base + l.off_bpart);
 	double* box = reinterpret_cast<double*>(base + l.off_box);
 	hipLaunchKernelGGL(k_bbox_partial, dim3(l.gbox), dim3(256), 0, ctx->stream, y, n, bpart);
@@ -976,7 +974,7 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	hipLaunchKernelGGL(k_morton_keys, dim3(l.gbox), dim3(256), 0, ctx->stream, y, n, box, keys, vals);
 	NBH_LAUNCHED();
 	uint32_t* perm = nullptr;
-	NBH_TRY(nbh::sort_pairs(ctx, keys, vals, keys + n, vals + n, n, 30, counts, scanp, &perm));
+	NBH_TRY(nbh::sort_pairs(ctx, keys, vals, keys + n, vals + n, n, 30, counts, &perm));
 	hipLaunchKernelGGL(k_sorted_copy, dim3(l.gbox), dim3(256), 0, ctx->stream, y, mass, perm, sorted, n);
 	NBH_LAUNCHED();
 	{

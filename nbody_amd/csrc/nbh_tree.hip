@@ -32,9 +32,13 @@
 namespace {
 
 constexpr int kRoot = 1;               // NBODY_HEAP_ROOT_INDEX
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;
+constexpr int kSortThreads = 512;
+constexpr int kSortItems = 8;
 constexpr int kSortTile = kSortThreads * kSortItems;   // 4096 keys per work-group
+constexpr int kSortOneThreads = 1024;                  // up to 4096 keys sorted by one work-group
+constexpr int kSortOneItems = kSortTile / kSortOneThreads;
+constexpr int kSortSets = 3;                           // lists sorted together
+constexpr int kSortPasses = 8;
 constexpr int kPartThreads = 256;
 constexpr int kPartItems = 4;
 constexpr int kPartTile = kPartThreads * kPartItems;   // 1024 entries per work-group
@@ -126,35 +130,143 @@ __device__ inline uint64_t order_key(double v)
 	return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
 }
 
-__global__ void __launch_bounds__(256)
-k_make_keys(const double* __restrict__ coord, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals, size_t n)
+// The buffers of one list to be sorted: pass p reads (k, v)[p % 2] and writes the
+// other half; the last pass writes the values to `out`.
+struct sort_list {
+	uint64_t* k[2];
+	uint32_t* v[2];
+	uint32_t* out;
+};
+struct sort_lists {
+	sort_list l[kSortSets];
+};
+
+// Scratch of one list's sort, in 32-bit words: per tile and digit a 64-bit status
+// word (step << 32 | count), the counts of every digit of every pass and the
+// tickets handed out in every pass.
+struct sort_scratch {
+	unsigned long long* status;
+	uint32_t* hist;
+	uint32_t* ticket;
+};
+
+constexpr size_t sort_words(size_t tiles)
 {
-	size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride)
+	return tiles * 256 * 2 + kSortPasses * 256 + kSortPasses;
+}
+
+__device__ inline sort_scratch sort_scratch_of(uint32_t* words, int set, size_t tiles)
+{
+	uint32_t* w = words + static_cast<size_t>(set) * sort_words(tiles);
+	sort_scratch s;
+	s.status = reinterpret_cast<unsigned long long*>(w);
+	s.hist = w + tiles * 512;
+	s.ticket = s.hist + kSortPasses * 256;
+	return s;
+}
+
+// Keys and body numbers of the three coordinate lists (blockIdx.y), and their
+// sorts' scratch cleared.
+__global__ void __launch_bounds__(256)
+k_make_keys(const double* __restrict__ y, sort_lists a, size_t n, uint32_t* __restrict__ scratch, size_t words)
+{
+	const double* coord = y + static_cast<size_t>(blockIdx.y) * n;
+	uint64_t* keys = a.l[blockIdx.y].k[0];
+	uint32_t* vals = a.l[blockIdx.y].v[0];
+	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+	const size_t first = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+	for(size_t i = first; i < n; i += stride)
 	{
 		keys[i] = order_key(coord[i]);
 		vals[i] = static_cast<uint32_t>(i);
 	}
+	for(size_t i = first; i < words; i += stride) { scratch[blockIdx.y * words + i] = 0; }
 }
 
-// counts[d * nblocks + b] = number of keys of tile b with digit d
-__global__ void __launch_bounds__(kSortThreads)
-k_radix_hist(const uint64_t* __restrict__ keys, size_t n, int shift, uint32_t* __restrict__ counts, int nblocks)
+__global__ void __launch_bounds__(256)
+k_sort_clear(uint32_t* __restrict__ scratch, size_t words)
 {
-	__shared__ uint32_t hist[256];
-	hist[threadIdx.x] = 0;
+	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < words; i += stride) { scratch[i] = 0; }
+}
+
+// Counts of the digits of all passes, once over the keys (their multiset does not
+// change from pass to pass).
+__global__ void __launch_bounds__(kSortThreads)
+k_sort_hist(sort_lists a, size_t n, int passes, uint32_t* __restrict__ scratch, size_t tiles)
+{
+	__shared__ uint32_t h[kSortPasses][256];
+	const uint64_t* keys = a.l[blockIdx.y].k[0];
+	for(int i = threadIdx.x; i < passes * 256; i += kSortThreads) { (&h[0][0])[i] = 0; }
 	__syncthreads();
-	size_t base = static_cast<size_t>(blockIdx.x) * kSortTile;
-	for(int k = 0; k < kSortItems; ++k)
+	const size_t stride = static_cast<size_t>(gridDim.x) * kSortThreads;
+	for(size_t i = static_cast<size_t>(blockIdx.x) * kSortThreads + threadIdx.x; i < n; i += stride)
 	{
-		size_t i = base + static_cast<size_t>(k) * kSortThreads + threadIdx.x;
-		if(i < n)
-		{
-			atomicAdd(&hist[(keys[i] >> shift) & 0xFF], 1u);
-		}
+		const uint64_t k = keys[i];
+		for(int p = 0; p < passes; ++p) { atomicAdd(&h[p][(k >> (8 * p)) & 0xFF], 1u); }
 	}
 	__syncthreads();
-	counts[static_cast<size_t>(threadIdx.x) * nblocks + blockIdx.x] = hist[threadIdx.x];
+	const sort_scratch s = sort_scratch_of(scratch, blockIdx.y, tiles);
+	for(int i = threadIdx.x; i < passes * 256; i += kSortThreads)
+	{
+		const uint32_t c = (&h[0][0])[i];
+		if(c != 0) { atomicAdd(&s.hist[i], c); }
+	}
+}
+
+// Exclusive prefix sum over the first 256 work-items of a group (the others pass
+// anything); ws: four words of LDS.
+__device__ inline uint32_t scan256(uint32_t v, uint32_t* ws)
+{
+	const int lane = threadIdx.x & 63;
+	const int wave = threadIdx.x >> 6;
+	uint32_t x = v;
+	for(int off = 1; off < 64; off <<= 1)
+	{
+		const uint32_t u = __shfl_up(x, off, 64);
+		if(lane >= off) { x += u; }
+	}
+	if(lane == 63 && wave < 4) { ws[wave] = x; }
+	__syncthreads();
+	uint32_t ex = x - v;
+	for(int w = 0; w < 4; ++w) { ex += w < wave ? ws[w] : 0; }
+	__syncthreads();
+	return ex;
+}
+
+// The lanes of the wave whose digit equals this one's.
+__device__ inline uint64_t digit_peers(uint32_t d, bool ok)
+{
+	uint64_t peers = __ballot(ok);
+#pragma unroll
+	for(int bit = 0; bit < 8; ++bit)
+	{
+		const uint64_t bal = __ballot((d >> bit) & 1u);
+		peers &= ((d >> bit) & 1u) ? bal : ~bal;
+	}
+	return peers;
+}
+
+// Ranks a tile's keys stably by digit, each wave its own run of keys with its own
+// counters (no work-group synchronisation between rows): rank[] within the wave's
+// keys of that digit.  counts[wave][256] end as the waves' digit counts.
+template <int kItems>
+__device__ inline void rank_tile(const uint64_t (&key)[kItems], const bool (&ok)[kItems], int shift,
+                                 uint32_t* __restrict__ counts, uint32_t (&rank)[kItems])
+{
+	const int lane = threadIdx.x & 63;
+	const uint64_t lt_mask = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+#pragma unroll
+	for(int k = 0; k < kItems; ++k)
+	{
+		const uint32_t d = static_cast<uint32_t>((key[k] >> shift) & 0xFF);
+		const uint64_t peers = digit_peers(d, ok[k]);
+		const uint32_t before = ok[k] ? counts[d] : 0;
+		rank[k] = before + static_cast<uint32_t>(__popcll(peers & lt_mask));
+		__builtin_amdgcn_wave_barrier();
+		if(ok[k] && (peers & lt_mask) == 0) { counts[d] = before + static_cast<uint32_t>(__popcll(peers)); }
+		__builtin_amdgcn_wave_barrier();
+	}
 }
 
 // Exclusive scan in place of `m` uint32 counts: chunk sums, a scan of the (at
@@ -272,88 +384,203 @@ k_scan_one(uint32_t* __restrict__ c, int m)
 	}
 }
 
-// Stable scatter of one 4096-key tile: rows of 256 keys are ranked in index
-// order, wave by wave, with a ballot match on the 8 digit bits, and placed in
-// LDS in digit order; the tile then leaves as one contiguous run per digit.
-// `offsets` is the exclusive scan (digit-major) of the per-tile digit counts,
-// so a tile's count of digit d is the next entry minus its own (n after the
-// last).
+// One pass of the sort in one launch: a tile ranks its keys, publishes its digit
+// counts, sums the counts of the tiles before it from their status words (the sums
+// of a tile that has done so itself end the search) and writes its keys out, one
+// contiguous run per digit.  Tiles are numbered by ticket, so every tile before one
+// that waits has started; it publishes its counts before it waits for any other,
+// so every wait ends.  A pass's words carry its number: those of the passes before
+// read as not there yet.  Latency bound below some 2^19 keys: with a histogram, a
+// scan and a scatter with a work-group barrier per row of keys for every pass, list
+// by list, the heap build of 2^17 bodies took 1065 us (24 passes of 31 us), now 366
+// us, and the Morton build of 2^22 bodies 1.96 ms, now 1.70.
 __global__ void __launch_bounds__(kSortThreads)
-k_radix_scatter(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, size_t n, int shift,
-                const uint32_t* __restrict__ offsets, int nblocks)
+k_sort_pass(sort_lists a, size_t n, int pass, int last, int keep_keys, uint32_t* __restrict__ scratch, size_t tiles)
 {
 	constexpr int kWaves = kSortThreads / 64;
+	constexpr int kLook = 8;                // status words read at a time
 	__shared__ uint64_t skey[kSortTile];
 	__shared__ uint32_t sval[kSortTile];
-	__shared__ uint32_t goff[256];     // first output position of digit d for this tile
-	__shared__ uint32_t loff[256];     // first LDS position of digit d
-	__shared__ uint32_t running[256];  // keys of digit d placed so far
-	__shared__ uint32_t wcount[kWaves][256];
-	__shared__ uint32_t wsum[kWaves];
-	const int lane = threadIdx.x & 63;
-	const int wave = threadIdx.x >> 6;
-	const size_t base = static_cast<size_t>(blockIdx.x) * kSortTile;
+	__shared__ uint32_t counts[kWaves][256];
+	__shared__ uint32_t goff[256];          // output position of the tile's first key of a digit, minus its place in LDS
+	__shared__ uint32_t loff[256];          // place of that key in LDS
+	__shared__ uint32_t ws[4];
+	__shared__ uint32_t my_tile;
+	const sort_scratch s = sort_scratch_of(scratch, blockIdx.y, tiles);
+	const sort_list& l = a.l[blockIdx.y];
+	const uint64_t* kin = l.k[pass & 1];
+	const uint32_t* vin = l.v[pass & 1];
+	uint64_t* kout = l.k[(pass & 1) ^ 1];
+	uint32_t* vout = last ? l.out : l.v[(pass & 1) ^ 1];
+	const int shift = 8 * pass;
+	if(threadIdx.x == 0) { my_tile = atomicAdd(&s.ticket[pass], 1u); }
+	for(int i = threadIdx.x; i < kWaves * 256; i += kSortThreads) { (&counts[0][0])[i] = 0; }
+	__syncthreads();
+	const uint32_t tile = my_tile;
+	const size_t base = static_cast<size_t>(tile) * kSortTile;
 	const int tcount = n - base < static_cast<size_t>(kSortTile) ? static_cast<int>(n - base) : kSortTile;
-	{
-		const size_t idx = static_cast<size_t>(threadIdx.x) * nblocks + blockIdx.x;
-		const uint32_t g0 = offsets[idx];
-		const size_t m = static_cast<size_t>(nblocks) * 256;
-		const uint32_t cnt = (idx + 1 < m ? offsets[idx + 1] : static_cast<uint32_t>(n)) - g0;
-		goff[threadIdx.x] = g0;
-		running[threadIdx.x] = 0;
-		uint32_t x = cnt;
-		for(int off = 1; off < 64; off <<= 1)
-		{
-			const uint32_t u = __shfl_up(x, off, 64);
-			if(lane >= off) { x += u; }
-		}
-		if(lane == 63) { wsum[wave] = x; }
-		__syncthreads();
-		uint32_t ex = x - cnt;
-		for(int w = 0; w < wave; ++w) { ex += wsum[w]; }
-		loff[threadIdx.x] = ex;
-	}
-	const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+	const int wave = threadIdx.x >> 6;
+	const int first = wave * (64 * kSortItems) + (threadIdx.x & 63);
+	uint64_t key[kSortItems];
+	uint32_t val[kSortItems], rank[kSortItems];
+	bool ok[kSortItems];
+#pragma unroll
 	for(int k = 0; k < kSortItems; ++k)
 	{
-		for(int w = 0; w < kWaves; ++w) { wcount[w][threadIdx.x] = 0; }
-		__syncthreads();
-		const int r = k * kSortThreads + threadIdx.x;
-		const bool ok = r < tcount;
-		const uint64_t key = ok ? kin[base + r] : 0;
-		const uint32_t val = ok ? vin[base + r] : 0;
-		const uint32_t d = static_cast<uint32_t>((key >> shift) & 0xFF);
-		uint64_t peers = __ballot(ok);
-		for(int bit = 0; bit < 8; ++bit)
+		const int r = first + 64 * k;
+		ok[k] = r < tcount;
+		key[k] = ok[k] ? kin[base + r] : 0;
+		val[k] = ok[k] ? vin[base + r] : 0;
+	}
+	rank_tile<kSortItems>(key, ok, shift, counts[wave], rank);
+	__syncthreads();
+	const bool digit = threadIdx.x < 256;
+	uint32_t total = 0;
+	if(digit)
+	{
+		for(int w = 0; w < kWaves; ++w)
 		{
-			const uint64_t bal = __ballot((d >> bit) & 1u);
-			peers &= ((d >> bit) & 1u) ? bal : ~bal;
+			const uint32_t c = counts[w][threadIdx.x];
+			counts[w][threadIdx.x] = total;
+			total += c;
 		}
-		const uint32_t rank = static_cast<uint32_t>(__popcll(peers & lt_mask));
-		const uint32_t cnt = static_cast<uint32_t>(__popcll(peers));
-		if(ok && (peers & lt_mask) == 0) { wcount[wave][d] = cnt; }
-		__syncthreads();
-		if(ok)
+		const unsigned long long tag = tile == 0 ? 2 * pass + 2 : 2 * pass + 1;
+		__hip_atomic_store(&s.status[static_cast<size_t>(tile) * 256 + threadIdx.x], tag << 32 | total,
+		                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
+	const uint32_t place = scan256(total, ws);
+	const uint32_t start = scan256(digit ? s.hist[pass * 256 + threadIdx.x] : 0, ws);
+	if(digit) { loff[threadIdx.x] = place; }
+	__syncthreads();
+#pragma unroll
+	for(int k = 0; k < kSortItems; ++k)
+	{
+		if(ok[k])
 		{
-			uint32_t pos = loff[d] + running[d] + rank;
-			for(int w = 0; w < wave; ++w) { pos += wcount[w][d]; }
-			skey[pos] = key;
-			sval[pos] = val;
+			const uint32_t d = static_cast<uint32_t>((key[k] >> shift) & 0xFF);
+			const uint32_t pos = loff[d] + counts[wave][d] + rank[k];
+			skey[pos] = key[k];
+			sval[pos] = val[k];
 		}
-		__syncthreads();
-		uint32_t add = 0;
-		for(int w = 0; w < kWaves; ++w) { add += wcount[w][threadIdx.x]; }
-		running[threadIdx.x] += add;
+	}
+	if(digit)
+	{
+		uint32_t before = 0;
+		const unsigned long long part = 2 * pass + 1, sum = 2 * pass + 2;
+		long long t = static_cast<long long>(tile) - 1;
+		while(t >= 0)
+		{
+			unsigned long long v[kLook];
+#pragma unroll
+			for(int k = 0; k < kLook; ++k)
+			{
+				v[k] = t - k >= 0 ? __hip_atomic_load(&s.status[static_cast<size_t>(t - k) * 256 + threadIdx.x],
+				                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+				                  : sum << 32;
+			}
+			bool open = true;
+			int used = 0;
+#pragma unroll
+			for(int k = 0; k < kLook; ++k)
+			{
+				const unsigned long long tag = v[k] >> 32;
+				if(open && (tag == part || tag == sum))
+				{
+					before += static_cast<uint32_t>(v[k]);
+					++used;
+					open = tag == part;
+					if(tag == sum) { t = -1; }
+				}
+				else
+				{
+					open = false;
+				}
+			}
+			if(t >= 0) { t -= used; }
+		}
+		if(tile != 0)
+		{
+			__hip_atomic_store(&s.status[static_cast<size_t>(tile) * 256 + threadIdx.x], sum << 32 | (before + total),
+			                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		}
+		goff[threadIdx.x] = start + before - place;
 	}
 	__syncthreads();
 	for(int i = threadIdx.x; i < tcount; i += kSortThreads)
 	{
-		const uint64_t key = skey[i];
-		const uint32_t d = static_cast<uint32_t>((key >> shift) & 0xFF);
-		const size_t pos = static_cast<size_t>(goff[d]) + static_cast<uint32_t>(i - static_cast<int>(loff[d]));
-		kout[pos] = key;
+		const uint64_t k = skey[i];
+		const uint32_t pos = goff[(k >> shift) & 0xFF] + static_cast<uint32_t>(i);
+		if(keep_keys || !last) { kout[pos] = k; }
 		vout[pos] = sval[i];
+	}
+}
+
+// All passes over at most kSortTile keys by one work-group per list, in LDS.
+__global__ void __launch_bounds__(kSortOneThreads)
+k_sort_one(sort_lists a, int n, int passes, int keep_keys)
+{
+	constexpr int kWaves = kSortOneThreads / 64;
+	__shared__ uint64_t skey[kSortTile];
+	__shared__ uint32_t sval[kSortTile];
+	__shared__ uint32_t counts[kWaves][256];
+	__shared__ uint32_t loff[256];
+	__shared__ uint32_t ws[4];
+	const sort_list& l = a.l[blockIdx.y];
+	const int wave = threadIdx.x >> 6;
+	const int first = wave * (64 * kSortOneItems) + (threadIdx.x & 63);
+	for(int i = threadIdx.x; i < n; i += kSortOneThreads)
+	{
+		skey[i] = l.k[0][i];
+		sval[i] = l.v[0][i];
+	}
+	for(int pass = 0; pass < passes; ++pass)
+	{
+		const int shift = 8 * pass;
+		for(int i = threadIdx.x; i < kWaves * 256; i += kSortOneThreads) { (&counts[0][0])[i] = 0; }
+		__syncthreads();
+		uint64_t key[kSortOneItems];
+		uint32_t val[kSortOneItems], rank[kSortOneItems];
+		bool ok[kSortOneItems];
+#pragma unroll
+		for(int k = 0; k < kSortOneItems; ++k)
+		{
+			const int r = first + 64 * k;
+			ok[k] = r < n;
+			key[k] = ok[k] ? skey[r] : 0;
+			val[k] = ok[k] ? sval[r] : 0;
+		}
+		rank_tile<kSortOneItems>(key, ok, shift, counts[wave], rank);
+		__syncthreads();
+		uint32_t total = 0;
+		if(threadIdx.x < 256)
+		{
+			for(int w = 0; w < kWaves; ++w)
+			{
+				const uint32_t c = counts[w][threadIdx.x];
+				counts[w][threadIdx.x] = total;
+				total += c;
+			}
+		}
+		const uint32_t place = scan256(total, ws);
+		if(threadIdx.x < 256) { loff[threadIdx.x] = place; }
+		__syncthreads();
+#pragma unroll
+		for(int k = 0; k < kSortOneItems; ++k)
+		{
+			if(ok[k])
+			{
+				const uint32_t d = static_cast<uint32_t>((key[k] >> shift) & 0xFF);
+				const uint32_t pos = loff[d] + counts[wave][d] + rank[k];
+				skey[pos] = key[k];
+				sval[pos] = val[k];
+			}
+		}
+		__syncthreads();
+	}
+	for(int i = threadIdx.x; i < n; i += kSortOneThreads)
+	{
+		if(keep_keys) { l.k[passes & 1][i] = skey[i]; }
+		l.out[i] = sval[i];
 	}
 }
 
@@ -3329,17 +3556,66 @@ nbh_status scan_exclusive(nbh_ctx* ctx, uint32_t* c, size_t m, uint32_t* scan_pa
 	return NBH_OK;
 }
 
-nbh_status radix_sort(nbh_ctx* ctx, nbh_tree* t, const double* coord, uint32_t* out_vals)
+// Sorts `sets` lists whose keys, values and cleared scratch (sort_words each) are
+// in place.
+nbh_status sort_run(nbh_ctx* ctx, const sort_lists& a, int sets, size_t n, int passes, bool keep_keys,
+                    uint32_t* scratch)
+{
+	const unsigned ys = static_cast<unsigned>(sets);
+	if(n <= static_cast<size_t>(kSortTile))
+	{
+		hipLaunchKernelGGL(k_sort_one, dim3(1, ys), dim3(kSortOneThreads), 0, ctx->stream, a, static_cast<int>(n),
+		                   passes, keep_keys ? 1 : 0);
+		NBH_LAUNCHED();
+		return NBH_OK;
+	}
+	const size_t tiles = (n + kSortTile - 1) / kSortTile;
+	hipLaunchKernelGGL(k_sort_hist, dim3(static_cast<unsigned>(std::min<size_t>(tiles, 512)), ys), dim3(kSortThreads),
+	                   0, ctx->stream, a, n, passes, scratch, tiles);
+	NBH_LAUNCHED();
+	for(int p = 0; p < passes; ++p)
+	{
+		hipLaunchKernelGGL(k_sort_pass, dim3(static_cast<unsigned>(tiles), ys), dim3(kSortThreads), 0, ctx->stream, a, n,
+		                   p, p + 1 == passes ? 1 : 0, keep_keys ? 1 : 0, scratch, tiles);
+		NBH_LAUNCHED();
+	}
+	return NBH_OK;
+}
+
+// The bodies in x, y and z order: t->list[0..2].  The three sorts run together;
+// their keys and values take the walk records' space, which the build writes
+// after them (record 0, which no build writes, stays).
+nbh_status sort_axes(nbh_ctx* ctx, nbh_tree* t, const double* y)
 {
 	const size_t n = t->n;
-	hipLaunchKernelGGL(k_make_keys, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, coord, t->keys,
-	                   t->vals, n);
+	if(n == 1)
+	{
+		for(int a = 0; a < 3; ++a)
+		{
+			hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, reinterpret_cast<int*>(t->list[a]),
+			                   static_cast<size_t>(1), 0);
+			NBH_LAUNCHED();
+		}
+		return NBH_OK;
+	}
+	static_assert(sizeof(nbh_walk_rec) * 3 >= 3 * 2 * 2 * (sizeof(uint64_t) + sizeof(uint32_t)), "n = 2 fits");
+	sort_lists a;
+	uint64_t* keys = reinterpret_cast<uint64_t*>(t->wrec + 1);
+	uint32_t* vals = reinterpret_cast<uint32_t*>(keys + 6 * n);
+	for(int d = 0; d < 3; ++d)
+	{
+		for(int h = 0; h < 2; ++h)
+		{
+			a.l[d].k[h] = keys + (2 * d + h) * n;
+			a.l[d].v[h] = vals + (2 * d + h) * n;
+		}
+		a.l[d].out = t->list[d];
+	}
+	const size_t words = sort_words((n + kSortTile - 1) / kSortTile);
+	hipLaunchKernelGGL(k_make_keys, dim3(nbh::grid_for(ctx, n, 256), 3), dim3(256), 0, ctx->stream, y, a, n, t->counts,
+	                   words);
 	NBH_LAUNCHED();
-	uint32_t* sorted = nullptr;
-	NBH_TRY(nbh::sort_pairs(ctx, t->keys, t->vals, t->keys + n, t->vals + n, n, 64, t->counts, t->scan_part,
-	                        &sorted));
-	NBH_HIP(hipMemcpyAsync(out_vals, sorted, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, ctx->stream));
-	return NBH_OK;
+	return sort_run(ctx, a, 3, n, 8, false, t->counts);
 }
 
 // Packed walk records of nodes 1 .. count-1.
@@ -3389,30 +3665,23 @@ nbh_status moments(nbh_ctx* ctx, nbh_tree* t, const double* y, const double* mas
 
 namespace nbh {
 
-size_t sort_counts_size(size_t n)
-{
-	return ((n + kSortTile - 1) / kSortTile) * 256 + 1;
-}
-
-size_t sort_scan_size() { return kScanParts; }
+size_t sort_counts_size(size_t n) { return sort_words((n + kSortTile - 1) / kSortTile); }
 
 nbh_status sort_pairs(nbh_ctx* ctx, uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, int bits,
-                      uint32_t* counts, uint32_t* scan_part, uint32_t** sorted_vals)
+                      uint32_t* counts, uint32_t** sorted_vals)
 {
-	const int nblocks = static_cast<int>((n + kSortTile - 1) / kSortTile);
-	for(int shift = 0; shift < bits; shift += 8)
+	const int passes = (bits + 7) / 8;
+	uint32_t* out = passes % 2 == 0 ? v0 : v1;
+	sort_lists a = {};
+	a.l[0] = {{k0, k1}, {v0, v1}, out};
+	const size_t words = sort_counts_size(n);
+	if(n > static_cast<size_t>(kSortTile))
 	{
-		hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortThreads), 0, ctx->stream, k0, n, shift, counts,
-		                   nblocks);
+		hipLaunchKernelGGL(k_sort_clear, dim3(grid_for(ctx, words, 256)), dim3(256), 0, ctx->stream, counts, words);
 		NBH_LAUNCHED();
-		NBH_TRY(scan_exclusive(ctx, counts, static_cast<size_t>(nblocks) * 256, scan_part));
-		hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kSortThreads), 0, ctx->stream, k0, v0, k1, v1, n,
-		                   shift, counts, nblocks);
-		NBH_LAUNCHED();
-		std::swap(k0, k1);
-		std::swap(v0, v1);
 	}
-	*sorted_vals = v0;
+	NBH_TRY(sort_run(ctx, a, 1, n, passes, true, counts));
+	*sorted_vals = out;
 	return NBH_OK;
 }
 
@@ -3425,8 +3694,8 @@ constexpr int kTreeBuffers = 17;
 static void tree_buffers(nbh_tree* t, void** ptrs[kTreeBuffers], size_t sizes[kTreeBuffers])
 {
 	const size_t n = t->n;
-	const size_t nb = (n + kSortTile - 1) / kSortTile;
-	const size_t ncounts = std::max(nb * 256, (n + kPartTile - 1) / kPartTile) + 1;
+	const size_t ncounts = std::max(kSortSets * sort_words((n + kSortTile - 1) / kSortTile),
+	                                (n + kPartTile - 1) / kPartTile) + 1;
 	int k = 0;
 	auto add = [&](void* p, size_t bytes) {
 		ptrs[k] = static_cast<void**>(p);
@@ -3625,7 +3894,7 @@ nbh_status nbh_tree_build_radix(nbh_ctx* ctx, nbh_tree* t, const double* y, cons
 	NBH_LAUNCHED();
 	uint32_t* order = nullptr;
 	// 63-bit keys: 8 passes, so the sorted keys end where they started
-	NBH_TRY(nbh::sort_pairs(ctx, t->keys, t->vals, t->keys + n, t->vals + n, n, 63, t->counts, t->scan_part, &order));
+	NBH_TRY(nbh::sort_pairs(ctx, t->keys, t->vals, t->keys + n, t->vals + n, n, 63, t->counts, &order));
 	const unsigned gn = nbh::grid_for(ctx, 2 * n, 256);
 	hipLaunchKernelGGL(k_fill_int, dim3(gn), dim3(256), 0, ctx->stream, t->parent, 2 * n, 0);
 	NBH_LAUNCHED();
@@ -3734,10 +4003,7 @@ nbh_status nbh_tree_build(nbh_ctx* ctx, nbh_tree* t, const double* y, const doub
 	nbh::scoped_timer timer(ctx, "tree_build");
 	const size_t n = t->n;
 	t->radix = false;
-	for(int a = 0; a < 3; ++a)
-	{
-		NBH_TRY(radix_sort(ctx, t, y + static_cast<size_t>(a) * n, t->list[a]));
-	}
+	NBH_TRY(sort_axes(ctx, t, y));
 	const size_t ntiles = (n + kPartTile - 1) / kPartTile;
 	// the last levels (segments of at most kLocalSeg bodies) run in LDS
 	const int local_levels = std::min(t->levels, 12);

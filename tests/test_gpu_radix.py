@@ -104,6 +104,18 @@ def test_radix_build_bit_exact(ctx, kind, n, seed):
     t.close()
 
 
+@pytest.mark.parametrize("kind", ["plummer", "coincident"])
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 8191, 8193, 36865, 70001])
+def test_radix_sort_tile_edges(ctx, kind, n):
+    """Body order on both sides of one 4096-key tile (one work-group sorts it all),
+    with a last tile of one key, and with more tiles than are looked back over at a
+    time (8); equal keys keep body order."""
+    y, m = _state(kind, n, n)
+    t = RTree(ctx, y, m, 1.6)
+    assert np.array_equal(t.arrays()["body"][n:], oracle_lib.radix_build(y, m, 1.6)["order"].astype(np.int32))
+    t.close()
+
+
 @pytest.mark.parametrize("kind,n,seed", [("plummer", 3, 8), ("plummer", 100, 10), ("plummer", 3000, 2),
                                          ("plummer", 1 << 15, 5), ("coincident", 2500, 6)])
 def test_radix_lean_walks_equal(ctx, kind, n, seed):
