@@ -33,7 +33,7 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "pair-interactions/s (direct); BH steps/s at N=4M, force err ≤1e-3 vs FP64"
 FLOP_PER_PAIR = 20.0
-VALU_PER_PAIR = 13           # inner loop of k_direct_fp32 per pair (12 VALU + v_rsq_f32 with clamp)
+VALU_PER_PAIR = 8.5          # inner loop of k_direct_fp32_sym: 16 VALU + v_rsq_f32 with clamp for both bodies of a pair
 PEAK_FP32_TFLOPS = 157.3
 
 
@@ -874,7 +874,7 @@ def main(argv=None) -> int:
             "avg_kernel_ms": avg_ms,
             "launches": cnt.value,
             "pairs_per_s_kernel": n * n / (avg_ms * 1e-3),
-            # issued instructions: 12 VALU + 1 v_rsq_f32 per pair against the
+            # issued instructions: 16 VALU + 1 v_rsq_f32 per two pairs against the
             # 157.3e12 / 2 lane-instructions/s behind the FP32 peak, and as wave
             # instructions per SIMD per clock (256 CUs x 4 SIMDs, 2.4 GHz)
             "valu_instr_per_pair": VALU_PER_PAIR,

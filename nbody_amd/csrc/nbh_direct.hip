@@ -8,18 +8,15 @@
 // (IEEE sqrt and division are correctly rounded on both sides).
 //
 // FP32 kernel (the throughput path): the bodies are sorted along a Morton curve
-// and copied once into records (x, y, z, m) in that order; each work-group owns
-// 256*TGT consecutive targets and a slice of the sources.  Sources are converted
-// once per work-group from FP64 to FP32 coordinates relative to the
-// work-group's origin (the FP64 position of its first target), staged in LDS as
-// float4 (x, y, z, m) and read back as wave-wide broadcasts; each work-item
-// reuses every source for TGT targets held in registers.  Per pair: 3 sub,
-// 3 mul/fma for r^2, 1 v_rsq_f32 whose output clamp is the reference's
-// r^2 >= 1e-8 clamp (in scaled units), 3 mul, 3 fma.  Partial sums of
-// one LDS tile stay in FP32 and are folded into a Kahan (summation_k) FP32
-// accumulator per tile; the source slices are then added in FP64 in a fixed
-// order by a second kernel, which also copies the velocities into f[0:3n].
+// and copied once into records (x, y, z, m) in that order; blocks of consecutive
+// bodies meet pairwise, and every pair is evaluated once for both its bodies.
+// Coordinates are FP32 offsets from the FP64 position of a body close to one of the
+// two.  Per pair: 3 sub, 3 mul/fma for r^2, 1 v_rsq_f32 whose output clamp is the
+// reference's r^2 >= 1e-8 clamp (in scaled units), 4 mul and 6 fma.  Partial sums
+// stay in FP32 over 64 terms; a second kernel adds the blocks' sums in FP64 in a
+// fixed order and copies the velocities into f[0:3n].
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -603,10 +600,7 @@ k_direct_sample64(const double* __restrict__ y, const double* __restrict__ mass,
 // ---------------------------------------------------------------------------
 // FP32 tiles
 // ---------------------------------------------------------------------------
-constexpr int kF32Threads = 256;   // work-items per work-group (4 waves)
-constexpr int kF32Tgt = 4;         // targets per work-item
-constexpr int kF32Tile = 256;      // sources per LDS tile (one per work-item)
-constexpr int kF32TgtPerGroup = kF32Threads * kF32Tgt;
+constexpr int kF32Group = 1024;    // bodies that share an origin
 
 // The tiles work in scaled units: offsets x' = 1e4 x and masses m' = 1e8 m (both
 // formed in FP64 and rounded once).  Then r'^2 = 1e8 r^2, and the reference's
@@ -621,14 +615,6 @@ constexpr double kF32Mass = 1e8;
 __device__ inline float rsq_clamped(float r2)
 {
 	return __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(r2), 0.0f, 1.0f);   // folds into v_rsq_f32 clamp
-}
-
-__device__ inline void kahan_f32(float& s, float& c, float v)
-{
-	float corrected = v - c;
-	float ns = s + corrected;
-	c = (ns - s) - corrected;
-	s = ns;
 }
 
 // The state in Morton order as one record per body: sorted[p] = (x, y, z, m) of
@@ -647,99 +633,260 @@ k_sorted_copy(const double* __restrict__ y, const double* __restrict__ mass, con
 	}
 }
 
-// part: [nsplit][3][n] doubles by Morton position, slice blockIdx.y of the
-// sources (also in Morton order).  A work-group's 1024 targets are consecutive
-// along the curve, so they are close together and their offsets from its
-// origin (its first target) -- and those of the sources near them -- are
-// small in FP32.
-__global__ void __launch_bounds__(kF32Threads)
-k_direct_fp32(const double4* __restrict__ sorted, double* __restrict__ part, size_t n, size_t jchunk)
+// A pair's offset, r^2 and v_rsq_f32 serve both bodies.  The bodies, in Morton
+// order, form nb blocks of kB = 256 kT; a work-group keeps block I in registers
+// (kT bodies per lane) and takes the blocks J = I + d, d = 1 .. nb / 2 (mod nb;
+// for even nb the last d only for I < nb / 2), so that every two blocks meet once,
+// and its own block (d = 0) pair by ordered pair.  A wave takes 64 bodies of J at a
+// time: lane l works on body l + k in step k, k = 0 .. 63, and the sums of what
+// that body receives move with it from lane to lane (one DPP rotation per step and
+// component, folded into the addition).
+//
+// Offsets are taken from the first body of the 1024 that a lane's bodies belong
+// to: FP64 difference, scaled, rounded once.  Those 1024 are consecutive along the
+// curve, so they are close together and their offsets -- and those of the bodies
+// near them -- are small in FP32.  Sums are FP32 over 64 terms (for J over 64 sums
+// of kT), then FP64.
+//
+// VALU issue bound: 16 instructions and one v_rsq_f32 for both bodies of a pair, at
+// the 2.4 to 2.9 clocks that e32 encodings take and 8 for the v_rsq_f32; one target
+// at a time costs 12 and one for each.  2^18 bodies: 19.3 -> 13.0 ms, 5.3e12 pairs/s.
+constexpr int kSymThreads = 256;
+constexpr int kSymWaves = kSymThreads / 64;
+
+__device__ inline float rot_left(float v)     // lane l gets lane l + 1 (mod 64)
 {
-	__shared__ float4 tile[kF32Tile];
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x134, 0xf, 0xf, false));
+}
 
-	const size_t tbase = static_cast<size_t>(blockIdx.x) * kF32TgtPerGroup;
-	const double4 org = sorted[tbase];
-	const double ox = org.x;
-	const double oy = org.y;
-	const double oz = org.z;
-
-	float xi[kF32Tgt], yi[kF32Tgt], zi[kF32Tgt];
-	float sx[kF32Tgt], sy[kF32Tgt], sz[kF32Tgt];
-	float cx[kF32Tgt], cy[kF32Tgt], cz[kF32Tgt];
+// 64 bodies of J (js[l], js[l + 64] = body l) against kT bodies per lane: p += what
+// the lane's bodies receive; kReact: r = what body `lane` of J receives.
+// kWide: coordinates so large that (1/r)^3 could leave the FP32 range.
+// kFine: each product goes to the FP64 sums ax by itself.
+template <int kT, bool kReact, bool kWide, bool kFine>
+__device__ inline void sym_block(const float4* js, int lane, const float (&x)[kT], const float (&y)[kT],
+                                 const float (&z)[kT], const float (&m)[kT], float (&px)[kT], float (&py)[kT],
+                                 float (&pz)[kT], double (&ax)[kT], double (&ay)[kT], double (&az)[kT], float& rx,
+                                 float& ry, float& rz)
+{
+	rx = ry = rz = 0.0f;
+#pragma unroll 4
+	for(int k = 0; k < 64; ++k)
+	{
+		const float4 s = js[lane + k];
+		float ux = 0.0f, uy = 0.0f, uz = 0.0f;
 #pragma unroll
-	for(int k = 0; k < kF32Tgt; ++k)
-	{
-		size_t i = tbase + static_cast<size_t>(k) * kF32Threads + threadIdx.x;
-		bool ok = i < n;
-		const double4 t = ok ? sorted[i] : org;
-		xi[k] = ok ? static_cast<float>((t.x - ox) * kF32Len) : 0.0f;
-		yi[k] = ok ? static_cast<float>((t.y - oy) * kF32Len) : 0.0f;
-		zi[k] = ok ? static_cast<float>((t.z - oz) * kF32Len) : 0.0f;
-		sx[k] = sy[k] = sz[k] = 0.0f;
-		cx[k] = cy[k] = cz[k] = 0.0f;
-	}
-
-	const size_t jbeg = static_cast<size_t>(blockIdx.y) * jchunk;
-	const size_t jend = jbeg + jchunk < n ? jbeg + jchunk : n;
-
-	for(size_t base = jbeg; base < jend; base += kF32Tile)
-	{
-		const size_t j = base + threadIdx.x;
-		__syncthreads();
-		if(j < jend)
+		for(int t = 0; t < kT; ++t)
 		{
-			const double4 sj = sorted[j];
-			tile[threadIdx.x] = make_float4(static_cast<float>((sj.x - ox) * kF32Len),
-			                                static_cast<float>((sj.y - oy) * kF32Len),
-			                                static_cast<float>((sj.z - oz) * kF32Len),
-			                                static_cast<float>(sj.w * kF32Mass));
+			const float dx = s.x - x[t];
+			const float dy = s.y - y[t];
+			const float dz = s.z - z[t];
+			const float q = rsq_clamped(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
+			const float q2 = q * q;
+			const float q3 = q2 * q;
+			const float wj = kWide ? (s.w * q) * q2 : s.w * q3;
+			if(kFine)
+			{
+				ax[t] += static_cast<double>(dx * wj);
+				ay[t] += static_cast<double>(dy * wj);
+				az[t] += static_cast<double>(dz * wj);
+			}
+			else
+			{
+				px[t] = fmaf(dx, wj, px[t]);
+				py[t] = fmaf(dy, wj, py[t]);
+				pz[t] = fmaf(dz, wj, pz[t]);
+			}
+			if(kReact)
+			{
+				const float wi = kWide ? (m[t] * q) * q2 : m[t] * q3;
+				ux = t == 0 ? dx * wi : fmaf(dx, wi, ux);
+				uy = t == 0 ? dy * wi : fmaf(dy, wi, uy);
+				uz = t == 0 ? dz * wi : fmaf(dz, wi, uz);
+			}
+		}
+		if(kReact)
+		{
+			rx = rot_left(rx) - ux;
+			ry = rot_left(ry) - uy;
+			rz = rot_left(rz) - uz;
+		}
+	}
+	if(kReact)
+	{
+		rx = rot_left(rx);
+		ry = rot_left(ry);
+		rz = rot_left(rz);
+	}
+}
+
+// Offsets d in [d0 + blockIdx.y * per, + per), below d1.  own: [gridDim.y][3][n]
+// doubles, the sums of block I's bodies; other: [d1 - d0][3][n] floats, what the
+// bodies of block J receive from block J - d (rows d >= 1 only).
+template <int kT>
+__global__ void __launch_bounds__(kSymThreads)
+k_direct_fp32_sym(const double4* __restrict__ sorted, const double* __restrict__ box, double* __restrict__ own,
+                  float* __restrict__ other, size_t n, int nb, int d0, int d1, int per)
+{
+	constexpr int kB = kSymThreads * kT;
+	constexpr int kSub = kB / 64;
+	__shared__ float4 js[kSymWaves][128];
+	__shared__ float react[3][kB];
+	const int lane = threadIdx.x & 63;
+	const int wave = threadIdx.x >> 6;
+	const int bi = blockIdx.x;
+	const size_t i0 = static_cast<size_t>(bi) * kB + static_cast<size_t>(wave) * (64 * kT) + lane;
+	bool wide = false;
+	for(int c = 0; c < 3; ++c) { wide = wide || !(box[3 + c] - box[c] < 5e7); }
+	// bodies beyond n: copies of the last one, without mass
+	const size_t g0 = i0 - lane < n ? (i0 - lane) / kF32Group * kF32Group : 0;
+	const double4 org = sorted[g0];
+	float x[kT], y[kT], z[kT], m[kT];
+	double ax[kT], ay[kT], az[kT];
+#pragma unroll
+	for(int t = 0; t < kT; ++t)
+	{
+		const size_t i = i0 + 64 * t;
+		const double4 si = sorted[i < n ? i : n - 1];
+		x[t] = static_cast<float>((si.x - org.x) * kF32Len);
+		y[t] = static_cast<float>((si.y - org.y) * kF32Len);
+		z[t] = static_cast<float>((si.z - org.z) * kF32Len);
+		m[t] = i < n ? static_cast<float>(si.w * kF32Mass) : 0.0f;
+		ax[t] = ay[t] = az[t] = 0.0;
+	}
+	const int first = d0 + static_cast<int>(blockIdx.y) * per;
+	const int last = first + per < d1 ? first + per : d1;
+	for(int d = first; d < last; ++d)
+	{
+		if(d > 0 && 2 * d == nb && bi >= d) { continue; }      // these blocks met the other way round
+		const int bj = bi + d < nb ? bi + d : bi + d - nb;
+		if(d > 0)
+		{
+			for(int i = threadIdx.x; i < kB; i += kSymThreads) { react[0][i] = react[1][i] = react[2][i] = 0.0f; }
+			__syncthreads();
+		}
+		for(int s = 0; s < kSub; ++s)
+		{
+			// the waves are a quarter of J apart, so no two add to the same bodies' sums
+			const int sub = (s + wave * (kSub / kSymWaves)) % kSub;
+			const size_t j0 = static_cast<size_t>(bj) * kB + 64 * sub;
+			if(j0 < n)
+			{
+				const size_t j = j0 + lane;
+				const double4 sj = sorted[j < n ? j : n - 1];
+				const float4 f = make_float4(static_cast<float>((sj.x - org.x) * kF32Len),
+				                             static_cast<float>((sj.y - org.y) * kF32Len),
+				                             static_cast<float>((sj.z - org.z) * kF32Len),
+				                             j < n ? static_cast<float>(sj.w * kF32Mass) : 0.0f);
+				__builtin_amdgcn_wave_barrier();
+				js[wave][lane] = f;
+				js[wave][lane + 64] = f;
+				__builtin_amdgcn_wave_barrier();
+				float px[kT], py[kT], pz[kT], rx, ry, rz;
+#pragma unroll
+				for(int t = 0; t < kT; ++t) { px[t] = py[t] = pz[t] = 0.0f; }
+				if(d == 0 && sub / kT == wave)
+				{
+					// the wave's own bodies, nearest neighbours among them: one large term
+					// must not take the last bits of the others
+					sym_block<kT, false, true, true>(js[wave], lane, x, y, z, m, px, py, pz, ax, ay, az, rx, ry, rz);
+				}
+				else if(d == 0)
+				{
+					sym_block<kT, false, true, false>(js[wave], lane, x, y, z, m, px, py, pz, ax, ay, az, rx, ry, rz);
+				}
+				else if(wide)
+				{
+					sym_block<kT, true, true, false>(js[wave], lane, x, y, z, m, px, py, pz, ax, ay, az, rx, ry, rz);
+				}
+				else
+				{
+					sym_block<kT, true, false, false>(js[wave], lane, x, y, z, m, px, py, pz, ax, ay, az, rx, ry, rz);
+				}
+#pragma unroll
+				for(int t = 0; t < kT; ++t)
+				{
+					ax[t] += static_cast<double>(px[t]);
+					ay[t] += static_cast<double>(py[t]);
+					az[t] += static_cast<double>(pz[t]);
+				}
+				if(d > 0)
+				{
+					react[0][64 * sub + lane] += rx;
+					react[1][64 * sub + lane] += ry;
+					react[2][64 * sub + lane] += rz;
+				}
+			}
+			if(d > 0) { __syncthreads(); }
+		}
+		if(d > 0)
+		{
+			float* out = other + static_cast<size_t>(d - d0) * 3 * n;
+			for(int i = threadIdx.x; i < kB; i += kSymThreads)
+			{
+				const size_t j = static_cast<size_t>(bj) * kB + i;
+				if(j < n)
+				{
+					out[j] = react[0][i];
+					out[n + j] = react[1][i];
+					out[2 * n + j] = react[2][i];
+				}
+			}
+			__syncthreads();
+		}
+	}
+	double* out = own + static_cast<size_t>(blockIdx.y) * 3 * n;
+#pragma unroll
+	for(int t = 0; t < kT; ++t)
+	{
+		const size_t i = i0 + 64 * t;
+		if(i < n)
+		{
+			out[i] = ax[t];
+			out[n + i] = ay[t];
+			out[2 * n + i] = az[t];
+		}
+	}
+}
+
+// Adds the sums of offsets d0 .. d1 - 1 (rows as written above) in a fixed order:
+// to acc[3][n] (begin: from 0), or, at the end, into f through the order, with
+// f[0:3n] = v.
+__global__ void __launch_bounds__(256)
+k_direct_fp32_sym_sum(const double* __restrict__ y, const uint32_t* __restrict__ perm, const double* __restrict__ own,
+                      const float* __restrict__ other, double* __restrict__ acc, double* __restrict__ f, size_t n, int kb,
+                      int nb, int d0, int d1, int rows, int begin, int end)
+{
+	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride)
+	{
+		double a[3] = {0.0, 0.0, 0.0};
+		for(int c = 0; c < 3 && !begin; ++c) { a[c] = acc[c * n + i]; }
+		for(int r = 0; r < rows; ++r)
+		{
+			const double* p = own + static_cast<size_t>(r) * 3 * n;
+			for(int c = 0; c < 3; ++c) { a[c] += p[c * n + i]; }
+		}
+		const int block = static_cast<int>(i / kb);
+		for(int d = d0 > 0 ? d0 : 1; d < d1; ++d)
+		{
+			const int from = block >= d ? block - d : block - d + nb;
+			if(2 * d == nb && from >= d) { continue; }
+			const float* p = other + static_cast<size_t>(d - d0) * 3 * n;
+			for(int c = 0; c < 3; ++c) { a[c] += static_cast<double>(p[c * n + i]); }
+		}
+		if(end)
+		{
+			const size_t b = perm[i];
+			for(int c = 0; c < 3; ++c)
+			{
+				f[c * n + i] = y[(3 + c) * n + i];
+				f[(3 + c) * n + b] = a[c];
+			}
 		}
 		else
 		{
-			tile[threadIdx.x] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // zero mass: no force
-		}
-		__syncthreads();
-
-		float px[kF32Tgt], py[kF32Tgt], pz[kF32Tgt];
-#pragma unroll
-		for(int k = 0; k < kF32Tgt; ++k) { px[k] = py[k] = pz[k] = 0.0f; }
-
-#pragma unroll 4
-		for(int jj = 0; jj < kF32Tile; ++jj)
-		{
-			const float4 s = tile[jj];
-#pragma unroll
-			for(int k = 0; k < kF32Tgt; ++k)
-			{
-				const float dx = s.x - xi[k];
-				const float dy = s.y - yi[k];
-				const float dz = s.z - zi[k];
-				const float q = rsq_clamped(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
-				const float w = (s.w * q) * (q * q);
-				px[k] = fmaf(dx, w, px[k]);
-				py[k] = fmaf(dy, w, py[k]);
-				pz[k] = fmaf(dz, w, pz[k]);
-			}
-		}
-#pragma unroll
-		for(int k = 0; k < kF32Tgt; ++k)
-		{
-			kahan_f32(sx[k], cx[k], px[k]);
-			kahan_f32(sy[k], cy[k], py[k]);
-			kahan_f32(sz[k], cz[k], pz[k]);
-		}
-	}
-
-	double* out = part + static_cast<size_t>(blockIdx.y) * 3 * n;
-#pragma unroll
-	for(int k = 0; k < kF32Tgt; ++k)
-	{
-		size_t i = tbase + static_cast<size_t>(k) * kF32Threads + threadIdx.x;
-		if(i < n)
-		{
-			out[i] = static_cast<double>(sx[k]) - static_cast<double>(cx[k]);
-			out[n + i] = static_cast<double>(sy[k]) - static_cast<double>(cy[k]);
-			out[2 * n + i] = static_cast<double>(sz[k]) - static_cast<double>(cz[k]);
+			for(int c = 0; c < 3; ++c) { acc[c * n + i] = a[c]; }
 		}
 	}
 }
@@ -748,38 +895,38 @@ k_direct_fp32(const double4* __restrict__ sorted, double* __restrict__ part, siz
 // the sources at positions p - w .. p + w (its neighbours along the curve, where
 // the FP32 rounding of the offsets weighs most) are recomputed in FP64 (force
 // law of nbody/nbody_data.cpp:35-44) and in the FP32 tiles' own arithmetic (same
-// work-group origin, scaled units and clamped rsq), and f gets the difference.
+// origin, scaled units and clamped rsq), and f gets the difference.  kb: bodies
+// per block of the tiles; a pair's origin is that of the body in the lower block,
+// and the target's own inside a block (blocks w apart or less are neighbours, and
+// of two neighbours the lower one is I).
 constexpr int kCorrWindow = 32;
 
 __global__ void __launch_bounds__(256)
 k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__ perm, double* __restrict__ f,
-                size_t n, int w)
+                size_t n, int w, int kb)
 {
 	const size_t p = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
 	if(p >= n) { return; }
 	const uint32_t i = perm[p];
-	const double4 org = sorted[p / kF32TgtPerGroup * kF32TgtPerGroup];     // the tile kernel's origin
-	const double ox = org.x, oy = org.y, oz = org.z;
 	const double4 me = sorted[p];
 	const double xi = me.x, yi = me.y, zi = me.z;
-	const float txf = static_cast<float>((xi - ox) * kF32Len);
-	const float tyf = static_cast<float>((yi - oy) * kF32Len);
-	const float tzf = static_cast<float>((zi - oz) * kF32Len);
 	double cx = 0.0, cy = 0.0, cz = 0.0;
 	const size_t q0 = p > static_cast<size_t>(w) ? p - w : 0;
 	const size_t q1 = p + w < n - 1 ? p + w : n - 1;
 	for(size_t q = q0; q <= q1; ++q)
 	{
 		if(q == p) { continue; }
+		const double4 org = sorted[(q / kb < p / kb ? q : p) / kF32Group * kF32Group];
+		const double ox = org.x, oy = org.y, oz = org.z;
 		const double4 sj = sorted[q];
 		const double xj = sj.x, yj = sj.y, zj = sj.z, mj = sj.w;
 		const double dx = xj - xi, dy = yj - yi, dz = zj - zi;
 		double r2 = dx * dx + dy * dy + dz * dz;
 		if(r2 < kMinDistance) { r2 = kMinDistance; }
 		const double c = mj / (r2 * sqrt(r2));
-		const float fx = static_cast<float>((xj - ox) * kF32Len) - txf;
-		const float fy = static_cast<float>((yj - oy) * kF32Len) - tyf;
-		const float fz = static_cast<float>((zj - oz) * kF32Len) - tzf;
+		const float fx = static_cast<float>((xj - ox) * kF32Len) - static_cast<float>((xi - ox) * kF32Len);
+		const float fy = static_cast<float>((yj - oy) * kF32Len) - static_cast<float>((yi - oy) * kF32Len);
+		const float fz = static_cast<float>((zj - oz) * kF32Len) - static_cast<float>((zi - oz) * kF32Len);
 		const float qf = rsq_clamped(fmaf(fz, fz, fmaf(fy, fy, fx * fx)));
 		const float wf = (static_cast<float>(mj * kF32Mass) * qf) * (qf * qf);
 		cx += dx * c - static_cast<double>(fx * wf);
@@ -789,32 +936,6 @@ k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__
 	f[3 * n + i] += cx;
 	f[4 * n + i] += cy;
 	f[5 * n + i] += cz;
-}
-
-// f[0:3n] = v, f[3n:6n] = sum over slices (fixed order).
-__global__ void __launch_bounds__(256)
-k_direct_fp32_finish(const double* __restrict__ y, const uint32_t* __restrict__ perm,
-                     const double* __restrict__ part, double* __restrict__ f, size_t n, int nsplit)
-{
-	size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride)
-	{
-		double ax = 0.0, ay = 0.0, az = 0.0;
-		for(int s = 0; s < nsplit; ++s)
-		{
-			const double* p = part + static_cast<size_t>(s) * 3 * n;
-			ax += p[i];
-			ay += p[n + i];
-			az += p[2 * n + i];
-		}
-		f[i] = y[3 * n + i];
-		f[n + i] = y[4 * n + i];
-		f[2 * n + i] = y[5 * n + i];
-		const size_t b = perm[i];
-		f[3 * n + b] = ax;
-		f[4 * n + b] = ay;
-		f[5 * n + b] = az;
-	}
 }
 
 // Bounding box of the positions: per work-group minima and maxima ...
@@ -918,33 +1039,56 @@ k_morton_keys(const double* __restrict__ y, size_t n, const double* __restrict__
 	}
 }
 
-// Launch shape and scratch layout of the FP32 path for n bodies: the sources
-// are split so that the grid holds ~8 work-groups per CU; the scratch holds
-// the split partial sums, the Morton-ordered records, the sort keys / values
-// (two halves each), the sort's scratch, bounding-box partials and the box, each
-// at a 256-byte boundary.
+// Launch shape and scratch layout of the FP32 path for n bodies: bodies per lane,
+// block offsets per work-group (per) and per pass (span), and the scratch: the
+// sums of one pass (own and other, k_direct_fp32_sym), the sums of the passes
+// before, the Morton-ordered records, the sort keys / values (two halves each), the
+// sort's scratch, bounding-box partials and the box, each at a 256-byte boundary.
 struct fp32_layout {
-	size_t gx, nsplit, jchunk;
+	int kt, nb, span, per;
 	unsigned gbox;
-	size_t off_sorted, off_keys, off_vals, off_counts, off_bpart, off_box, bytes;
+	size_t off_other, off_acc, off_sorted, off_keys, off_vals, off_counts, off_bpart, off_box, bytes;
 };
+
+// Sums of one pass take at most this much (a pass has one offset at least): 52 MiB
+// up to 131072 bodies, which leaves the whole scratch under the 64 MiB that
+// nbh_fcompute_direct_noalloc has.
+constexpr size_t kSymBytesSmall = static_cast<size_t>(52) << 20;
+constexpr size_t kSymBytes = static_cast<size_t>(256) << 20;
+constexpr size_t kNoAllocMaxBodies = 131072;
 
 fp32_layout fp32_plan(const nbh_ctx* ctx, size_t n)
 {
 	fp32_layout l;
-	l.gx = (n + kF32TgtPerGroup - 1) / kF32TgtPerGroup;
-	const size_t want = static_cast<size_t>(ctx->cu_count > 0 ? ctx->cu_count : 256) * 8;
-	size_t nsplit = (want + l.gx - 1) / l.gx;
-	const size_t max_split = (n + kF32Tile - 1) / kF32Tile;
-	if(nsplit > max_split) { nsplit = max_split; }
-	if(nsplit > 64) { nsplit = 64; }
-	if(nsplit < 1) { nsplit = 1; }
-	size_t jchunk = (n + nsplit - 1) / nsplit;
-	l.jchunk = (jchunk + kF32Tile - 1) / kF32Tile * kF32Tile;
-	l.nsplit = (n + l.jchunk - 1) / l.jchunk;
+	// More bodies per lane cost fewer rotations and LDS reads per pair but leave
+	// fewer blocks: 1, 2, 4 and 8 took 200, 204, 222 and - us at 20000 bodies, 367,
+	// 344, 394 and - at 32768, -, 1.08, 1.03 and 1.27 ms at 65536, -, 4.1, 3.9 and 4.0
+	// at 2^17 and -, 9.4, 8.9 and 8.1 at 200003.
+	l.kt = n < 24576 ? 1 : n < 49152 ? 2 : n < 163840 ? 4 : 8;
+	const size_t kb = static_cast<size_t>(kSymThreads) * l.kt;
+	l.nb = static_cast<int>((n + kb - 1) / kb);
+	const size_t offsets = static_cast<size_t>(l.nb) / 2 + 1;
+	const size_t cap = n <= kNoAllocMaxBodies ? kSymBytesSmall : kSymBytes;
+	auto pass_bytes = [&](size_t span, size_t per) { return (span * 12 + (span + per - 1) / per * 24) * n; };
+	// 16 work-groups per CU where there are that many; up to four offsets each if
+	// that makes it one pass, else equal passes
+	const size_t want = static_cast<size_t>(ctx->cu_count > 0 ? ctx->cu_count : 256) * 16;
+	const size_t least = std::min<size_t>(std::max<size_t>(l.nb * offsets / want, 1), 8);
+	size_t per = least, span = offsets;
+	while(pass_bytes(span, per) > cap && per < 4) { ++per; }
+	if(pass_bytes(span, per) > cap)
+	{
+		per = least;
+		size_t passes = 1;
+		while(span > 1 && pass_bytes(span, per) > cap) { span = (offsets + passes) / (passes + 1); ++passes; }
+	}
+	l.per = static_cast<int>(per);
+	l.span = static_cast<int>(span);
 	l.gbox = nbh::grid_for(ctx, n, 256);
 	auto align = [](size_t b) { return (b + 255) / 256 * 256; };
-	l.off_sorted = align(l.nsplit * 3 * n * sizeof(double));
+	l.off_other = align((span + per - 1) / per * 3 * n * sizeof(double));
+	l.off_acc = l.off_other + align(span * 3 * n * sizeof(float));
+	l.off_sorted = l.off_acc + (span < offsets ? align(3 * n * sizeof(double)) : 0);
 	l.off_keys = l.off_sorted + align(n * sizeof(double4));
 	l.off_vals = l.off_keys + align(2 * n * sizeof(uint64_t));
 	l.off_counts = l.off_vals + align(2 * n * sizeof(uint32_t));
@@ -960,7 +1104,9 @@ fp32_layout fp32_plan(const nbh_ctx* ctx, size_t n)
 nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f, size_t n, nbh_precision precision,
                     const fp32_layout& l, char* base, bool timed)
 {
-	double* part = reinterpret_cast<double*>(base);
+	double* own = reinterpret_cast<double*>(base);
+	float* other = reinterpret_cast<float*>(base + l.off_other);
+	double* acc = reinterpret_cast<double*>(base + l.off_acc);
 	double4* sorted = reinterpret_cast<double4*>(base + l.off_sorted);
 	uint64_t* keys = reinterpret_cast<uint64_t*>(base + l.off_keys);
 	uint32_t* vals = reinterpret_cast<uint32_t*>(base + l.off_vals);
@@ -977,19 +1123,28 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	NBH_TRY(nbh::sort_pairs(ctx, keys, vals, keys + n, vals + n, n, 30, counts, &perm));
 	hipLaunchKernelGGL(k_sorted_copy, dim3(l.gbox), dim3(256), 0, ctx->stream, y, mass, perm, sorted, n);
 	NBH_LAUNCHED();
+	const int kb = kSymThreads * l.kt;
+	const int offsets = l.nb / 2 + 1;
 	{
 		nbh::scoped_timer timer(timed ? ctx : nullptr, "direct_fp32");
-		hipLaunchKernelGGL(k_direct_fp32, dim3(static_cast<unsigned>(l.gx), static_cast<unsigned>(l.nsplit)),
-		                   dim3(kF32Threads), 0, ctx->stream, sorted, part, n, l.jchunk);
-		NBH_LAUNCHED();
+		for(int d0 = 0; d0 < offsets; d0 += l.span)
+		{
+			const int d1 = d0 + l.span < offsets ? d0 + l.span : offsets;
+			const int rows = (d1 - d0 + l.per - 1) / l.per;
+			hipLaunchKernelGGL(l.kt == 8 ? k_direct_fp32_sym<8> : l.kt == 4 ? k_direct_fp32_sym<4> :
+			                   l.kt == 2 ? k_direct_fp32_sym<2> : k_direct_fp32_sym<1>,
+			                   dim3(static_cast<unsigned>(l.nb), static_cast<unsigned>(rows)), dim3(kSymThreads), 0,
+			                   ctx->stream, sorted, box, own, other, n, l.nb, d0, d1, l.per);
+			NBH_LAUNCHED();
+			hipLaunchKernelGGL(k_direct_fp32_sym_sum, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, y, perm,
+			                   own, other, acc, f, n, kb, l.nb, d0, d1, rows, d0 == 0 ? 1 : 0, d1 == offsets ? 1 : 0);
+			NBH_LAUNCHED();
+		}
 	}
-	hipLaunchKernelGGL(k_direct_fp32_finish, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0,
-	                   ctx->stream, y, perm, part, f, n, static_cast<int>(l.nsplit));
-	NBH_LAUNCHED();
 	if(precision == NBH_FP32_CORR)
 	{
 		hipLaunchKernelGGL(k_direct_window, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, ctx->stream,
-		                   sorted, perm, f, n, kCorrWindow);
+		                   sorted, perm, f, n, kCorrWindow, kb);
 		NBH_LAUNCHED();
 	}
 	return NBH_OK;
@@ -1066,7 +1221,6 @@ extern "C" nbh_status nbh_fcompute_direct(nbh_ctx* ctx, const double* y, const d
 namespace {
 
 constexpr size_t kNoAllocBytes = static_cast<size_t>(64) << 20;
-constexpr size_t kNoAllocMaxBodies = 131072;
 constexpr int kNoAllocDevices = 64;
 
 }  // namespace

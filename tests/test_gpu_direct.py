@@ -138,6 +138,39 @@ def _check_rel(rel):
     assert rms < FP32_RMS_REL, f"rms rel {rms:.3e}"
 
 
+# blocks of 256, 512, 1024 and 2048 bodies (1, 2, 4, 8 per lane), odd and even
+# numbers of blocks, last blocks of one body, one 64-body row and one missing body
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 511, 513, 769, 1025, 4095, 4097, 24575, 24576, 24577,
+                               49151, 49153, 163839, 163841])
+def test_fp32_block_edges(ctx, n):
+    """Every pair once: a block pair left out or met twice shows as an error of at
+    least a few bodies in n, far above FP32 rounding."""
+    y, m = _state("ball", n, 3 + n)
+    m = m * np.random.default_rng(n).uniform(0.5, 1.5, n)
+    f = _run(ctx, y, m, NBH_FP32)
+    f64 = _run(ctx, y, m, NBH_FP64)
+    assert np.array_equal(f[:3 * n], y[3 * n:])
+    if n > 1:
+        _check_rel(_rel_err(f, f64, n))
+    assert np.array_equal(f, _run(ctx, y, m, NBH_FP32))      # the same bits again
+    fc = _run(ctx, y, m, NBH_FP32_CORR)
+    if n > 1:
+        assert _rel_err(fc, f64, n).mean() <= 1.5 * _rel_err(f, f64, n).mean()
+
+
+@pytest.mark.parametrize("scale", [1e-3, 1e9])
+def test_fp32_far_apart_and_clamped(ctx, scale):
+    """Distances whose cube leaves FP32 (1e9) and distances around the clamp (1e-3)."""
+    n = 3000
+    y, m = _state("ball", n, 8)
+    y[:3 * n] *= scale
+    f = _run(ctx, y, m, NBH_FP32)
+    f64 = _run(ctx, y, m, NBH_FP64)
+    rel = np.linalg.norm((f - f64)[3 * n:].reshape(3, n), axis=0)
+    rel /= np.sqrt(np.mean(np.sum(f64[3 * n:].reshape(3, n) ** 2, axis=0)))
+    assert np.sqrt(np.mean(rel ** 2)) < FP32_RMS_REL and rel.max() < FP32_MAX_REL
+
+
 def test_fp32_matches_fp64_kernel_large(ctx):
     """At 2^17 bodies (no CPU reference needed) the FP32 tiles agree with the
     FP64 kernel, which is bit-exact with the oracle at every smaller size."""
