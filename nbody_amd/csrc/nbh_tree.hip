@@ -2191,7 +2191,9 @@ __device__ inline void sweep32_n(const float4* __restrict__ buf, int count, cons
 	float px[kT], py[kT], pz[kT];
 #pragma unroll
 	for(int t = 0; t < kT; ++t) { px[t] = py[t] = pz[t] = 0.0f; }
-#pragma unroll 2
+	// four chains in flight (one body per lane: 2^18 bodies, monopole, 1.85 ms
+	// against 1.94 with two)
+#pragma unroll kT == 1 ? 4 : 2
 	for(int j = 0; j < count; ++j)
 	{
 		const float4 s = buf[j];
@@ -2843,10 +2845,21 @@ __device__ inline void group_walk_one(int gi, int* __restrict__ stack, float4* _
 }
 
 // The group walk kernel, one work-group per group: the heap's groups in
-// XCD-contiguous order, the Morton tree's in launch order.  (Measured at 4M
-// Plummer bodies: persistent work-groups that take groups from counters, per
-// XCD or in one queue, and chunked XCD orders all ran the Morton walk 9-19%
-// slower than this.)
+// XCD-contiguous order, the Morton tree's in runs of 128 per XCD (at 4M Plummer
+// bodies 2.66 ms against 2.80 in launch order, 2.72 in runs of 32: neighbours share
+// their super-group's list and nodes in one L2; persistent work-groups that take
+// groups from counters, per XCD or in one queue, ran 9-19% slower; two waves that
+// share a group's list gain 17% at 16384-50000 bodies and lose from 100003 on).
+constexpr int kXcdRun = 128;
+
+__device__ inline int xcd_run_group(int block, int nblocks)
+{
+	const int whole = nblocks / (kXcds * kXcdRun) * (kXcds * kXcdRun);
+	if(block >= whole) { return block; }
+	const int i = block / kXcds;
+	return (i / kXcdRun * kXcds + block % kXcds) * kXcdRun + i % kXcdRun;
+}
+
 template <bool kQuad, bool kLocal = false, bool kTwo = false, bool kRadix = false>
 __global__ void __launch_bounds__(kGroup)
 k_bh_group32(const nbh_walk_rec* __restrict__ wr, const double* __restrict__ bmin, const double* __restrict__ bmax,
@@ -2858,7 +2871,7 @@ k_bh_group32(const nbh_walk_rec* __restrict__ wr, const double* __restrict__ bmi
 	__shared__ float4 buf[kWalkBuf];
 	__shared__ quad_lds<kQuad ? kQuadBuf : 1> qbuf;
 	__shared__ int farn[kQuad ? kFarRing : 1];
-	const int gi = kRadix ? static_cast<int>(blockIdx.x) : xcd_group(blockIdx.x, gridDim.x);
+	const int gi = kRadix ? xcd_run_group(blockIdx.x, gridDim.x) : xcd_group(blockIdx.x, gridDim.x);
 	group_walk_one<kQuad, kLocal, kTwo, kRadix>(gi, stack, buf, qbuf, farn, wr, bmin, bmax, body_n, y, f, n, near_k,
 	                                             counters, two, tree);
 }
