@@ -806,9 +806,22 @@ k_leaves(const uint32_t* __restrict__ order, const double* __restrict__ y, const
 __device__ inline double min_ref(double a, double b) { return (b < a) ? b : a; }   // std::min
 __device__ inline double max_ref(double a, double b) { return (a < b) ? b : a; }   // std::max
 
+// Opening radius crit_r2 = (radius * ratio)^2 of a node with mass centre c and
+// box lo, hi, in the heap's operation order.
+__device__ inline double crit_radius(double cx, double cy, double cz, const double* lo, const double* hi,
+                                     double ratio_sqr)
+{
+	double ex = hi[0] - lo[0], ey = hi[1] - lo[1], ez = hi[2] - lo[2];
+	double gx = (hi[0] + lo[0]) / 2.0 - cx;
+	double gy = (hi[1] + lo[1]) / 2.0 - cy;
+	double gz = (hi[2] + lo[2]) / 2.0 - cz;
+	double rad = sqrt(ex * ex + ey * ey + ez * ez) * 0.5 + sqrt(gx * gx + gy * gy + gz * gz);
+	return (rad * rad) * ratio_sqr;
+}
+
 // A node's moments from its children's (mass centre cl / cr, masses ml / mr,
-// boxes lol..hil / lor..hir): mass, mass centre, box and crit_r2 = (radius *
-// ratio)^2 with the heap's operation order.
+// boxes lol..hil / lor..hir): mass, mass centre, box and opening radius with the
+// heap's operation order.
 __device__ inline void combine_node(const double4& cl, double ml, const double* lol, const double* hil,
                                     const double4& cr, double mr, const double* lor, const double* hir,
                                     double ratio_sqr, double4& c, double& m, double* lo, double* hi)
@@ -822,33 +835,10 @@ __device__ inline void combine_node(const double4& cl, double ml, const double* 
 		lo[d] = min_ref(lol[d], lor[d]);
 		hi[d] = max_ref(hil[d], hir[d]);
 	}
-	double ex = hi[0] - lo[0], ey = hi[1] - lo[1], ez = hi[2] - lo[2];
-	double gx = (hi[0] + lo[0]) / 2.0 - cx;
-	double gy = (hi[1] + lo[1]) / 2.0 - cy;
-	double gz = (hi[2] + lo[2]) / 2.0 - cz;
-	double rad = sqrt(ex * ex + ey * ey + ez * ez) * 0.5 + sqrt(gx * gx + gy * gy + gz * gz);
-	c = make_double4(cx, cy, cz, (rad * rad) * ratio_sqr);
+	c = make_double4(cx, cy, cz, crit_radius(cx, cy, cz, lo, hi, ratio_sqr));
 }
 
-// Node idx from its children l and r (2 idx and 2 idx + 1 in the heap).
-__device__ inline void update_node(size_t idx, size_t l, size_t r, double4* __restrict__ xyzr,
-                                   double* __restrict__ nmass, double* __restrict__ bmin, double* __restrict__ bmax,
-                                   double ratio_sqr)
-{
-	double4 c;
-	double m, lo[3], hi[3];
-	combine_node(xyzr[l], nmass[l], bmin + 3 * l, bmax + 3 * l, xyzr[r], nmass[r], bmin + 3 * r, bmax + 3 * r,
-	             ratio_sqr, c, m, lo, hi);
-	for(int d = 0; d < 3; ++d)
-	{
-		bmin[3 * idx + d] = lo[d];
-		bmax[3 * idx + d] = hi[d];
-	}
-	nmass[idx] = m;
-	xyzr[idx] = c;
-}
-
-// Second central moments Q = sum m (x - cm)(x - cm)^T of node idx from its
+// Second central moments Q = sum m (x - cm)(x - cm)^T of a node from its
 // children (parallel-axis theorem); components xx yy zz xy xz yz.  Not part of
 // the reference tree: input of the learned correction.
 __device__ inline void combine_quad(const double4& c, const double4& cl, double ml, const double* ql,
@@ -870,12 +860,44 @@ __device__ inline void combine_quad(const double4& c, const double4& cl, double 
 	}
 }
 
-__device__ inline void update_quad(size_t idx, size_t l, size_t r, const double4* __restrict__ xyzr,
-                                   const double* __restrict__ nmass, double* __restrict__ quad)
+// Node idx from its children l and r (2 idx and 2 idx + 1 in the heap), each
+// child read once; kRecord: its walk record too (as k_pack_records).
+template <bool kRecord>
+__device__ inline void join_nodes(size_t idx, size_t l, size_t r, double4* xyzr, double* nmass, double* bmin,
+                                  double* bmax, double* quad, double ratio_sqr, nbh_walk_rec* wr = nullptr)
 {
-	double q[6];
-	combine_quad(xyzr[idx], xyzr[l], nmass[l], quad + 6 * l, xyzr[r], nmass[r], quad + 6 * r, q);
+	const double4 cl = xyzr[l], cr = xyzr[r];
+	const double ml = nmass[l], mr = nmass[r];
+	double lol[3], hil[3], lor[3], hir[3], ql[6], qr[6];
+	for(int d = 0; d < 3; ++d)
+	{
+		lol[d] = bmin[3 * l + d];
+		hil[d] = bmax[3 * l + d];
+		lor[d] = bmin[3 * r + d];
+		hir[d] = bmax[3 * r + d];
+	}
+	for(int k = 0; k < 6; ++k)
+	{
+		ql[k] = quad[6 * l + k];
+		qr[k] = quad[6 * r + k];
+	}
+	nbh_walk_rec rec;
+	double lo[3], hi[3], q[6];
+	combine_node(cl, ml, lol, hil, cr, mr, lor, hir, ratio_sqr, rec.c, rec.m, lo, hi);
+	combine_quad(rec.c, cl, ml, ql, cr, mr, qr, q);
+	xyzr[idx] = rec.c;
+	nmass[idx] = rec.m;
+	for(int d = 0; d < 3; ++d)
+	{
+		bmin[3 * idx + d] = lo[d];
+		bmax[3 * idx + d] = hi[d];
+	}
 	for(int k = 0; k < 6; ++k) { quad[6 * idx + k] = q[k]; }
+	if constexpr(kRecord)
+	{
+		for(int k = 0; k < 6; ++k) { rec.q[k] = static_cast<float>(q[k]); }
+		wr[idx] = rec;
+	}
 }
 
 // nodes [lo, hi) of one level
@@ -886,8 +908,7 @@ k_level(size_t lo, size_t hi, double4* __restrict__ xyzr, double* __restrict__ n
 	size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
 	for(size_t idx = lo + static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; idx < hi; idx += stride)
 	{
-		update_node(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, bmin, bmax, ratio_sqr);
-		update_quad(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, quad);
+		join_nodes<false>(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, bmin, bmax, quad, ratio_sqr);
 	}
 }
 
@@ -900,8 +921,7 @@ k_levels_top(size_t top, double4* __restrict__ xyzr, double* __restrict__ nmass,
 	{
 		for(size_t idx = lo + threadIdx.x; idx < 2 * lo; idx += blockDim.x)
 		{
-			update_node(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, bmin, bmax, ratio_sqr);
-			update_quad(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, quad);
+			join_nodes<false>(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, bmin, bmax, quad, ratio_sqr);
 		}
 		__syncthreads();
 	}
@@ -1263,20 +1283,9 @@ k_radix_level_lists(const int* __restrict__ level, size_t n, const int* __restri
 	}
 }
 
-// Walk record of node id from its moments (as k_pack_records).
-__device__ inline void put_record(int id, const double4* __restrict__ xyzr, const double* __restrict__ nmass,
-                                  const double* __restrict__ quad, nbh_walk_rec* __restrict__ wr)
-{
-	nbh_walk_rec r;
-	r.c = xyzr[id];
-	r.m = nmass[id];
-	for(int k = 0; k < 6; ++k) { r.q[k] = static_cast<float>(quad[6 * static_cast<size_t>(id) + k]); }
-	wr[id] = r;
-}
-
 // Moments of the internal ids list[0, count) of one level, from their children
-// (the heap's update_node and update_quad); the levels run from the longest
-// prefix to the root, one launch each.
+// (join_nodes, as the heap's levels); the levels run from the longest prefix to the
+// root, one launch each.
 __global__ void __launch_bounds__(256)
 k_radix_level(const int* __restrict__ list, int count, const int2* __restrict__ child, double4* __restrict__ xyzr,
               double* __restrict__ nmass, double* __restrict__ bmin, double* __restrict__ bmax,
@@ -1287,25 +1296,39 @@ k_radix_level(const int* __restrict__ list, int count, const int2* __restrict__ 
 	{
 		const int id = list[k];
 		const int2 c = child[id];
-		update_node(id, c.x, c.y, xyzr, nmass, bmin, bmax, ratio_sqr);
-		update_quad(id, c.x, c.y, xyzr, nmass, quad);
-		put_record(id, xyzr, nmass, quad, wr);
+		join_nodes<true>(id, c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr);
 	}
 }
 
-// Leaves and internal nodes of each walk group (a subtree of at most
+// `v` of another lane of the same four (kCtrl: the source lane of each, 2 bits a lane).
+template <int kCtrl>
+__device__ inline double quad_lane(double v)
+{
+	const long long b = __double_as_longlong(v);
+	const int lo = __builtin_amdgcn_mov_dpp(static_cast<int>(b), kCtrl, 0xF, 0xF, true);
+	const int hi = __builtin_amdgcn_mov_dpp(static_cast<int>(b >> 32), kCtrl, 0xF, 0xF, true);
+	return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// Leaves and internal nodes of each build group (a subtree of at most
 // kRadixGroup leaves), one wave per group, with their walk records.  The
 // group's leaves (as k_leaves; kBuild: the body at sorted position s is
 // order[s], read from its packed record; refit: the body numbers of the build,
-// positions from y and the masses of the leaf records) and node moments are held in LDS: leaf
-// first + j in slot j, internal id k in slot kRadixGroup + k - first - 1 (the
-// internal ids of a subtree over the sorted leaves [a, b] lie in [a + 1, b + 1]:
-// each internal node's index is one end of its key range).  The internal nodes
-// are listed breadth-first, then taken depth by depth from the deepest (the
-// heap's update_node and update_quad on the LDS slots), and written out.
+// positions from y and the masses of the leaf records) and node moments are held
+// in LDS: leaf first + j in slot j, internal id k in slot k - first - 1 (the
+// internal ids of a subtree over the sorted leaves [a, b] are the ids [a + 1, b + 1]
+// without the end that is not its root: each internal node's index is one end of
+// its key range).  The internal nodes are listed breadth-first, then taken depth by
+// depth from the deepest (combine_node and combine_quad on the LDS slots), four
+// lanes a node: lane d has coordinate d, its diagonal second moment and one of the
+// other three.  The opening radii, which no parent reads, follow for all nodes at
+// once, and the nodes go out in id order.
 // lean: every node's walk record is written (and each leaf's body number), the
 // FP64 node arrays only for the group's root, which the levels above read, or
 // for a group of one leaf.
+// With a lane per node, radius and stores in the depth loop, it was bound by FP64
+// issue there (some 40 nodes in 10 depths): 541 us at 4M bodies, now 363 (0.8 GB
+// moved), latency of the depths and memory alike.
 template <bool kBuild>
 __global__ void __launch_bounds__(kRadixGroup)
 k_radix_group_moments(const int4* __restrict__ grp, int n, const int2* __restrict__ child,
@@ -1314,22 +1337,19 @@ k_radix_group_moments(const int4* __restrict__ grp, int n, const int2* __restric
                       double* __restrict__ bmin, double* __restrict__ bmax, double* __restrict__ quad,
                       double ratio_sqr, nbh_walk_rec* __restrict__ wr, int lean)
 {
-	// leaves: position (box and mass centre) and mass; internal slots: all moments
-	__shared__ double4 s_lc[kRadixGroup];
-	__shared__ double s_lm[kRadixGroup];
-	__shared__ double4 s_c[kRadixGroup];
-	__shared__ double s_m[kRadixGroup];
-	__shared__ double s_lo[3 * kRadixGroup];
-	__shared__ double s_hi[3 * kRadixGroup];
-	__shared__ double s_q[6 * kRadixGroup];
-	__shared__ int2 s_child[kRadixGroup];
-	__shared__ int q[kRadixGroup];          // internal nodes, breadth-first (at most kRadixGroup - 1)
-	__shared__ int start[kRadixGroup + 1];  // first entry of each depth
-	__shared__ double s_zero[6];            // the second moments of a leaf
+	// LDS of doubles: leaf positions and masses; the internal slots' mass centres,
+	// masses, boxes and second moments; the second moments of a leaf
+	constexpr int kG = kRadixGroup;
+	constexpr int kLC = 0, kLM = 3 * kG, kC = 4 * kG, kM = 7 * kG, kLo = 8 * kG, kHi = 11 * kG, kQ = 14 * kG,
+	              kZero = 20 * kG;
+	__shared__ double sh[20 * kG + 6];
+	__shared__ int2 s_child[kG];
+	__shared__ int q[kG];          // internal nodes, breadth-first (at most kRadixGroup - 1)
+	__shared__ int start[kG + 1];  // first entry of each depth
 	const int lane = threadIdx.x;
 	const int4 gr = grp[blockIdx.x];
 	const int root = gr.x, first = gr.y, cnt = gr.z;
-	if(lane < 6) { s_zero[lane] = 0.0; }
+	if(lane < 6) { sh[kZero + lane] = 0.0; }
 	if(lane < cnt)
 	{
 		const size_t sidx = static_cast<size_t>(first) + lane;
@@ -1355,20 +1375,21 @@ k_radix_group_moments(const int4* __restrict__ grp, int n, const int2* __restric
 			z = y[2 * static_cast<size_t>(n) + b];
 			m = wr[idx].m;
 		}
-		const double4 c = make_double4(x, yy, z, 0.0);
+		nbh_walk_rec r;
+		r.c = make_double4(x, yy, z, 0.0);
+		r.m = m;
+		for(int k = 0; k < 6; ++k) { r.q[k] = 0.0f; }
 		if(!lean || root >= n)
 		{
-			xyzr[idx] = c;
+			xyzr[idx] = r.c;
 			bmin[3 * idx] = x; bmin[3 * idx + 1] = yy; bmin[3 * idx + 2] = z;
 			bmax[3 * idx] = x; bmax[3 * idx + 1] = yy; bmax[3 * idx + 2] = z;
 		}
-		nbh_walk_rec r;
-		r.c = c;
-		r.m = m;
-		for(int k = 0; k < 6; ++k) { r.q[k] = 0.0f; }
 		wr[idx] = r;
-		s_lc[lane] = c;
-		s_lm[lane] = m;
+		sh[kLC + 3 * lane] = x;
+		sh[kLC + 3 * lane + 1] = yy;
+		sh[kLC + 3 * lane + 2] = z;
+		sh[kLM + lane] = m;
 		const int id = first + 1 + lane;
 		s_child[lane] = id < n ? child[id] : make_int2(0, 0);
 	}
@@ -1399,101 +1420,118 @@ k_radix_group_moments(const int4* __restrict__ grp, int n, const int2* __restric
 	}
 	// depth d holds q[start[d], start[d + 1]); start[depth] == tail.  A child is
 	// leaf first + j (id n + first + j) or internal slot id - first - 1.
+	const int part = lane & 3, dim = part < 3 ? part : 2;
 	for(int d = depth - 1; d >= 0; --d)
 	{
-		const int i = start[d] + lane;
-		if(i < start[d + 1])
+		const int end = start[d + 1];
+		for(int i = start[d] + (lane >> 2); i < end; i += kG / 4)
 		{
-			const int id = q[i];
-			const int k = id - first - 1;
+			const int k = q[i] - first - 1;
 			const int2 ch = s_child[k];
-			double4 cc[2];
-			double mm[2];
-			double lo2[2][3], hi2[2][3];
-			const double* qq[2];
+			double cc[2], mm[2], lo2[2], hi2[2], qd[2], qo[2];
 			for(int side = 0; side < 2; ++side)
 			{
 				const int cid = side == 0 ? ch.x : ch.y;
-				if(cid >= n)
-				{
-					const int j = cid - n - first;
-					cc[side] = s_lc[j];
-					mm[side] = s_lm[j];
-					lo2[side][0] = hi2[side][0] = cc[side].x;
-					lo2[side][1] = hi2[side][1] = cc[side].y;
-					lo2[side][2] = hi2[side][2] = cc[side].z;
-					qq[side] = s_zero;
-				}
-				else
-				{
-					const int j = cid - first - 1;
-					cc[side] = s_c[j];
-					mm[side] = s_m[j];
-					for(int e = 0; e < 3; ++e)
-					{
-						lo2[side][e] = s_lo[3 * j + e];
-						hi2[side][e] = s_hi[3 * j + e];
-					}
-					qq[side] = s_q + 6 * j;
-				}
+				const bool leaf = cid >= n;
+				const int j = leaf ? cid - n - first : cid - first - 1;
+				const int at = 3 * j + dim;
+				const int qat = leaf ? kZero : kQ + 6 * j;
+				cc[side] = sh[(leaf ? kLC : kC) + at];
+				mm[side] = sh[(leaf ? kLM : kM) + j];
+				lo2[side] = sh[(leaf ? kLC : kLo) + at];
+				hi2[side] = sh[(leaf ? kLC : kHi) + at];
+				qd[side] = sh[qat + dim];
+				qo[side] = sh[qat + 3 + dim];
 			}
-			double4 c;
-			double m, lo[3], hi[3], qv[6];
-			combine_node(cc[0], mm[0], lo2[0], hi2[0], cc[1], mm[1], lo2[1], hi2[1], ratio_sqr, c, m, lo, hi);
-			combine_quad(c, cc[0], mm[0], qq[0], cc[1], mm[1], qq[1], qv);
-			s_c[k] = c;
-			s_m[k] = m;
-			const size_t gid = static_cast<size_t>(id);
-			nbh_walk_rec rec;
-			rec.c = c;
-			rec.m = m;
-			for(int e = 0; e < 3; ++e)
+			const double m = mm[0] + mm[1];
+			const double c = (cc[0] * mm[0] + cc[1] * mm[1]) / m;
+			double qdd = 0.0, qoo = 0.0;
+			for(int side = 0; side < 2; ++side)
 			{
-				s_lo[3 * k + e] = lo[e];
-				s_hi[3 * k + e] = hi[e];
+				const double e = cc[side] - c;
+				// the factors of xy, xz, yz: (x, x, y) and (y, z, z)
+				const double ea = quad_lane<0xD0>(e), eb = quad_lane<0xE9>(e);
+				qdd += qd[side] + mm[side] * e * e;
+				qoo += qo[side] + mm[side] * ea * eb;
 			}
-			for(int e = 0; e < 6; ++e)
+			if(part < 3)
 			{
-				s_q[6 * k + e] = qv[e];
-				rec.q[e] = static_cast<float>(qv[e]);
+				sh[kC + 3 * k + part] = c;
+				sh[kLo + 3 * k + part] = min_ref(lo2[0], lo2[1]);
+				sh[kHi + 3 * k + part] = max_ref(hi2[0], hi2[1]);
+				sh[kQ + 6 * k + part] = qdd;
+				sh[kQ + 6 * k + 3 + part] = qoo;
 			}
-			wr[gid] = rec;
-			if(!lean || id == root)
+			else
 			{
-				xyzr[gid] = c;
-				nmass[gid] = m;
-				for(int e = 0; e < 3; ++e)
-				{
-					bmin[3 * gid + e] = lo[e];
-					bmax[3 * gid + e] = hi[e];
-				}
-				for(int e = 0; e < 6; ++e) { quad[6 * gid + e] = qv[e]; }
+				sh[kM + k] = m;
 			}
 		}
 		__syncthreads();
 	}
+	const int k = lane + (root == first + 1 ? 0 : 1);
+	if(lane < cnt - 1)
+	{
+		const size_t gid = static_cast<size_t>(first) + 1 + k;
+		const double* lo = sh + kLo + 3 * k;
+		const double* hi = sh + kHi + 3 * k;
+		const double cx = sh[kC + 3 * k], cy = sh[kC + 3 * k + 1], cz = sh[kC + 3 * k + 2];
+		nbh_walk_rec rec;
+		rec.c = make_double4(cx, cy, cz, crit_radius(cx, cy, cz, lo, hi, ratio_sqr));
+		rec.m = sh[kM + k];
+		for(int e = 0; e < 6; ++e) { rec.q[e] = static_cast<float>(sh[kQ + 6 * k + e]); }
+		wr[gid] = rec;
+		if(!lean || gid == static_cast<size_t>(root))
+		{
+			xyzr[gid] = rec.c;
+			nmass[gid] = rec.m;
+			for(int e = 0; e < 3; ++e)
+			{
+				bmin[3 * gid + e] = lo[e];
+				bmax[3 * gid + e] = hi[e];
+			}
+			for(int e = 0; e < 6; ++e) { quad[6 * gid + e] = sh[kQ + 6 * k + e]; }
+		}
+	}
 }
 
-// Levels lv_hi down to lv_lo, each too small to fill the device, in one
-// work-group (info: the level counts, then their offsets in list).
-__global__ void __launch_bounds__(1024)
+// Levels lv_hi down to lv_lo, each of fewer nodes than kRadixSmallLevel, in one
+// work-group (info: the level counts, then their offsets in list): a node per
+// work-item, whose id and children are read a level ahead.  Bound by one dependent
+// chain of reads, FP64 divides and roots and a barrier per level: 79 us for the
+// levels of 100003 bodies (99 with the node's own moments read back for the second
+// moments and the record).
+constexpr int kRadixSmallLevel = 512;
+__global__ void __launch_bounds__(kRadixSmallLevel)
 k_radix_levels_small(const int* __restrict__ list, const int* __restrict__ info, int lv_hi, int lv_lo,
                      const int2* __restrict__ child, double4* __restrict__ xyzr, double* __restrict__ nmass,
                      double* __restrict__ bmin, double* __restrict__ bmax, double* __restrict__ quad,
                      double ratio_sqr, nbh_walk_rec* __restrict__ wr)
 {
+	__shared__ int s_info[2 * kRadixLevels];
+	const int t = threadIdx.x;
+	for(int i = t; i < 2 * kRadixLevels; i += blockDim.x) { s_info[i] = info[i]; }
+	__syncthreads();
+	int id = -1;
+	int2 c = make_int2(0, 0);
+	if(t < s_info[lv_hi])
+	{
+		id = list[s_info[kRadixLevels + lv_hi] + t];
+		c = child[id];
+	}
 	for(int lv = lv_hi; lv >= lv_lo; --lv)
 	{
-		const int count = info[lv], off = info[kRadixLevels + lv];
-		for(int k = threadIdx.x; k < count; k += blockDim.x)
+		int next_id = -1;
+		int2 next = make_int2(0, 0);
+		if(lv > lv_lo && t < s_info[lv - 1])
 		{
-			const int id = list[off + k];
-			const int2 c = child[id];
-			update_node(id, c.x, c.y, xyzr, nmass, bmin, bmax, ratio_sqr);
-			update_quad(id, c.x, c.y, xyzr, nmass, quad);
-			put_record(id, xyzr, nmass, quad, wr);
+			next_id = list[s_info[kRadixLevels + lv - 1] + t];
+			next = child[next_id];
 		}
-		__syncthreads();
+		if(id >= 0) { join_nodes<true>(id, c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr); }
+		if(s_info[lv] != 0) { __syncthreads(); }
+		id = next_id;
+		c = next;
 	}
 }
 
@@ -3824,9 +3862,6 @@ static nbh_status radix_alloc(nbh_tree* t)
 	return NBH_OK;
 }
 
-// Levels with fewer internal nodes than this run together in one work-group.
-constexpr int kRadixSmallLevel = 512;
-
 // Moments and walk records of the Morton tree (its structure, groups and level
 // lists already built): the leaves and the nodes inside the walk groups one wave
 // per group, then the nodes above them level by level from the longest prefix
@@ -3879,7 +3914,7 @@ static nbh_status radix_moments(nbh_ctx* ctx, nbh_tree* t, const double* y, cons
 		}
 		int lo = lv;
 		while(lo > 0 && t->level_count[lo - 1] < kRadixSmallLevel) { --lo; }
-		hipLaunchKernelGGL(k_radix_levels_small, dim3(1), dim3(1024), 0, ctx->stream, t->level_list, t->level_info, lv,
+		hipLaunchKernelGGL(k_radix_levels_small, dim3(1), dim3(kRadixSmallLevel), 0, ctx->stream, t->level_list, t->level_info, lv,
 		                   lo, t->child, t->xyzr, t->mass, t->bmin, t->bmax, t->quad, ratio_sqr, t->wrec);
 		NBH_LAUNCHED();
 		lv = lo - 1;
