@@ -21,6 +21,7 @@
 // Traversal: one target per work-item, targets in heap-leaf order (spatially
 // coherent), nodes as 32-byte AoS records {cm.xyz, crit_r2} plus mass.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -49,7 +50,8 @@ constexpr int kScanOneItems = 16;                    // scans of up to 16384 cou
 constexpr int kLocalSeg = 4096;                      // segments split in LDS, one work-group each
 constexpr int kLocalThreads = 1024;
 constexpr int kBoxParts = 2048;                      // partial boxes of the Morton tree's bounding box
-constexpr int kRadixLevels = 128;                    // prefix lengths of index-extended 63-bit keys: 0..127
+constexpr int kRadixTiers = 6;                       // sizes 64 * 32^t of the Morton tree's subtrees, t = 0..5
+constexpr int kMarkParts = 1024;                     // runs of group mark words that are counted together
 
 }  // namespace
 
@@ -95,13 +97,12 @@ struct nbh_tree {
 	// Morton radix tree (nbh_tree_build_radix; allocated on its first build)
 	int2*     child = nullptr;     // [n] children of internal ids 1..n-1
 	int*      parent = nullptr;    // [2n] parent id of every non-root node
-	int*      level = nullptr;     // [n] level of internal ids: the common prefix length of their keys
-	int*      level_list = nullptr;   // [n] internal ids level by level
-	int*      level_info = nullptr;   // [3 * kRadixLevels + 3] level counts, offsets, cursors; the group counts
+	uint8_t*  tier = nullptr;      // [n] tier of internal ids (k_radix_nodes)
+	int*      tier_list = nullptr; // [n + kRadixTiers] roots of the tiers' subtrees, tier by tier
 	int2*     gmark = nullptr;     // [n] group marks at their first sorted leaf (build scratch)
 	int2*     smark = nullptr;     // [n] super-group marks
 	int2*     wmark = nullptr;     // [n] walk group marks
-	uint32_t* flags = nullptr;     // [3n] build group, super-group and walk group flags, scanned in place
+	uint32_t* marks = nullptr;     // mark_words(n): bits of the three kinds of marks, counts, then the info counts
 	int4*     grp = nullptr;       // [n] build groups (node, first leaf, leaves)
 	int4*     wgrp = nullptr;      // [n] walk groups (node, first leaf, leaves, super-group)
 	int2*     sup = nullptr;       // [n / kRadixWalk + 1] super-groups (node, first leaf)
@@ -110,7 +111,8 @@ struct nbh_tree {
 	int       ngroups = 0;         // build groups, walk groups and super-groups of the last Morton build
 	int       nwalk = 0;
 	int       nsupers = 0;
-	int       level_count[kRadixLevels] = {};   // host copy of the level counts (refit)
+	int       tier_count[kRadixTiers] = {};   // subtrees of each tier of the last Morton build
+	hipEvent_t info_ready = nullptr;          // the counts of a Morton build are in pinned memory
 	int       two_slots = 0;       // super-groups the two-level buffers hold
 	bool      radix = false;       // the last build made the Morton tree
 	bool      radix_lean = false;  // Morton node arrays only where the build reads them back
@@ -967,7 +969,8 @@ __device__ inline uint64_t morton_cell(double x, double lo, double scale)
 // box[6] = bounding box lo.xyz hi.xyz of the bodies: scale = 2^21 / longest side
 __global__ void __launch_bounds__(256)
 k_morton_codes(const double* __restrict__ y, const double* __restrict__ mass, size_t n, const double* __restrict__ box,
-               uint64_t* __restrict__ keys, uint32_t* __restrict__ vals, double4* __restrict__ pk)
+               uint64_t* __restrict__ keys, uint32_t* __restrict__ vals, double4* __restrict__ pk,
+               uint32_t* __restrict__ marks, size_t words, int* __restrict__ parent)
 {
 	const double side = fmax(fmax(box[3] - box[0], box[4] - box[1]), box[5] - box[2]);
 	const double scale = side > 0.0 ? 2097152.0 / side : 0.0;
@@ -982,6 +985,9 @@ k_morton_codes(const double* __restrict__ y, const double* __restrict__ mass, si
 		vals[i] = static_cast<uint32_t>(i);
 		pk[i] = make_double4(x, yy, z, mass[i]);
 	}
+	// what the tree's kernels count and mark in, and the parents that no node has
+	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < words; i += stride) { marks[i] = 0; }
+	if(blockIdx.x == 0 && threadIdx.x < 2) { parent[threadIdx.x] = 0; }
 }
 
 // Bounding box partials of the positions, then the box (lo.xyz hi.xyz).
@@ -1074,20 +1080,74 @@ constexpr int kRadixWalk = 128;
 constexpr int kRadixSuper = 2048;
 constexpr int kRadixSuperMin = kRadixWalk + 1;   // at least two walk groups
 
+// Scratch of a Morton build: a bit per sorted position and kind of mark (a mark sits
+// at the first sorted position of its group's leaves), the marks counted by runs of
+// `run` words, and the info counts: subtrees of each tier, then build groups,
+// super-groups and walk groups.
+enum MarkKind { kMarkBuild, kMarkSuper, kMarkWalk };
+
+struct RadixMarks {
+	uint32_t* bits;
+	uint32_t* part;
+	int*      info;
+	size_t    words;      // of one kind
+	int       run;        // log2 of the positions of a part
+	__host__ __device__ int parts() const
+	{
+		return static_cast<int>(((words << 5) + (static_cast<size_t>(1) << run) - 1) >> run);
+	}
+};
+
+constexpr int kInfoCounts = kRadixTiers + 3;
+
+inline size_t mark_words(size_t n) { return 3 * ((n + 31) / 32) + 3 * kMarkParts + kInfoCounts; }
+
+inline RadixMarks radix_marks(uint32_t* p, size_t n)
+{
+	RadixMarks m;
+	m.words = (n + 31) / 32;
+	m.bits = p;
+	m.part = p + 3 * m.words;
+	m.info = reinterpret_cast<int*>(m.part + 3 * kMarkParts);
+	m.run = 11;           // one wave takes 64 words at a time
+	while(m.parts() > kMarkParts) { ++m.run; }
+	return m;
+}
+
+__device__ inline void put_mark(const RadixMarks& m, MarkKind kind, int2* __restrict__ mark, long long pos, int id,
+                                long long cnt)
+{
+	mark[pos] = make_int2(id, static_cast<int>(cnt));
+	atomicOr(&m.bits[kind * m.words + (pos >> 5)], 1u << (pos & 31));
+	atomicAdd(&m.part[kind * kMarkParts + (pos >> m.run)], 1u);
+}
+
+// Subtrees of the Morton tree by size: a node of more than 64 * 32^(t - 1) and at
+// most 64 * 32^t leaves has tier t (0: inside a build group).
+__device__ inline int radix_tier(long long cnt)
+{
+	int t = 0;
+	while(cnt > (static_cast<long long>(kRadixGroup) << (5 * t))) { ++t; }
+	return t;
+}
+
+// First entry of tier t in the list of subtree roots: a tier-t subtree has more than
+// 64 * 32^(t - 1) leaves.
+__host__ __device__ inline size_t tier_offset(size_t n, int t)
+{
+	size_t off = 0;
+	for(int k = 1; k < t; ++k) { off += n / (static_cast<size_t>(kRadixGroup) << (5 * (k - 1))) + 1; }
+	return off;
+}
+
 // Internal node i of [0, n - 1): its key range, split and children (ids), the
-// parent links of the children, its level (the common prefix length of its
-// keys, which grows strictly from a node to its children, so nodes of one level
-// are independent; -1 inside a walk group, whose nodes k_radix_group_moments
-// takes), the count of each level, and the marks of walk groups and
-// super-groups at the first sorted position of their leaves: (node id, leaves).
+// parent links of the children, its tier, the roots of the tiers' subtrees (in any
+// order) and the marks of build groups, walk groups and super-groups: (node id, leaves).
 __global__ void __launch_bounds__(256)
 k_radix_nodes(const uint64_t* __restrict__ k, long long n, int2* __restrict__ child, int* __restrict__ parent,
-              int* __restrict__ level, int* __restrict__ level_count, int2* __restrict__ gmark,
+              uint8_t* __restrict__ tier, int* __restrict__ tier_list, RadixMarks marks, int2* __restrict__ gmark,
               int2* __restrict__ smark, int2* __restrict__ wmark)
 {
-	__shared__ int hist[kRadixLevels];
-	for(int b = threadIdx.x; b < kRadixLevels; b += blockDim.x) { hist[b] = 0; }
-	__syncthreads();
 	const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
 	for(long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n - 1; i += stride)
 	{
@@ -1117,32 +1177,28 @@ k_radix_nodes(const uint64_t* __restrict__ k, long long n, int2* __restrict__ ch
 		parent[left] = id;
 		parent[right] = id;
 		const long long cnt = hi - lo + 1;
-		level[id] = cnt > kRadixGroup ? dnode : -1;
-		if(cnt > kRadixGroup) { atomicAdd(&hist[dnode], 1); }
-		const long long cl = gamma - lo + 1, cr = hi - gamma;
-		if(id == kRoot && cnt <= kRadixGroup) { gmark[lo] = make_int2(id, static_cast<int>(cnt)); }
-		if(id == kRoot && cnt <= kRadixSuper && cnt >= kRadixSuperMin) { smark[lo] = make_int2(id, static_cast<int>(cnt)); }
-		if(cnt > kRadixGroup)
+		tier[id] = static_cast<uint8_t>(radix_tier(cnt));
+		if(cnt <= kRadixGroup && id != kRoot) { continue; }     // inside a build group
+		const auto mark = [&](int node, long long pos, long long leaves, long long above, bool internal)
 		{
-			if(cl <= kRadixGroup) { gmark[lo] = make_int2(left, static_cast<int>(cl)); }
-			if(cr <= kRadixGroup) { gmark[gamma + 1] = make_int2(right, static_cast<int>(cr)); }
-		}
-		if(id == kRoot && cnt <= kRadixWalk) { wmark[lo] = make_int2(id, static_cast<int>(cnt)); }
-		if(cnt > kRadixWalk)
-		{
-			if(cl <= kRadixWalk) { wmark[lo] = make_int2(left, static_cast<int>(cl)); }
-			if(cr <= kRadixWalk) { wmark[gamma + 1] = make_int2(right, static_cast<int>(cr)); }
-		}
-		if(cnt > kRadixSuper)
-		{
-			if(cl <= kRadixSuper && cl >= kRadixSuperMin) { smark[lo] = make_int2(left, static_cast<int>(cl)); }
-			if(cr <= kRadixSuper && cr >= kRadixSuperMin) { smark[gamma + 1] = make_int2(right, static_cast<int>(cr)); }
-		}
-	}
-	__syncthreads();
-	for(int b = threadIdx.x; b < kRadixLevels; b += blockDim.x)
-	{
-		if(hist[b] != 0) { atomicAdd(&level_count[b], hist[b]); }
+			if(above > kRadixGroup && leaves <= kRadixGroup) { put_mark(marks, kMarkBuild, gmark, pos, node, leaves); }
+			if(above > kRadixWalk && leaves <= kRadixWalk) { put_mark(marks, kMarkWalk, wmark, pos, node, leaves); }
+			if(above > kRadixSuper && leaves <= kRadixSuper && leaves >= kRadixSuperMin)
+			{
+				put_mark(marks, kMarkSuper, smark, pos, node, leaves);
+			}
+			if(internal && leaves > kRadixGroup)
+			{
+				const int t = radix_tier(leaves);
+				if(above > (static_cast<long long>(kRadixGroup) << (5 * t)))
+				{
+					tier_list[tier_offset(static_cast<size_t>(n), t) + atomicAdd(&marks.info[t], 1)] = node;
+				}
+			}
+		};
+		if(id == kRoot) { mark(id, lo, cnt, LLONG_MAX, true); }
+		mark(left, lo, gamma - lo + 1, cnt, lo != gamma);
+		mark(right, gamma + 1, hi - gamma, cnt, hi != gamma + 1);
 	}
 }
 
@@ -1153,151 +1209,102 @@ k_fill_int(int* __restrict__ a, size_t count, int v)
 	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += stride) { a[i] = v; }
 }
 
-// 1 where a mark starts a group / super-group / walk group, for the scans that
-// number them.
-__global__ void __launch_bounds__(256)
-k_radix_flags(const int2* __restrict__ gmark, const int2* __restrict__ smark, const int2* __restrict__ wmark,
-              size_t n, uint32_t* __restrict__ gflag, uint32_t* __restrict__ sflag, uint32_t* __restrict__ wflag)
-{
-	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t p = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < n; p += stride)
-	{
-		gflag[p] = gmark[p].x != 0 ? 1u : 0u;
-		sflag[p] = smark[p].x != 0 ? 1u : 0u;
-		wflag[p] = wmark[p].x != 0 ? 1u : 0u;
-	}
-}
-
 // Build groups grp[g] and walk groups wgrp[w] = (node id, first sorted leaf,
-// leaves, super-group or -1), super-groups sup[s] = (node id, first sorted
-// leaf), all in Morton order (gidx / sidx / widx: exclusive scans of the flags);
-// info[0] = build groups, info[1] = super-groups, info[2] = walk groups.
+// leaves, super-group or -1) and super-groups sup[s] = (node id, first sorted
+// leaf), all in Morton order, and their counts; a wave per part of the marks, 64 words
+// at a time, from the counts of the parts before it.  The super-group of a walk group
+// is the last one marked at or before its first leaf, if its leaves reach it (both are
+// subtrees); it lies at most kRadixSuper positions, 64 words, back.  Latency bound:
+// with flags, three scans, a compaction, a search per walk group and cleared marks of
+// 8 bytes per position this took 85 us in 17 launches at 100003 bodies and 240 us at
+// 4M.
 __global__ void __launch_bounds__(256)
-k_radix_compact(const int2* __restrict__ gmark, const int2* __restrict__ smark, const int2* __restrict__ wmark,
-                const uint32_t* __restrict__ gidx, const uint32_t* __restrict__ sidx,
-                const uint32_t* __restrict__ widx, size_t n, int4* __restrict__ grp, int2* __restrict__ sup,
-                int4* __restrict__ wgrp, int* __restrict__ info)
+k_radix_groups(RadixMarks m, const int2* __restrict__ gmark, const int2* __restrict__ smark,
+               const int2* __restrict__ wmark, int4* __restrict__ grp, int2* __restrict__ sup,
+               int4* __restrict__ wgrp)
 {
-	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t p = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < n; p += stride)
+	const int lane = threadIdx.x & 63;
+	const int part = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, parts = m.parts();
+	if(part >= parts) { return; }
+	const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+	uint32_t base[3];
+	for(int kind = 0; kind < 3; ++kind)
 	{
-		const int2 g = gmark[p];
-		if(g.x != 0) { grp[gidx[p]] = make_int4(g.x, static_cast<int>(p), g.y, -1); }
-		const int2 sm = smark[p];
-		if(sm.x != 0) { sup[sidx[p]] = make_int2(sm.x, static_cast<int>(p)); }
-		const int2 w = wmark[p];
-		if(w.x != 0) { wgrp[widx[p]] = make_int4(w.x, static_cast<int>(p), w.y, -1); }
-		if(p == n - 1)
+		uint32_t v = 0;
+		for(int i = lane; i < part; i += 64) { v += m.part[kind * kMarkParts + i]; }
+		for(int sh = 32; sh > 0; sh >>= 1) { v += __shfl_xor(v, sh, 64); }
+		base[kind] = v;
+		if(part == parts - 1 && lane == 0)
 		{
-			info[0] = static_cast<int>(gidx[p] + (g.x != 0 ? 1u : 0u));
-			info[1] = static_cast<int>(sidx[p] + (sm.x != 0 ? 1u : 0u));
-			info[2] = static_cast<int>(widx[p] + (w.x != 0 ? 1u : 0u));
+			m.info[kRadixTiers + kind] = static_cast<int>(v + m.part[kind * kMarkParts + part]);
 		}
+	}
+	const size_t w0 = (static_cast<size_t>(part) << m.run) >> 5;
+	const size_t w1 = w0 + ((static_cast<size_t>(1) << m.run) >> 5) < m.words
+	                      ? w0 + ((static_cast<size_t>(1) << m.run) >> 5) : m.words;
+	// position of the last super-group mark before the words at hand, -1: none in reach
+	const auto last_of = [](uint32_t word, size_t first, uint64_t has)
+	{
+		const int src = 63 - __clzll(static_cast<long long>(has));
+		const uint32_t v = __shfl(word, src & 63, 64);
+		return has != 0 ? static_cast<int>((first + src) * 32 + 31 - __clz(static_cast<int>(v))) : -1;
+	};
+	int carry = -1;
+	if(w0 >= 64)
+	{
+		const uint32_t sw = m.bits[kMarkSuper * m.words + w0 - 64 + lane];
+		carry = last_of(sw, w0 - 64, __ballot(sw != 0));
+	}
+	for(size_t wb = w0; wb < w1; wb += 64)
+	{
+		const size_t w = wb + lane;
+		uint32_t word[3], at[3];
+		for(int kind = 0; kind < 3; ++kind)
+		{
+			word[kind] = w < w1 ? m.bits[kind * m.words + w] : 0;
+			const uint32_t c = __popc(word[kind]);
+			uint32_t x = c;
+			for(int sh = 1; sh < 64; sh <<= 1)
+			{
+				const uint32_t u = __shfl_up(x, sh, 64);
+				if(lane >= sh) { x += u; }
+			}
+			at[kind] = base[kind] + x - c;
+			base[kind] += __shfl(x, 63, 64);
+		}
+		const uint64_t has = __ballot(word[kMarkSuper] != 0);
+		const int before = last_of(word[kMarkSuper], wb, has & lt);
+		const int last = (has & lt) != 0 ? before : carry;
+		for(uint32_t b = word[kMarkBuild]; b != 0; b &= b - 1)
+		{
+			const int p = static_cast<int>(w * 32) + __builtin_ctz(b);
+			const int2 g = gmark[p];
+			grp[at[kMarkBuild]++] = make_int4(g.x, p, g.y, -1);
+		}
+		for(uint32_t b = word[kMarkWalk]; b != 0; b &= b - 1)
+		{
+			const int bit = __builtin_ctz(b), p = static_cast<int>(w * 32) + bit;
+			const int2 g = wmark[p];
+			const uint32_t mine = word[kMarkSuper] & (0xFFFFFFFFu >> (31 - bit));
+			const int sp = mine != 0 ? static_cast<int>(w * 32) + 31 - __clz(static_cast<int>(mine)) : last;
+			const bool in = sp >= 0 && sp + smark[sp < 0 ? 0 : sp].y > p;
+			wgrp[at[kMarkWalk]++] = make_int4(g.x, p, g.y, in ? static_cast<int>(at[kMarkSuper] + __popc(mine)) - 1 : -1);
+		}
+		for(uint32_t b = word[kMarkSuper]; b != 0; b &= b - 1)
+		{
+			const int p = static_cast<int>(w * 32) + __builtin_ctz(b);
+			sup[at[kMarkSuper]++] = make_int2(smark[p].x, p);
+		}
+		const int end = last_of(word[kMarkSuper], wb, has);
+		if(has != 0) { carry = end; }
 	}
 }
 
-// The super-group of each walk group: the last super-group starting at or
-// before the group's first leaf, if its node's leaves reach the group (a walk
-// group lies inside at most one super-group: both are subtrees).
-__global__ void __launch_bounds__(256)
-k_radix_group_super(int4* __restrict__ grp, const int2* __restrict__ sup, const int* __restrict__ info,
-                    const int2* __restrict__ child, size_t n)
+// LDS written by some lanes of a wave is read by others after this.
+__device__ inline void wave_sync()
 {
-	const int ng = info[2], ns = info[1];
-	for(int g = blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += gridDim.x * blockDim.x)
-	{
-		const int first = grp[g].y;
-		int lo = 0, hi = ns - 1, s = -1;
-		while(lo <= hi)
-		{
-			const int mid = (lo + hi) >> 1;
-			if(sup[mid].y <= first) { s = mid; lo = mid + 1; }
-			else { hi = mid - 1; }
-		}
-		if(s >= 0)
-		{
-			// leaves of the super-group's node: its first leaf and its size, found
-			// by walking its rightmost branch down to a leaf
-			int node = sup[s].x;
-			while(node < static_cast<int>(n)) { node = child[node].y; }
-			const int last = node - static_cast<int>(n);
-			if(first > last) { s = -1; }
-		}
-		grp[g].w = s;
-	}
-}
-
-// Offsets of the levels (exclusive scan of kRadixLevels counts, one work-group).
-__global__ void __launch_bounds__(kRadixLevels)
-k_radix_level_offsets(const int* __restrict__ count, int* __restrict__ offset, int* __restrict__ cursor)
-{
-	__shared__ int sh[kRadixLevels];
-	const int t = threadIdx.x;
-	sh[t] = count[t];
-	__syncthreads();
-	if(t == 0)
-	{
-		int run = 0;
-		for(int b = 0; b < kRadixLevels; ++b)
-		{
-			const int c = sh[b];
-			sh[b] = run;
-			run += c;
-		}
-	}
-	__syncthreads();
-	offset[t] = sh[t];
-	cursor[t] = 0;
-}
-
-// Internal ids above the walk groups listed level by level, kRadixListTile ids
-// per work-group: counts per level in LDS, one global reservation per level
-// present, then ranks from LDS counters.
-constexpr int kRadixListTile = 4096;
-__global__ void __launch_bounds__(256)
-k_radix_level_lists(const int* __restrict__ level, size_t n, const int* __restrict__ offset, int* __restrict__ cursor,
-                    int* __restrict__ list)
-{
-	__shared__ int cnt[kRadixLevels];
-	__shared__ int base[kRadixLevels];
-	for(int b = threadIdx.x; b < kRadixLevels; b += blockDim.x) { cnt[b] = 0; }
-	__syncthreads();
-	const size_t lo = 1 + static_cast<size_t>(blockIdx.x) * kRadixListTile;
-	const size_t hi = lo + kRadixListTile < n ? lo + kRadixListTile : n;
-	for(size_t id = lo + threadIdx.x; id < hi; id += blockDim.x)
-	{
-		const int lv = level[id];
-		if(lv >= 0) { atomicAdd(&cnt[lv], 1); }
-	}
-	__syncthreads();
-	for(int b = threadIdx.x; b < kRadixLevels; b += blockDim.x)
-	{
-		base[b] = cnt[b] != 0 ? offset[b] + atomicAdd(&cursor[b], cnt[b]) : 0;
-		cnt[b] = 0;
-	}
-	__syncthreads();
-	for(size_t id = lo + threadIdx.x; id < hi; id += blockDim.x)
-	{
-		const int lv = level[id];
-		if(lv >= 0) { list[base[lv] + atomicAdd(&cnt[lv], 1)] = static_cast<int>(id); }
-	}
-}
-
-// Moments of the internal ids list[0, count) of one level, from their children
-// (join_nodes, as the heap's levels); the levels run from the longest prefix to the
-// root, one launch each.
-__global__ void __launch_bounds__(256)
-k_radix_level(const int* __restrict__ list, int count, const int2* __restrict__ child, double4* __restrict__ xyzr,
-              double* __restrict__ nmass, double* __restrict__ bmin, double* __restrict__ bmax,
-              double* __restrict__ quad, double ratio_sqr, nbh_walk_rec* __restrict__ wr)
-{
-	const int stride = gridDim.x * blockDim.x;
-	for(int k = blockIdx.x * blockDim.x + threadIdx.x; k < count; k += stride)
-	{
-		const int id = list[k];
-		const int2 c = child[id];
-		join_nodes<true>(id, c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr);
-	}
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
 }
 
 // `v` of another lane of the same four (kCtrl: the source lane of each, 2 bits a lane).
@@ -1308,6 +1315,29 @@ __device__ inline double quad_lane(double v)
 	const int lo = __builtin_amdgcn_mov_dpp(static_cast<int>(b), kCtrl, 0xF, 0xF, true);
 	const int hi = __builtin_amdgcn_mov_dpp(static_cast<int>(b >> 32), kCtrl, 0xF, 0xF, true);
 	return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// A node's moments from its children's by four lanes: lane d (at most 2) takes
+// coordinate d of the mass centre and box, the diagonal second moment dd and one of
+// xy, xz, yz (combine_node and combine_quad, in their order).
+__device__ inline void join_part(const double (&cc)[2], const double (&mm)[2], const double (&lo2)[2],
+                                 const double (&hi2)[2], const double (&qd)[2], const double (&qo)[2], double& c,
+                                 double& m, double& lo, double& hi, double& qdd, double& qoo)
+{
+	m = mm[0] + mm[1];
+	c = (cc[0] * mm[0] + cc[1] * mm[1]) / m;
+	lo = min_ref(lo2[0], lo2[1]);
+	hi = max_ref(hi2[0], hi2[1]);
+	qdd = 0.0;
+	qoo = 0.0;
+	for(int side = 0; side < 2; ++side)
+	{
+		const double e = cc[side] - c;
+		// the factors of xy, xz, yz: (x, x, y) and (y, z, z)
+		const double ea = quad_lane<0xD0>(e), eb = quad_lane<0xE9>(e);
+		qdd += qd[side] + mm[side] * e * e;
+		qoo += qo[side] + mm[side] * ea * eb;
+	}
 }
 
 // Leaves and internal nodes of each build group (a subtree of at most
@@ -1331,7 +1361,7 @@ __device__ inline double quad_lane(double v)
 // moved), latency of the depths and memory alike.
 template <bool kBuild>
 __global__ void __launch_bounds__(kRadixGroup)
-k_radix_group_moments(const int4* __restrict__ grp, int n, const int2* __restrict__ child,
+k_radix_group_moments(const int4* __restrict__ grp, const int* __restrict__ groups, int n, const int2* __restrict__ child,
                       const uint32_t* __restrict__ order, const double4* __restrict__ pk, const double* __restrict__ y,
                       int32_t* __restrict__ body_n, double4* __restrict__ xyzr, double* __restrict__ nmass,
                       double* __restrict__ bmin, double* __restrict__ bmax, double* __restrict__ quad,
@@ -1347,191 +1377,340 @@ k_radix_group_moments(const int4* __restrict__ grp, int n, const int2* __restric
 	__shared__ int q[kG];          // internal nodes, breadth-first (at most kRadixGroup - 1)
 	__shared__ int start[kG + 1];  // first entry of each depth
 	const int lane = threadIdx.x;
-	const int4 gr = grp[blockIdx.x];
-	const int root = gr.x, first = gr.y, cnt = gr.z;
 	if(lane < 6) { sh[kZero + lane] = 0.0; }
-	if(lane < cnt)
+	const int count = *groups;
+	for(int g = blockIdx.x; g < count; g += gridDim.x)
 	{
-		const size_t sidx = static_cast<size_t>(first) + lane;
-		const size_t idx = static_cast<size_t>(n) + sidx;
-		double x, yy, z, m;
-		if constexpr(kBuild)
-		{
-			const uint32_t b = order[sidx];
-			const double4 p = pk[b];
-			x = p.x;
-			yy = p.y;
-			z = p.z;
-			m = p.w;
-			body_n[idx] = static_cast<int32_t>(b);
-			if(!lean || root >= n) { nmass[idx] = m; }
-		}
-		else
-		{
-			// the mass from the leaf's walk record, which every build writes
-			const size_t b = static_cast<uint32_t>(body_n[idx]);
-			x = y[b];
-			yy = y[n + b];
-			z = y[2 * static_cast<size_t>(n) + b];
-			m = wr[idx].m;
-		}
-		nbh_walk_rec r;
-		r.c = make_double4(x, yy, z, 0.0);
-		r.m = m;
-		for(int k = 0; k < 6; ++k) { r.q[k] = 0.0f; }
-		if(!lean || root >= n)
-		{
-			xyzr[idx] = r.c;
-			bmin[3 * idx] = x; bmin[3 * idx + 1] = yy; bmin[3 * idx + 2] = z;
-			bmax[3 * idx] = x; bmax[3 * idx + 1] = yy; bmax[3 * idx + 2] = z;
-		}
-		wr[idx] = r;
-		sh[kLC + 3 * lane] = x;
-		sh[kLC + 3 * lane + 1] = yy;
-		sh[kLC + 3 * lane + 2] = z;
-		sh[kLM + lane] = m;
-		const int id = first + 1 + lane;
-		s_child[lane] = id < n ? child[id] : make_int2(0, 0);
-	}
-	if(root >= n) { return; }              // a group of one leaf
-	const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-	if(lane == 0)
-	{
-		q[0] = root;
-		start[0] = 0;
-	}
-	int head = 0, tail = 1, depth = 0;
-	__syncthreads();
-	while(head < tail)
-	{
-		const int width = tail - head;
-		const bool act = lane < width;
-		const int2 c = act ? s_child[q[head + lane] - first - 1] : make_int2(n, n);
-		const bool li = c.x < n, ri = c.y < n;
-		const uint64_t bl = __ballot(li), br = __ballot(ri);
-		int pos = tail + __popcll(bl & lt) + __popcll(br & lt);
-		if(li) { q[pos++] = c.x; }
-		if(ri) { q[pos] = c.y; }
-		head = tail;
-		tail += __popcll(bl) + __popcll(br);
-		++depth;
-		if(lane == 0) { start[depth] = head; }
 		__syncthreads();
-	}
-	// depth d holds q[start[d], start[d + 1]); start[depth] == tail.  A child is
-	// leaf first + j (id n + first + j) or internal slot id - first - 1.
-	const int part = lane & 3, dim = part < 3 ? part : 2;
-	for(int d = depth - 1; d >= 0; --d)
-	{
-		const int end = start[d + 1];
-		for(int i = start[d] + (lane >> 2); i < end; i += kG / 4)
+		const int4 gr = grp[g];
+		const int root = gr.x, first = gr.y, cnt = gr.z;
+		if(lane < cnt)
 		{
-			const int k = q[i] - first - 1;
-			const int2 ch = s_child[k];
-			double cc[2], mm[2], lo2[2], hi2[2], qd[2], qo[2];
-			for(int side = 0; side < 2; ++side)
+			const size_t sidx = static_cast<size_t>(first) + lane;
+			const size_t idx = static_cast<size_t>(n) + sidx;
+			double x, yy, z, m;
+			if constexpr(kBuild)
 			{
-				const int cid = side == 0 ? ch.x : ch.y;
-				const bool leaf = cid >= n;
-				const int j = leaf ? cid - n - first : cid - first - 1;
-				const int at = 3 * j + dim;
-				const int qat = leaf ? kZero : kQ + 6 * j;
-				cc[side] = sh[(leaf ? kLC : kC) + at];
-				mm[side] = sh[(leaf ? kLM : kM) + j];
-				lo2[side] = sh[(leaf ? kLC : kLo) + at];
-				hi2[side] = sh[(leaf ? kLC : kHi) + at];
-				qd[side] = sh[qat + dim];
-				qo[side] = sh[qat + 3 + dim];
-			}
-			const double m = mm[0] + mm[1];
-			const double c = (cc[0] * mm[0] + cc[1] * mm[1]) / m;
-			double qdd = 0.0, qoo = 0.0;
-			for(int side = 0; side < 2; ++side)
-			{
-				const double e = cc[side] - c;
-				// the factors of xy, xz, yz: (x, x, y) and (y, z, z)
-				const double ea = quad_lane<0xD0>(e), eb = quad_lane<0xE9>(e);
-				qdd += qd[side] + mm[side] * e * e;
-				qoo += qo[side] + mm[side] * ea * eb;
-			}
-			if(part < 3)
-			{
-				sh[kC + 3 * k + part] = c;
-				sh[kLo + 3 * k + part] = min_ref(lo2[0], lo2[1]);
-				sh[kHi + 3 * k + part] = max_ref(hi2[0], hi2[1]);
-				sh[kQ + 6 * k + part] = qdd;
-				sh[kQ + 6 * k + 3 + part] = qoo;
+				const uint32_t b = order[sidx];
+				const double4 p = pk[b];
+				x = p.x;
+				yy = p.y;
+				z = p.z;
+				m = p.w;
+				body_n[idx] = static_cast<int32_t>(b);
+				if(!lean || root >= n) { nmass[idx] = m; }
 			}
 			else
 			{
-				sh[kM + k] = m;
+				// the mass from the leaf's walk record, which every build writes
+				const size_t b = static_cast<uint32_t>(body_n[idx]);
+				x = y[b];
+				yy = y[n + b];
+				z = y[2 * static_cast<size_t>(n) + b];
+				m = wr[idx].m;
 			}
-		}
-		__syncthreads();
-	}
-	const int k = lane + (root == first + 1 ? 0 : 1);
-	if(lane < cnt - 1)
-	{
-		const size_t gid = static_cast<size_t>(first) + 1 + k;
-		const double* lo = sh + kLo + 3 * k;
-		const double* hi = sh + kHi + 3 * k;
-		const double cx = sh[kC + 3 * k], cy = sh[kC + 3 * k + 1], cz = sh[kC + 3 * k + 2];
-		nbh_walk_rec rec;
-		rec.c = make_double4(cx, cy, cz, crit_radius(cx, cy, cz, lo, hi, ratio_sqr));
-		rec.m = sh[kM + k];
-		for(int e = 0; e < 6; ++e) { rec.q[e] = static_cast<float>(sh[kQ + 6 * k + e]); }
-		wr[gid] = rec;
-		if(!lean || gid == static_cast<size_t>(root))
-		{
-			xyzr[gid] = rec.c;
-			nmass[gid] = rec.m;
-			for(int e = 0; e < 3; ++e)
+			nbh_walk_rec r;
+			r.c = make_double4(x, yy, z, 0.0);
+			r.m = m;
+			for(int k = 0; k < 6; ++k) { r.q[k] = 0.0f; }
+			if(!lean || root >= n)
 			{
-				bmin[3 * gid + e] = lo[e];
-				bmax[3 * gid + e] = hi[e];
+				xyzr[idx] = r.c;
+				bmin[3 * idx] = x; bmin[3 * idx + 1] = yy; bmin[3 * idx + 2] = z;
+				bmax[3 * idx] = x; bmax[3 * idx + 1] = yy; bmax[3 * idx + 2] = z;
 			}
-			for(int e = 0; e < 6; ++e) { quad[6 * gid + e] = sh[kQ + 6 * k + e]; }
+			wr[idx] = r;
+			sh[kLC + 3 * lane] = x;
+			sh[kLC + 3 * lane + 1] = yy;
+			sh[kLC + 3 * lane + 2] = z;
+			sh[kLM + lane] = m;
+			const int id = first + 1 + lane;
+			s_child[lane] = id < n ? child[id] : make_int2(0, 0);
+		}
+		if(root >= n) { continue; }            // a group of one leaf
+		const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+		if(lane == 0)
+		{
+			q[0] = root;
+			start[0] = 0;
+		}
+		int head = 0, tail = 1, depth = 0;
+		__syncthreads();
+		while(head < tail)
+		{
+			const int width = tail - head;
+			const bool act = lane < width;
+			const int2 c = act ? s_child[q[head + lane] - first - 1] : make_int2(n, n);
+			const bool li = c.x < n, ri = c.y < n;
+			const uint64_t bl = __ballot(li), br = __ballot(ri);
+			int pos = tail + __popcll(bl & lt) + __popcll(br & lt);
+			if(li) { q[pos++] = c.x; }
+			if(ri) { q[pos] = c.y; }
+			head = tail;
+			tail += __popcll(bl) + __popcll(br);
+			++depth;
+			if(lane == 0) { start[depth] = head; }
+			__syncthreads();
+		}
+		// depth d holds q[start[d], start[d + 1]); start[depth] == tail.  A child is
+		// leaf first + j (id n + first + j) or internal slot id - first - 1.
+		const int part = lane & 3, dim = part < 3 ? part : 2;
+		for(int d = depth - 1; d >= 0; --d)
+		{
+			const int end = start[d + 1];
+			for(int i = start[d] + (lane >> 2); i < end; i += kG / 4)
+			{
+				const int k = q[i] - first - 1;
+				const int2 ch = s_child[k];
+				double cc[2], mm[2], lo2[2], hi2[2], qd[2], qo[2];
+				for(int side = 0; side < 2; ++side)
+				{
+					const int cid = side == 0 ? ch.x : ch.y;
+					const bool leaf = cid >= n;
+					const int j = leaf ? cid - n - first : cid - first - 1;
+					const int at = 3 * j + dim;
+					const int qat = leaf ? kZero : kQ + 6 * j;
+					cc[side] = sh[(leaf ? kLC : kC) + at];
+					mm[side] = sh[(leaf ? kLM : kM) + j];
+					lo2[side] = sh[(leaf ? kLC : kLo) + at];
+					hi2[side] = sh[(leaf ? kLC : kHi) + at];
+					qd[side] = sh[qat + dim];
+					qo[side] = sh[qat + 3 + dim];
+				}
+				double c, m, lo, hi, qdd, qoo;
+				join_part(cc, mm, lo2, hi2, qd, qo, c, m, lo, hi, qdd, qoo);
+				if(part < 3)
+				{
+					sh[kC + 3 * k + part] = c;
+					sh[kLo + 3 * k + part] = lo;
+					sh[kHi + 3 * k + part] = hi;
+					sh[kQ + 6 * k + part] = qdd;
+					sh[kQ + 6 * k + 3 + part] = qoo;
+				}
+				else
+				{
+					sh[kM + k] = m;
+				}
+			}
+			__syncthreads();
+		}
+		const int k = lane + (root == first + 1 ? 0 : 1);
+		if(lane < cnt - 1)
+		{
+			const size_t gid = static_cast<size_t>(first) + 1 + k;
+			const double* lo = sh + kLo + 3 * k;
+			const double* hi = sh + kHi + 3 * k;
+			const double cx = sh[kC + 3 * k], cy = sh[kC + 3 * k + 1], cz = sh[kC + 3 * k + 2];
+			nbh_walk_rec rec;
+			rec.c = make_double4(cx, cy, cz, crit_radius(cx, cy, cz, lo, hi, ratio_sqr));
+			rec.m = sh[kM + k];
+			for(int e = 0; e < 6; ++e) { rec.q[e] = static_cast<float>(sh[kQ + 6 * k + e]); }
+			wr[gid] = rec;
+			if(!lean || gid == static_cast<size_t>(root))
+			{
+				xyzr[gid] = rec.c;
+				nmass[gid] = rec.m;
+				for(int e = 0; e < 3; ++e)
+				{
+					bmin[3 * gid + e] = lo[e];
+					bmax[3 * gid + e] = hi[e];
+				}
+				for(int e = 0; e < 6; ++e) { quad[6 * gid + e] = sh[kQ + 6 * k + e]; }
+			}
 		}
 	}
 }
 
-// Levels lv_hi down to lv_lo, each of fewer nodes than kRadixSmallLevel, in one
-// work-group (info: the level counts, then their offsets in list): a node per
-// work-item, whose id and children are read a level ahead.  Bound by one dependent
-// chain of reads, FP64 divides and roots and a barrier per level: 79 us for the
-// levels of 100003 bodies (99 with the node's own moments read back for the second
-// moments and the record).
-constexpr int kRadixSmallLevel = 512;
-__global__ void __launch_bounds__(kRadixSmallLevel)
-k_radix_levels_small(const int* __restrict__ list, const int* __restrict__ info, int lv_hi, int lv_lo,
-                     const int2* __restrict__ child, double4* __restrict__ xyzr, double* __restrict__ nmass,
-                     double* __restrict__ bmin, double* __restrict__ bmax, double* __restrict__ quad,
-                     double ratio_sqr, nbh_walk_rec* __restrict__ wr)
+// Moments of the nodes of one tier, a work-group per subtree of more than
+// 64 * 32^(t - 1) and at most 64 * 32^t leaves: the nodes of the tier below its root are
+// listed breadth-first (at most 31 in a depth, as each holds more than 1/32 of the
+// leaves, and at most kTierDepth depths, as prefixes grow along a branch), then taken
+// depth by depth from the deepest, like a build group.  The first kTierNodes of
+// them and their children of lower tiers are held in LDS; any further ones, which
+// only branches of bodies at ever closer distances bring about, go through the node
+// arrays.  Latency bound (a read per depth down, divides per depth up); with a launch
+// or a barrier per prefix length in place of a depth of one subtree, the nodes above
+// the build groups took 88 us at 100003 bodies and 310 at 4M.
+constexpr int kTierDepth = 96;
+constexpr int kTierList = 31 * kTierDepth;
+constexpr int kTierNodes = 80;
+constexpr int kTierSlots = 2 * kTierNodes + 1;
+__global__ void __launch_bounds__(256)
+k_radix_tier(const int* __restrict__ roots, int t, int n, const int2* __restrict__ child,
+             const uint8_t* __restrict__ tier, double4* xyzr, double* nmass, double* bmin, double* bmax, double* quad,
+             double ratio_sqr, nbh_walk_rec* __restrict__ wr)
 {
-	__shared__ int s_info[2 * kRadixLevels];
-	const int t = threadIdx.x;
-	for(int i = t; i < 2 * kRadixLevels; i += blockDim.x) { s_info[i] = info[i]; }
-	__syncthreads();
-	int id = -1;
-	int2 c = make_int2(0, 0);
-	if(t < s_info[lv_hi])
+	// per slot: mass centre, mass, box, second moments
+	constexpr int kC = 0, kM = 3, kLo = 4, kHi = 7, kQ = 10, kPer = 17;
+	__shared__ double sh[kTierSlots * kPer];
+	__shared__ int q[kTierList];
+	__shared__ int start[kTierDepth + 1];
+	__shared__ int2 ref[kTierNodes];       // children: ~slot or node id
+	__shared__ int below[kTierNodes + 1];  // children of lower tiers
+	__shared__ int2 kids[64];              // children of the depth at hand
+	__shared__ int s_depth, s_below;
+	const int tid = threadIdx.x;
+	if(tid < 64)
 	{
-		id = list[s_info[kRadixLevels + lv_hi] + t];
-		c = child[id];
-	}
-	for(int lv = lv_hi; lv >= lv_lo; --lv)
-	{
-		int next_id = -1;
-		int2 next = make_int2(0, 0);
-		if(lv > lv_lo && t < s_info[lv - 1])
+		const uint64_t lt = tid == 0 ? 0ull : (~0ull >> (64 - tid));
+		if(tid == 0)
 		{
-			next_id = list[s_info[kRadixLevels + lv - 1] + t];
-			next = child[next_id];
+			const int root = roots[blockIdx.x];
+			q[0] = root;
+			start[0] = 0;
+			kids[0] = child[root];
 		}
-		if(id >= 0) { join_nodes<true>(id, c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr); }
-		if(s_info[lv] != 0) { __syncthreads(); }
-		id = next_id;
-		c = next;
+		int head = 0, tail = 1, depth = 0, nb = 0;
+		wave_sync();
+		while(head < tail)
+		{
+			const bool act = tid < tail - head;
+			const int2 c = act ? kids[tid] : make_int2(n, n);
+			bool in[2], out[2];
+			int2 kk[2];
+			for(int side = 0; side < 2; ++side)
+			{
+				const int id = side == 0 ? c.x : c.y;
+				const int safe = id < n ? id : kRoot;
+				kk[side] = child[safe];
+				in[side] = act && id < n && tier[safe] == t;
+				out[side] = act && !in[side] && head + tid < kTierNodes;
+			}
+			const uint64_t bl = __ballot(in[0]), br = __ballot(in[1]);
+			const uint64_t ol = __ballot(out[0]), orr = __ballot(out[1]);
+			int pos = tail + __popcll(bl & lt) + __popcll(br & lt);
+			int bpos = nb + __popcll(ol & lt) + __popcll(orr & lt);
+			int r[2];
+			wave_sync();
+			for(int side = 0; side < 2; ++side)
+			{
+				const int id = side == 0 ? c.x : c.y;
+				r[side] = id;
+				if(in[side])
+				{
+					if(pos < kTierNodes) { r[side] = ~pos; }
+					q[pos] = id;
+					kids[pos - tail] = kk[side];
+					++pos;
+				}
+				else if(out[side])
+				{
+					r[side] = ~(kTierNodes + bpos);
+					below[bpos++] = id;
+				}
+			}
+			if(act && head + tid < kTierNodes) { ref[head + tid] = make_int2(r[0], r[1]); }
+			head = tail;
+			tail += __popcll(bl) + __popcll(br);
+			nb += __popcll(ol) + __popcll(orr);
+			++depth;
+			if(tid == 0) { start[depth] = head; }
+			wave_sync();
+		}
+		if(tid == 0)
+		{
+			s_depth = depth;
+			s_below = nb;
+		}
+	}
+	__syncthreads();
+	const int depth = s_depth, nbelow = s_below, count = start[depth];
+	const int part = tid & 3, dim = part < 3 ? part : 2;
+	// one coordinate of a node's moments, from the node arrays
+	const auto read = [&](int id, double& c, double& m, double& lo, double& hi, double& qd, double& qo)
+	{
+		const size_t i = static_cast<size_t>(id);
+		c = reinterpret_cast<const double*>(xyzr)[4 * i + dim];
+		m = nmass[i];
+		lo = bmin[3 * i + dim];
+		hi = bmax[3 * i + dim];
+		qd = quad[6 * i + dim];
+		qo = quad[6 * i + 3 + dim];
+	};
+	const auto put = [&](int slot, double c, double m, double lo, double hi, double qd, double qo)
+	{
+		double* p = sh + slot * kPer;
+		if(part < 3)
+		{
+			p[kC + part] = c;
+			p[kLo + part] = lo;
+			p[kHi + part] = hi;
+			p[kQ + part] = qd;
+			p[kQ + 3 + part] = qo;
+		}
+		else
+		{
+			p[kM] = m;
+		}
+	};
+	for(int i = tid >> 2; i < nbelow; i += 64)
+	{
+		double c, m, lo, hi, qd, qo;
+		read(below[i], c, m, lo, hi, qd, qo);
+		put(kTierNodes + i, c, m, lo, hi, qd, qo);
+	}
+	for(int d = depth - 1; d >= 0 && start[d + 1] > kTierNodes; --d)
+	{
+		const int lo = start[d] > kTierNodes ? start[d] : kTierNodes;
+		const int i = lo + tid;
+		if(i < start[d + 1])
+		{
+			const int2 c = child[q[i]];
+			join_nodes<true>(q[i], c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr);
+		}
+		__syncthreads();
+	}
+	__syncthreads();
+	for(int d = depth - 1; d >= 0; --d)
+	{
+		const int i = start[d] + (tid >> 2);
+		const bool act = i < start[d + 1] && i < kTierNodes;
+		double cc[2] = {}, mm[2] = {}, lo2[2] = {}, hi2[2] = {}, qd[2] = {}, qo[2] = {};
+		if(act)
+		{
+			const int2 rr = ref[i];
+			for(int side = 0; side < 2; ++side)
+			{
+				const int r = side == 0 ? rr.x : rr.y;
+				if(r < 0)
+				{
+					const double* p = sh + ~r * kPer;
+					cc[side] = p[kC + dim];
+					mm[side] = p[kM];
+					lo2[side] = p[kLo + dim];
+					hi2[side] = p[kHi + dim];
+					qd[side] = p[kQ + dim];
+					qo[side] = p[kQ + 3 + dim];
+				}
+				else
+				{
+					read(r, cc[side], mm[side], lo2[side], hi2[side], qd[side], qo[side]);
+				}
+			}
+			double c, m, lo, hi, qdd, qoo;
+			join_part(cc, mm, lo2, hi2, qd, qo, c, m, lo, hi, qdd, qoo);
+			put(i, c, m, lo, hi, qdd, qoo);
+		}
+		__syncthreads();
+	}
+	if(tid < count && tid < kTierNodes)
+	{
+		const double* p = sh + tid * kPer;
+		const size_t id = static_cast<size_t>(q[tid]);
+		nbh_walk_rec rec;
+		rec.c = make_double4(p[kC], p[kC + 1], p[kC + 2],
+		                     crit_radius(p[kC], p[kC + 1], p[kC + 2], p + kLo, p + kHi, ratio_sqr));
+		rec.m = p[kM];
+		for(int e = 0; e < 6; ++e) { rec.q[e] = static_cast<float>(p[kQ + e]); }
+		wr[id] = rec;
+		xyzr[id] = rec.c;
+		nmass[id] = rec.m;
+		for(int e = 0; e < 3; ++e)
+		{
+			bmin[3 * id + e] = p[kLo + e];
+			bmax[3 * id + e] = p[kHi + e];
+		}
+		for(int e = 0; e < 6; ++e) { quad[6 * id + e] = p[kQ + e]; }
 	}
 }
 
@@ -3825,17 +4004,21 @@ static nbh_status radix_alloc(nbh_tree* t)
 		return NBH_OK;
 	}
 	const size_t n = t->n;
-	constexpr int kBufs = 14;
+	constexpr int kBufs = 13;
 	void* p[kBufs] = {};
-	const size_t sizes[kBufs] = { n * sizeof(int2), 2 * n * sizeof(int), n * sizeof(int), n * sizeof(int),
-	                              (3 * kRadixLevels + 3) * sizeof(int), n * sizeof(int2), n * sizeof(int2),
-	                              3 * n * sizeof(uint32_t), n * sizeof(int4),
+	const size_t sizes[kBufs] = { n * sizeof(int2), 2 * n * sizeof(int), n * sizeof(uint8_t),
+	                              (n + kRadixTiers) * sizeof(int), n * sizeof(int2), n * sizeof(int2),
+	                              mark_words(n) * sizeof(uint32_t), n * sizeof(int4),
 	                              (n / kRadixWalk + 1) * sizeof(int2), 6 * (kBoxParts + 1) * sizeof(double),
 	                              n * sizeof(double4), n * sizeof(int2), n * sizeof(int4) };
 	hipError_t e = hipSuccess;
 	for(int k = 0; k < kBufs && e == hipSuccess; ++k)
 	{
 		e = hipMalloc(&p[k], sizes[k]);
+	}
+	if(e == hipSuccess && t->info_ready == nullptr)
+	{
+		e = hipEventCreateWithFlags(&t->info_ready, hipEventDisableTiming);
 	}
 	if(e != hipSuccess)
 	{
@@ -3847,77 +4030,46 @@ static nbh_status radix_alloc(nbh_tree* t)
 	}
 	t->child = static_cast<int2*>(p[0]);
 	t->parent = static_cast<int*>(p[1]);
-	t->level = static_cast<int*>(p[2]);
-	t->level_list = static_cast<int*>(p[3]);
-	t->level_info = static_cast<int*>(p[4]);
-	t->gmark = static_cast<int2*>(p[5]);
-	t->smark = static_cast<int2*>(p[6]);
-	t->flags = static_cast<uint32_t*>(p[7]);
-	t->grp = static_cast<int4*>(p[8]);
-	t->sup = static_cast<int2*>(p[9]);
-	t->box = static_cast<double*>(p[10]);
-	t->pk = static_cast<double4*>(p[11]);
-	t->wmark = static_cast<int2*>(p[12]);
-	t->wgrp = static_cast<int4*>(p[13]);
+	t->tier = static_cast<uint8_t*>(p[2]);
+	t->tier_list = static_cast<int*>(p[3]);
+	t->gmark = static_cast<int2*>(p[4]);
+	t->smark = static_cast<int2*>(p[5]);
+	t->marks = static_cast<uint32_t*>(p[6]);
+	t->grp = static_cast<int4*>(p[7]);
+	t->sup = static_cast<int2*>(p[8]);
+	t->box = static_cast<double*>(p[9]);
+	t->pk = static_cast<double4*>(p[10]);
+	t->wmark = static_cast<int2*>(p[11]);
+	t->wgrp = static_cast<int4*>(p[12]);
 	return NBH_OK;
 }
 
-// Moments and walk records of the Morton tree (its structure, groups and level
-// lists already built): the leaves and the nodes inside the walk groups one wave
-// per group, then the nodes above them level by level from the longest prefix
-// up to the root.  build: leaves from `order` (sorted body numbers) and the
-// packed bodies, else from the body numbers of the last build and the
-// positions y.
-static nbh_status radix_moments(nbh_ctx* ctx, nbh_tree* t, const double* y, const uint32_t* order, double ratio,
-                                bool build)
+// Leaves, moments and walk records of the Morton tree's build groups, one wave per
+// group (any number of work-groups will do).  build: leaves from `order` (sorted body
+// numbers) and the packed bodies, else from the body numbers of the last build and
+// the positions y.
+static nbh_status radix_groups(nbh_ctx* ctx, nbh_tree* t, const double* y, const uint32_t* order, bool build,
+                               size_t blocks)
 {
-	const size_t n = t->n;
-	t->ratio = ratio;
-	const double ratio_sqr = ratio * ratio;
-	// the leaves and the nodes inside the walk groups, then the levels above them
-	if(build)
-	{
-		hipLaunchKernelGGL(k_radix_group_moments<true>, dim3(static_cast<unsigned>(t->ngroups)), dim3(kRadixGroup), 0,
-		                   ctx->stream, t->grp, static_cast<int>(n), t->child, order, t->pk, y, t->body_n, t->xyzr,
-		                   t->mass, t->bmin, t->bmax, t->quad, ratio_sqr, t->wrec, t->radix_lean ? 1 : 0);
-	}
-	else
-	{
-		hipLaunchKernelGGL(k_radix_group_moments<false>, dim3(static_cast<unsigned>(t->ngroups)), dim3(kRadixGroup),
-		                   0, ctx->stream, t->grp, static_cast<int>(n), t->child, order, t->pk, y, t->body_n,
-		                   t->xyzr, t->mass, t->bmin, t->bmax, t->quad, ratio_sqr, t->wrec, t->radix_lean ? 1 : 0);
-	}
+	const auto kernel = build ? k_radix_group_moments<true> : k_radix_group_moments<false>;
+	hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kRadixGroup), 0, ctx->stream, t->grp,
+	                   radix_marks(t->marks, t->n).info + kRadixTiers + kMarkBuild, static_cast<int>(t->n), t->child,
+	                   order, t->pk, y, t->body_n, t->xyzr, t->mass, t->bmin, t->bmax, t->quad, t->ratio * t->ratio,
+	                   t->wrec, t->radix_lean ? 1 : 0);
 	NBH_LAUNCHED();
-	int offset[kRadixLevels];
-	int run = 0;
-	for(int lv = 0; lv < kRadixLevels; ++lv)
+	return NBH_OK;
+}
+
+// The nodes above the build groups, tier by tier up to the root.
+static nbh_status radix_tiers(nbh_ctx* ctx, nbh_tree* t)
+{
+	for(int k = 1; k < kRadixTiers; ++k)
 	{
-		offset[lv] = run;
-		run += t->level_count[lv];
-	}
-	int lv = kRadixLevels - 1;
-	while(lv >= 0)
-	{
-		if(t->level_count[lv] == 0)
-		{
-			--lv;
-			continue;
-		}
-		if(t->level_count[lv] >= kRadixSmallLevel)
-		{
-			hipLaunchKernelGGL(k_radix_level, dim3(nbh::grid_for(ctx, t->level_count[lv], 256)), dim3(256), 0,
-			                   ctx->stream, t->level_list + offset[lv], t->level_count[lv], t->child, t->xyzr, t->mass,
-			                   t->bmin, t->bmax, t->quad, ratio_sqr, t->wrec);
-			NBH_LAUNCHED();
-			--lv;
-			continue;
-		}
-		int lo = lv;
-		while(lo > 0 && t->level_count[lo - 1] < kRadixSmallLevel) { --lo; }
-		hipLaunchKernelGGL(k_radix_levels_small, dim3(1), dim3(kRadixSmallLevel), 0, ctx->stream, t->level_list, t->level_info, lv,
-		                   lo, t->child, t->xyzr, t->mass, t->bmin, t->bmax, t->quad, ratio_sqr, t->wrec);
+		if(t->tier_count[k] == 0) { continue; }
+		hipLaunchKernelGGL(k_radix_tier, dim3(static_cast<unsigned>(t->tier_count[k])), dim3(256), 0, ctx->stream,
+		                   t->tier_list + tier_offset(t->n, k), k, static_cast<int>(t->n), t->child, t->tier, t->xyzr,
+		                   t->mass, t->bmin, t->bmax, t->quad, t->ratio * t->ratio, t->wrec);
 		NBH_LAUNCHED();
-		lv = lo - 1;
 	}
 	return NBH_OK;
 }
@@ -3938,64 +4090,49 @@ nbh_status nbh_tree_build_radix(nbh_ctx* ctx, nbh_tree* t, const double* y, cons
 	hipLaunchKernelGGL(k_box_final, dim3(1), dim3(256), 0, ctx->stream, t->box + 6, static_cast<int>(parts), t->box);
 	NBH_LAUNCHED();
 	hipLaunchKernelGGL(k_morton_codes, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, y, mass, n,
-	                   t->box, t->keys, t->vals, t->pk);
+	                   t->box, t->keys, t->vals, t->pk, t->marks, mark_words(n), t->parent);
 	NBH_LAUNCHED();
 	uint32_t* order = nullptr;
 	// 63-bit keys: 8 passes, so the sorted keys end where they started
 	NBH_TRY(nbh::sort_pairs(ctx, t->keys, t->vals, t->keys + n, t->vals + n, n, 63, t->counts, &order));
-	const unsigned gn = nbh::grid_for(ctx, 2 * n, 256);
-	hipLaunchKernelGGL(k_fill_int, dim3(gn), dim3(256), 0, ctx->stream, t->parent, 2 * n, 0);
-	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_fill_int, dim3(gn), dim3(256), 0, ctx->stream, reinterpret_cast<int*>(t->gmark), 2 * n, 0);
-	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_fill_int, dim3(gn), dim3(256), 0, ctx->stream, reinterpret_cast<int*>(t->smark), 2 * n, 0);
-	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_fill_int, dim3(gn), dim3(256), 0, ctx->stream, reinterpret_cast<int*>(t->wmark), 2 * n, 0);
-	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, ctx->stream, t->level_info,
-	                   static_cast<size_t>(3 * kRadixLevels + 3), 0);
-	NBH_LAUNCHED();
+	const RadixMarks marks = radix_marks(t->marks, n);
 	hipLaunchKernelGGL(k_radix_nodes, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, t->keys,
-	                   static_cast<long long>(n), t->child, t->parent, t->level, t->level_info, t->gmark, t->smark,
-	                   t->wmark);
+	                   static_cast<long long>(n), t->child, t->parent, t->tier, t->tier_list, marks, t->gmark,
+	                   t->smark, t->wmark);
 	NBH_LAUNCHED();
-	// groups and super-groups numbered in Morton order
-	hipLaunchKernelGGL(k_radix_flags, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, t->gmark,
-	                   t->smark, t->wmark, n, t->flags, t->flags + n, t->flags + 2 * n);
+	hipLaunchKernelGGL(k_radix_groups, dim3(static_cast<unsigned>((marks.parts() + 3) / 4)), dim3(256), 0, ctx->stream,
+	                   marks, t->gmark, t->smark, t->wmark, t->grp, t->sup, t->wgrp);
 	NBH_LAUNCHED();
-	NBH_TRY(scan_exclusive(ctx, t->flags, n, t->scan_part));
-	NBH_TRY(scan_exclusive(ctx, t->flags + n, n, t->scan_part));
-	NBH_TRY(scan_exclusive(ctx, t->flags + 2 * n, n, t->scan_part));
-	int* info = t->level_info + 3 * kRadixLevels;
-	hipLaunchKernelGGL(k_radix_compact, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, t->gmark,
-	                   t->smark, t->wmark, t->flags, t->flags + n, t->flags + 2 * n, n, t->grp, t->sup, t->wgrp, info);
-	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_radix_group_super, dim3(nbh::grid_for(ctx, n / 16 + 1, 256)), dim3(256), 0, ctx->stream,
-	                   t->wgrp, t->sup, info, t->child, n);
-	NBH_LAUNCHED();
-	// internal ids listed by level
-	hipLaunchKernelGGL(k_radix_level_offsets, dim3(1), dim3(kRadixLevels), 0, ctx->stream, t->level_info,
-	                   t->level_info + kRadixLevels, t->level_info + 2 * kRadixLevels);
-	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_radix_level_lists, dim3(static_cast<unsigned>((n - 1 + kRadixListTile - 1) / kRadixListTile)),
-	                   dim3(256), 0, ctx->stream, t->level, n, t->level_info + kRadixLevels,
-	                   t->level_info + 2 * kRadixLevels, t->level_list);
-	NBH_LAUNCHED();
-	// the level counts and the group counts drive the launches that follow
-	constexpr size_t kInfoBytes = (3 * kRadixLevels + 3) * sizeof(int);
+	// the counts drive the launches that follow the build groups' moments, which run
+	// while they travel (a group holds some 40 leaves)
+	constexpr size_t kInfoBytes = kInfoCounts * sizeof(int);
 	NBH_TRY(nbh::pinned(ctx, kInfoBytes));
 	const int* host_info = reinterpret_cast<const int*>(ctx->pinned);
-	NBH_HIP(hipMemcpyAsync(ctx->pinned, t->level_info, kInfoBytes, hipMemcpyDeviceToHost, ctx->stream));
-	NBH_HIP(hipStreamSynchronize(ctx->stream));
-	for(int lv = 0; lv < kRadixLevels; ++lv) { t->level_count[lv] = host_info[lv]; }
-	t->ngroups = host_info[3 * kRadixLevels];
-	t->nsupers = host_info[3 * kRadixLevels + 1];
-	t->nwalk = host_info[3 * kRadixLevels + 2];
+	NBH_HIP(hipMemcpyAsync(ctx->pinned, marks.info, kInfoBytes, hipMemcpyDeviceToHost, ctx->stream));
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	NBH_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+	if(capture != hipStreamCaptureStatusNone)
+	{
+		NBH_HIP(hipStreamSynchronize(ctx->stream));      // not in a capture: the host needs the counts
+	}
+	NBH_HIP(hipEventRecord(t->info_ready, ctx->stream));
+	t->ratio = ratio;
+	NBH_TRY(radix_groups(ctx, t, y, order, true, n / 32 + 1));
+	NBH_HIP(hipEventSynchronize(t->info_ready));
+	for(int k = 0; k < kRadixTiers; ++k)
+	{
+		t->tier_count[k] = host_info[k];
+		NBH_CHECK(k == 0 || (t->tier_count[k] >= 0 && tier_offset(n, k) + t->tier_count[k] <= tier_offset(n, k + 1)),
+		          "bad count %d of tier %d", t->tier_count[k], k);
+	}
+	t->ngroups = host_info[kRadixTiers + kMarkBuild];
+	t->nsupers = host_info[kRadixTiers + kMarkSuper];
+	t->nwalk = host_info[kRadixTiers + kMarkWalk];
 	NBH_CHECK(t->ngroups >= 1 && static_cast<size_t>(t->ngroups) <= n, "bad group count %d", t->ngroups);
 	NBH_CHECK(t->nwalk >= 1 && t->nwalk <= t->ngroups, "bad walk group count %d", t->nwalk);
 	NBH_CHECK(t->nsupers >= 0 && static_cast<size_t>(t->nsupers) <= n / kRadixWalk + 1,
 	          "bad super-group count %d", t->nsupers);
-	NBH_TRY(radix_moments(ctx, t, y, order, ratio, true));
+	NBH_TRY(radix_tiers(ctx, t));
 	t->radix = true;
 	t->built = true;
 	return NBH_OK;
@@ -4032,12 +4169,13 @@ nbh_status nbh_tree_destroy(nbh_tree* t)
 	void* ptrs[] = { t->list[0], t->list[1], t->list[2], t->tmp, t->side, t->keys, t->vals, t->counts, t->scan_part,
 	                 t->xyzr, t->mass, t->bmin, t->bmax, t->quad, t->wrec, t->body_n, t->counters,
 	                 t->two_lists, t->two_count, t->two_coef, t->far_list, t->far_count,
-	                 t->child, t->parent, t->level, t->level_list, t->level_info, t->gmark, t->smark, t->flags,
+	                 t->child, t->parent, t->tier, t->tier_list, t->gmark, t->smark, t->marks,
 	                 t->grp, t->sup, t->box, t->pk, t->wmark, t->wgrp };
 	for(void* p : ptrs)
 	{
 		if(p != nullptr) { (void)hipFree(p); }
 	}
+	if(t->info_ready != nullptr) { (void)hipEventDestroy(t->info_ready); }
 	delete t;
 	return NBH_OK;
 }
@@ -4110,7 +4248,9 @@ nbh_status nbh_tree_refit(nbh_ctx* ctx, nbh_tree* t, const double* y, double rat
 	nbh::scoped_timer timer(ctx, "tree_refit");
 	if(t->radix)
 	{
-		return radix_moments(ctx, t, y, nullptr, ratio, false);
+		t->ratio = ratio;
+		NBH_TRY(radix_groups(ctx, t, y, nullptr, false, static_cast<size_t>(t->ngroups)));
+		return radix_tiers(ctx, t);
 	}
 	return moments(ctx, t, y, nullptr, ratio, false);
 }

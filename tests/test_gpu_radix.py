@@ -116,6 +116,42 @@ def test_radix_sort_tile_edges(ctx, kind, n):
     t.close()
 
 
+def _cusps(n, seed):
+    """Bodies that close in on 6 points, two to a halving of the distance: branches of
+    single bodies, so that a subtree of 2048 leaves has over 80 nodes above its build
+    groups."""
+    rng = np.random.default_rng(seed)
+    centre = 1000.0 * rng.random((6, 3))[np.arange(n) % 6]
+    u = rng.standard_normal((n, 3))
+    shell = np.arange(n) // 6 // 2 % 18
+    pos = centre + 50.0 * 0.5 ** shell[:, None] * u / np.linalg.norm(u, axis=1)[:, None]
+    return np.concatenate([pos[:, 0], pos[:, 1], pos[:, 2], np.zeros(3 * n)]), rng.random(n) + 0.1
+
+
+@pytest.mark.parametrize("kind,n", [("plummer", 65), ("plummer", 129), ("plummer", 2049), ("plummer", 70001),
+                                    ("cusps", 1200), ("cusps", 2048), ("cusps", 30011)])
+def test_radix_tier_edges(ctx, kind, n):
+    """Trees whose root is the smallest above a build group, a walk group and a
+    2048-leaf subtree, and of several tiers; build and refit bit for bit, and every
+    body in one walk group, under the super-group that holds it (a lost or doubled
+    body, or a wrong list, shows in the accelerations against the direct sum)."""
+    y, m = _cusps(n, n) if kind == "cusps" else _state(kind, n, n)
+    ratio = 1.6
+    o = oracle_lib.radix_build(y, m, ratio)
+    t = RTree(ctx, y, m, ratio)
+    for step in ("build", "refit"):
+        if step == "refit":
+            native.check(ctx.lib.nbh_tree_refit(ctx.h, t.h, t.dy.ptr, ratio), "refit")
+        g = t.arrays()
+        for k in ("cm", "mass", "crit", "bmin", "bmax"):
+            assert np.array_equal(g[k][1:2 * n], o[k][1:2 * n]), (step, k)
+    idx = np.arange(0, n, max(1, n // 1000))
+    a0 = _direct(y, m, idx)
+    e2, e1 = _rms(t.walk("local2"), a0, n, idx), _rms(t.walk("local"), a0, n, idx)
+    assert e2[0] < 2e-2 and e2[0] < 1.25 * e1[0] + 1e-6, (e2, e1)
+    t.close()
+
+
 @pytest.mark.parametrize("kind,n,seed", [("plummer", 3, 8), ("plummer", 100, 10), ("plummer", 3000, 2),
                                          ("plummer", 1 << 15, 5), ("coincident", 2500, 6)])
 def test_radix_lean_walks_equal(ctx, kind, n, seed):
