@@ -43,6 +43,7 @@ constexpr int kSortPasses = 8;
 constexpr int kPartThreads = 256;
 constexpr int kPartItems = 4;
 constexpr int kPartTile = kPartThreads * kPartItems;   // 1024 entries per work-group
+constexpr size_t kPartSum = 4096;                    // tiles of a segment that a tile sums itself, without a scan
 constexpr int kScanThreads = 256;
 constexpr int kScanParts = 1024;                     // chunks of one scan
 constexpr int kScanOneThreads = 1024;
@@ -601,19 +602,19 @@ k_mark_side(const uint32_t* __restrict__ list_a, uint8_t* __restrict__ side, siz
 	}
 }
 
-// rights[b] = number of upper-half bodies in tile b of `list`
+// The two lists that a level partitions: from in[] to out[].
+struct part_lists {
+	const uint32_t* in[2];
+	uint32_t*       out[2];
+};
+
+// rights[list][b] = number of upper-half bodies in tile b of a list (blockIdx.y)
 __global__ void __launch_bounds__(kPartThreads)
-k_part_count(const uint32_t* __restrict__ list, const uint8_t* __restrict__ side, size_t n,
-             uint32_t* __restrict__ rights)
+k_part_count(part_lists l, const uint8_t* __restrict__ side, uint32_t* __restrict__ rights)
 {
 	__shared__ uint32_t wsum[kPartThreads / 64];
-	size_t base = static_cast<size_t>(blockIdx.x) * kPartTile + static_cast<size_t>(threadIdx.x) * kPartItems;
-	uint32_t c = 0;
-	for(int k = 0; k < kPartItems; ++k)
-	{
-		size_t p = base + k;
-		if(p < n) { c += side[list[p]]; }
-	}
+	const uint4 body = reinterpret_cast<const uint4*>(l.in[blockIdx.y])[blockIdx.x * kPartThreads + threadIdx.x];
+	uint32_t c = side[body.x] + side[body.y] + side[body.z] + side[body.w];
 	for(int off = 32; off > 0; off >>= 1) { c += __shfl_down(c, off, 64); }
 	if((threadIdx.x & 63) == 0) { wsum[threadIdx.x >> 6] = c; }
 	__syncthreads();
@@ -621,64 +622,68 @@ k_part_count(const uint32_t* __restrict__ list, const uint8_t* __restrict__ side
 	{
 		uint32_t t = 0;
 		for(int w = 0; w < kPartThreads / 64; ++w) { t += wsum[w]; }
-		rights[blockIdx.x] = t;
+		rights[blockIdx.y * gridDim.x + blockIdx.x] = t;
 	}
 }
 
-// Stable partition of every segment of `list` into lower-half then upper-half
-// bodies (flags in `side`), written to `out`.  `tile_off` holds, per tile, the
-// number of upper-half bodies in all tiles before it (exclusive scan over the
-// whole list); for segments of at least one tile the count inside the segment
-// is that minus the value at the segment's first tile.  Smaller segments are
-// handled inside the tile.
+// Stable partition of every segment (at least a tile) of both lists into lower-half
+// then upper-half bodies (flags in `side`).  The upper-half bodies of the segment's
+// tiles before this one are summed here from `rights`, or, scanned != 0, `rights` is
+// its exclusive scan.  The list of the next level's axis (next, -1: none) also sets
+// that level's flags, side_next.  Latency bound at 2^18 bodies: a list and a step at a
+// time (mark, then count, scan and scatter twice), the six levels above the LDS took
+// 190 us there, now 70.
 __global__ void __launch_bounds__(kPartThreads)
-k_part_scatter(const uint32_t* __restrict__ list, const uint8_t* __restrict__ side, size_t n, size_t seg,
-               const uint32_t* __restrict__ tile_off, uint32_t* __restrict__ out)
+k_part_scatter(part_lists l, const uint8_t* __restrict__ side, size_t seg, const uint32_t* __restrict__ rights,
+               int scanned, int next, uint8_t* __restrict__ side_next)
 {
-	__shared__ uint32_t excl[kPartTile];
-	__shared__ uint32_t tsum[kPartThreads];
-	const size_t tile = static_cast<size_t>(blockIdx.x) * kPartTile;
-	const int tb = threadIdx.x * kPartItems;
-	uint32_t body[kPartItems];
-	uint8_t fl[kPartItems];
-	uint32_t c = 0;
+	constexpr int kWaves = kPartThreads / 64;
+	__shared__ uint32_t wsum[kWaves], wbefore[kWaves];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const uint32_t* r = rights + blockIdx.y * gridDim.x;
+	const uint32_t first = blockIdx.x & ~static_cast<uint32_t>(seg / kPartTile - 1);
+	const uint4 b4 = reinterpret_cast<const uint4*>(l.in[blockIdx.y])[blockIdx.x * kPartThreads + threadIdx.x];
+	const uint32_t body[kPartItems] = {b4.x, b4.y, b4.z, b4.w};
+	uint32_t fl[kPartItems], c = 0, before = 0;
 	for(int k = 0; k < kPartItems; ++k)
 	{
-		size_t p = tile + tb + k;
-		body[k] = p < n ? list[p] : 0;
-		fl[k] = p < n ? side[body[k]] : 0;
-		excl[tb + k] = c;
+		fl[k] = side[body[k]];
 		c += fl[k];
 	}
-	tsum[threadIdx.x] = c;
-	__syncthreads();
-	for(int off = 1; off < kPartThreads; off <<= 1)
+	if(scanned != 0)
 	{
-		uint32_t v = threadIdx.x >= static_cast<unsigned>(off) ? tsum[threadIdx.x - off] : 0;
-		__syncthreads();
-		tsum[threadIdx.x] += v;
-		__syncthreads();
+		before = threadIdx.x == 0 ? r[blockIdx.x] - r[first] : 0;
 	}
-	uint32_t add = threadIdx.x == 0 ? 0 : tsum[threadIdx.x - 1];
-	for(int k = 0; k < kPartItems; ++k) { excl[tb + k] += add; }
+	else
+	{
+		for(uint32_t i = first + threadIdx.x; i < blockIdx.x; i += kPartThreads) { before += r[i]; }
+	}
+	uint32_t x = c;
+	for(int off = 1; off < 64; off <<= 1)
+	{
+		const uint32_t u = __shfl_up(x, off, 64);
+		if(lane >= off) { x += u; }
+		before += __shfl_xor(before, off, 64);
+	}
+	if(lane == 63)
+	{
+		wsum[wave] = x;
+		wbefore[wave] = before;
+	}
 	__syncthreads();
+	uint32_t ex = x - c;
+	for(int w = 0; w < kWaves; ++w) { ex += wbefore[w] + (w < wave ? wsum[w] : 0); }
+	uint32_t* out = l.out[blockIdx.y];
+	const bool flags = static_cast<int>(blockIdx.y) == next;
 	const size_t half = seg >> 1;
+	const size_t p0 = static_cast<size_t>(blockIdx.x) * kPartTile + threadIdx.x * kPartItems;
+	const size_t upper = (p0 & ~(seg - 1)) + half;
 	for(int k = 0; k < kPartItems; ++k)
 	{
-		size_t p = tile + tb + k;
-		if(p >= n) { continue; }
-		size_t seg_start = p & ~(seg - 1);
-		uint32_t before;
-		if(seg >= static_cast<size_t>(kPartTile))
-		{
-			before = tile_off[blockIdx.x] - tile_off[seg_start / kPartTile] + excl[tb + k];
-		}
-		else
-		{
-			before = excl[tb + k] - excl[seg_start - tile];
-		}
-		size_t pos = fl[k] ? seg_start + half + before : p - before;
+		const size_t pos = fl[k] ? upper + ex : p0 + k - ex;
 		out[pos] = body[k];
+		if(flags) { side_next[body[k]] = (pos & (half - 1)) >= half >> 1 ? 1 : 0; }
+		ex += fl[k];
 	}
 }
 
@@ -687,16 +692,20 @@ k_part_scatter(const uint32_t* __restrict__ list, const uint8_t* __restrict__ si
 // segment, in LDS.  Bodies get local numbers (their position in list0's
 // segment, through the global table g2l) so that the side flags live in LDS.
 // Only the final order is written back, to list0: after the last level every
-// segment holds one body and the three lists agree.
+// segment holds one body and the three lists agree.  A work-item has kLocalItems
+// positions of both lists that move, their counts in one word, and writes the next
+// level's flags with the list that sets them: two barriers a level, 38 us at 2^18
+// bodies, 87 with eleven.
+constexpr int kLocalItems = kLocalSeg / kLocalThreads;
+static_assert(kLocalItems == 4 && kLocalSeg < (1 << 16), "positions of a work-item in 8 bytes, two counts in a word");
+
 __global__ void __launch_bounds__(kLocalThreads)
 k_split_local(uint32_t* __restrict__ list0, const uint32_t* __restrict__ list1, const uint32_t* __restrict__ list2,
               uint32_t* __restrict__ g2l, int seg0, int first_level, int levels)
 {
-	__shared__ uint16_t ls[3][kLocalSeg];
-	__shared__ uint16_t tmp[kLocalSeg];
-	__shared__ uint16_t excl[kLocalSeg];
+	__shared__ __align__(8) uint16_t ls[5][kLocalSeg];     // three lists and two to write
 	__shared__ uint32_t l2g[kLocalSeg];
-	__shared__ uint8_t side[kLocalSeg];
+	__shared__ uint8_t side[2][kLocalSeg];
 	__shared__ uint32_t ws[kLocalThreads / 64];
 	const size_t base = static_cast<size_t>(blockIdx.x) * seg0;
 	const int lane = threadIdx.x & 63;
@@ -715,69 +724,73 @@ k_split_local(uint32_t* __restrict__ list0, const uint32_t* __restrict__ list1, 
 		ls[2][p] = static_cast<uint16_t>(g2l[list2[base + p]]);
 	}
 	__syncthreads();
-	// work-item t owns positions [t * per, t * per + per) of a list
-	const int per = (seg0 + kLocalThreads - 1) / kLocalThreads;
-	const int p0 = static_cast<int>(threadIdx.x) * per;
+	{
+		const uint16_t* l = ls[first_level % 3];
+		for(int p = threadIdx.x; p < seg0; p += kLocalThreads) { side[0][l[p]] = p >= seg0 >> 1 ? 1 : 0; }
+	}
+	__syncthreads();
+	const int p0 = static_cast<int>(threadIdx.x) * kLocalItems;
+	int cur0 = 0, cur1 = 1, cur2 = 2, free0 = 3, free1 = 4;   // rows of ls: the lists, the two to write
 	for(int level = first_level; level < levels; ++level)
 	{
 		const int seg = seg0 >> (level - first_level);
 		const int half = seg >> 1;
 		const int a = level % 3;
-		for(int p = threadIdx.x; p < seg0; p += kLocalThreads)
+		const uint8_t* now = side[(level - first_level) & 1];
+		uint8_t* then = side[~(level - first_level) & 1];
+		// the list of the next level's axis first
+		const int from[2] = {a == 0 ? cur1 : a == 1 ? cur2 : cur0, a == 0 ? cur2 : a == 1 ? cur0 : cur1};
+		const int to[2] = {free0, free1};
+		uint16_t id[2][kLocalItems];
+		uint32_t up[kLocalItems], c = 0;       // flags of the two lists, counts: 16 bits each
+		for(int b = 0; b < 2; ++b)
 		{
-			side[ls[a][p]] = (p & (seg - 1)) >= half ? 1 : 0;
+			const ushort4 v = *reinterpret_cast<const ushort4*>(&ls[from[b]][p0]);
+			id[b][0] = v.x; id[b][1] = v.y; id[b][2] = v.z; id[b][3] = v.w;
+		}
+		for(int k = 0; k < kLocalItems; ++k)
+		{
+			const bool in = p0 + k < seg0;
+			up[k] = in ? now[id[0][k]] | static_cast<uint32_t>(now[id[1][k]]) << 16 : 0;
+			c += up[k];
+		}
+		uint32_t x = c;
+		for(int off = 1; off < 64; off <<= 1)
+		{
+			const uint32_t u = __shfl_up(x, off, 64);
+			if(lane >= off) { x += u; }
+		}
+		if(lane == 63) { ws[wave] = x; }
+		__syncthreads();
+		uint32_t ex = x - c;
+		for(int w = 0; w < wave; ++w) { ex += ws[w]; }
+		for(int k = 0; k < kLocalItems; ++k)
+		{
+			const int p = p0 + k;
+			if(p < seg0)
+			{
+				const int start = p & ~(seg - 1);
+				for(int b = 0; b < 2; ++b)
+				{
+					// upper-half bodies of the segment before p: half of every earlier
+					// segment's bodies are
+					const int before = static_cast<int>(b == 0 ? ex & 0xFFFF : ex >> 16) - (start >> 1);
+					const bool u = ((b == 0 ? up[k] : up[k] >> 16) & 1) != 0;
+					const int pos = u ? start + half + before : p - before;
+					ls[to[b]][pos] = id[b][k];
+					if(b == 0) { then[id[0][k]] = (pos & (half - 1)) >= half >> 1 ? 1 : 0; }
+				}
+			}
+			ex += up[k];
 		}
 		__syncthreads();
-		for(int b = 0; b < 3; ++b)
-		{
-			if(b == a) { continue; }
-			uint32_t c = 0;
-			for(int k = 0; k < per; ++k)
-			{
-				const int p = p0 + k;
-				if(p < seg0)
-				{
-					excl[p] = static_cast<uint16_t>(c);
-					c += side[ls[b][p]];
-				}
-			}
-			uint32_t x = c;
-			for(int off = 1; off < 64; off <<= 1)
-			{
-				const uint32_t u = __shfl_up(x, off, 64);
-				if(lane >= off) { x += u; }
-			}
-			if(lane == 63) { ws[wave] = x; }
-			__syncthreads();
-			uint32_t add = x - c;
-			for(int w = 0; w < wave; ++w) { add += ws[w]; }
-			for(int k = 0; k < per; ++k)
-			{
-				const int p = p0 + k;
-				if(p < seg0) { excl[p] = static_cast<uint16_t>(excl[p] + add); }
-			}
-			__syncthreads();
-			for(int k = 0; k < per; ++k)
-			{
-				const int p = p0 + k;
-				if(p < seg0)
-				{
-					const uint16_t id = ls[b][p];
-					const int seg_start = p & ~(seg - 1);
-					const int before = excl[p] - excl[seg_start];
-					tmp[side[id] ? seg_start + half + before : p - before] = id;
-				}
-			}
-			__syncthreads();
-			for(int k = 0; k < per; ++k)
-			{
-				const int p = p0 + k;
-				if(p < seg0) { ls[b][p] = tmp[p]; }
-			}
-			__syncthreads();
-		}
+		free0 = from[0];
+		free1 = from[1];
+		if(a == 0) { cur1 = to[0]; cur2 = to[1]; }
+		else if(a == 1) { cur2 = to[0]; cur0 = to[1]; }
+		else { cur0 = to[0]; cur1 = to[1]; }
 	}
-	for(int p = threadIdx.x; p < seg0; p += kLocalThreads) { list0[base + p] = l2g[ls[0][p]]; }
+	for(int p = threadIdx.x; p < seg0; p += kLocalThreads) { list0[base + p] = l2g[ls[cur0][p]]; }
 }
 
 // ---------------------------------------------------------------------------
@@ -3883,12 +3896,12 @@ k_pack_records(const double4* __restrict__ xyzr, const double* __restrict__ mass
 	}
 }
 
-nbh_status moments(nbh_ctx* ctx, nbh_tree* t, const double* y, const double* mass, double ratio, bool build)
+nbh_status moments(nbh_ctx* ctx, nbh_tree* t, const double* y, const double* mass, const uint32_t* order, double ratio)
 {
 	t->ratio = ratio;
 	const size_t n = t->n;
-	hipLaunchKernelGGL(k_leaves, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, t->list[0], y, mass,
-	                   n, t->xyzr, t->mass, t->bmin, t->bmax, t->body_n, build ? 1 : 0);
+	hipLaunchKernelGGL(k_leaves, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, order, y, mass,
+	                   n, t->xyzr, t->mass, t->bmin, t->bmax, t->body_n, order != nullptr ? 1 : 0);
 	NBH_LAUNCHED();
 	const double ratio_sqr = ratio * ratio;
 	size_t lo = n / 2;
@@ -3944,7 +3957,7 @@ static void tree_buffers(nbh_tree* t, void** ptrs[kTreeBuffers], size_t sizes[kT
 {
 	const size_t n = t->n;
 	const size_t ncounts = std::max(kSortSets * sort_words((n + kSortTile - 1) / kSortTile),
-	                                (n + kPartTile - 1) / kPartTile) + 1;
+	                                2 * ((n + kPartTile - 1) / kPartTile)) + 1;
 	int k = 0;
 	auto add = [&](void* p, size_t bytes) {
 		ptrs[k] = static_cast<void**>(p);
@@ -4212,43 +4225,45 @@ nbh_status nbh_tree_build(nbh_ctx* ctx, nbh_tree* t, const double* y, const doub
 	const size_t n = t->n;
 	t->radix = false;
 	NBH_TRY(sort_axes(ctx, t, y));
-	const size_t ntiles = (n + kPartTile - 1) / kPartTile;
+	const unsigned ntiles = static_cast<unsigned>((n + kPartTile - 1) / kPartTile);
 	// the last levels (segments of at most kLocalSeg bodies) run in LDS
 	const int local_levels = std::min(t->levels, 12);
-	static_assert(kLocalSeg == 1 << 12, "kLocalSeg is 2^12");
+	static_assert(kLocalSeg == 1 << 12 && kLocalSeg >= kPartTile, "kLocalSeg is 2^12, whole tiles");
 	const int global_levels = t->levels - local_levels;
+	// lists to write and the next level's flags: what the sort no longer needs
+	uint32_t* cur[3] = {t->list[0], t->list[1], t->list[2]};
+	uint32_t* spare[2] = {t->tmp, reinterpret_cast<uint32_t*>(t->keys)};
+	uint8_t*  side[2] = {t->side, reinterpret_cast<uint8_t*>(t->vals)};
+	if(global_levels > 0)
+	{
+		hipLaunchKernelGGL(k_mark_side, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, cur[0], side[0], n,
+		                   n);
+		NBH_LAUNCHED();
+	}
 	for(int level = 0; level < global_levels; ++level)
 	{
 		const size_t seg = n >> level;
-		const int a = level % 3;
-		hipLaunchKernelGGL(k_mark_side, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, t->list[a],
-		                   t->side, n, seg);
+		const int b0 = (level + 1) % 3, b1 = (level + 2) % 3;
+		const part_lists lists = {{cur[b0], cur[b1]}, {spare[0], spare[1]}};
+		hipLaunchKernelGGL(k_part_count, dim3(ntiles, 2), dim3(kPartThreads), 0, ctx->stream, lists, side[level & 1],
+		                   t->counts);
 		NBH_LAUNCHED();
-		for(int b = 0; b < 3; ++b)
-		{
-			if(b == a) { continue; }
-			if(seg >= static_cast<size_t>(kPartTile))
-			{
-				hipLaunchKernelGGL(k_part_count, dim3(static_cast<unsigned>(ntiles)), dim3(kPartThreads), 0,
-				                   ctx->stream, t->list[b], t->side, n, t->counts);
-				NBH_LAUNCHED();
-				NBH_TRY(scan_exclusive(ctx, t->counts, ntiles, t->scan_part));
-			}
-			hipLaunchKernelGGL(k_part_scatter, dim3(static_cast<unsigned>(ntiles)), dim3(kPartThreads), 0,
-			                   ctx->stream, t->list[b], t->side, n, seg, t->counts, t->tmp);
-			NBH_LAUNCHED();
-			std::swap(t->list[b], t->tmp);
-		}
+		const int scanned = seg / kPartTile > kPartSum ? 1 : 0;
+		if(scanned != 0) { NBH_TRY(scan_exclusive(ctx, t->counts, 2 * static_cast<size_t>(ntiles), t->scan_part)); }
+		hipLaunchKernelGGL(k_part_scatter, dim3(ntiles, 2), dim3(kPartThreads), 0, ctx->stream, lists, side[level & 1],
+		                   seg, t->counts, scanned, level + 1 < global_levels ? 0 : -1, side[~level & 1]);
+		NBH_LAUNCHED();
+		std::swap(cur[b0], spare[0]);
+		std::swap(cur[b1], spare[1]);
 	}
 	if(local_levels > 0)
 	{
 		const size_t seg0 = n >> global_levels;
 		hipLaunchKernelGGL(k_split_local, dim3(static_cast<unsigned>(n / seg0)), dim3(kLocalThreads), 0, ctx->stream,
-		                   t->list[0], t->list[1], t->list[2], t->tmp, static_cast<int>(seg0), global_levels,
-		                   t->levels);
+		                   cur[0], cur[1], cur[2], spare[0], static_cast<int>(seg0), global_levels, t->levels);
 		NBH_LAUNCHED();
 	}
-	NBH_TRY(moments(ctx, t, y, mass, ratio, true));
+	NBH_TRY(moments(ctx, t, y, mass, cur[0], ratio));
 	t->built = true;
 	return NBH_OK;
 }
@@ -4274,7 +4289,7 @@ nbh_status nbh_tree_refit(nbh_ctx* ctx, nbh_tree* t, const double* y, double rat
 		NBH_TRY(radix_groups(ctx, t, y, nullptr, false, static_cast<size_t>(t->ngroups)));
 		return radix_tiers(ctx, t);
 	}
-	return moments(ctx, t, y, nullptr, ratio, false);
+	return moments(ctx, t, y, nullptr, nullptr, ratio);
 }
 
 nbh_status nbh_bh_fcompute(nbh_ctx* ctx, const nbh_tree* t, const double* y, const double* mass, double* f,

@@ -88,6 +88,31 @@ def test_build_bit_exact(ctx, kind, n):
     t.close()
 
 
+@pytest.mark.parametrize("ties", [False, True])
+@pytest.mark.parametrize("n", [4, 8, 2048, 8192, 16384, 1 << 23])
+def test_build_split_edges(ctx, n, ties):
+    """Segments split in LDS alone, one and two levels above it, and segments of more
+    tiles than a tile sums itself (2^23): every level's segments hold their lower half
+    first along its axis, equal coordinates by body index, and each body once."""
+    rng = np.random.default_rng(n)
+    pos = rng.integers(0, 50, size=(3, n)).astype(np.float64) if ties else rng.random((3, n))
+    y = np.concatenate([pos.reshape(-1), np.zeros(3 * n)])
+    t = GpuTree(ctx, n)
+    dy, dm = ctx.put(y), ctx.put(np.ones(n))
+    t.build(dy, dm, 2.0)
+    body = np.empty(2 * n, np.int32)
+    native.check(ctx.lib.nbh_tree_get(ctx.h, t.h, body.ctypes.data_as(C.c_void_p), None, None, None, None, None))
+    order = body[n:].astype(np.int64)
+    assert np.array_equal(np.sort(order), np.arange(n))
+    for level in range(n.bit_length() - 1 if n < 1 << 20 else 13):
+        x = pos[level % 3, order]
+        if ties:
+            x = x * n + order          # whole numbers: coordinate, then body
+        x = x.reshape(1 << level, 2, -1)
+        assert np.all(x[:, 0].max(1) < x[:, 1].min(1)), level
+    t.close()
+
+
 def test_build_ties_follow_index_order(ctx):
     """Equal coordinates: both sides break ties by body index."""
     n = 256
