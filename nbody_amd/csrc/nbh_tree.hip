@@ -796,28 +796,6 @@ k_split_local(uint32_t* __restrict__ list0, const uint32_t* __restrict__ list1, 
 // ---------------------------------------------------------------------------
 // moments (nbody/nbody_space_heap.cpp:119-134), FP64, contraction off
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-k_leaves(const uint32_t* __restrict__ order, const double* __restrict__ y, const double* __restrict__ mass,
-         size_t n, double4* __restrict__ xyzr, double* __restrict__ nmass, double* __restrict__ bmin,
-         double* __restrict__ bmax, int32_t* __restrict__ body_n, int set_body)
-{
-	size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t s = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; s < n; s += stride)
-	{
-		size_t idx = n + s;
-		uint32_t b = set_body ? order[s] : static_cast<uint32_t>(body_n[idx]);
-		double x = y[b], yy = y[n + b], z = y[2 * n + b];
-		xyzr[idx] = make_double4(x, yy, z, 0.0);
-		if(set_body)
-		{
-			body_n[idx] = static_cast<int32_t>(b);
-			nmass[idx] = mass[b];
-		}
-		bmin[3 * idx] = x; bmin[3 * idx + 1] = yy; bmin[3 * idx + 2] = z;
-		bmax[3 * idx] = x; bmax[3 * idx + 1] = yy; bmax[3 * idx + 2] = z;
-	}
-}
-
 __device__ inline double min_ref(double a, double b) { return (b < a) ? b : a; }   // std::min
 __device__ inline double max_ref(double a, double b) { return (a < b) ? b : a; }   // std::max
 
@@ -875,11 +853,9 @@ __device__ inline void combine_quad(const double4& c, const double4& cl, double 
 	}
 }
 
-// Node idx from its children l and r (2 idx and 2 idx + 1 in the heap), each
-// child read once; kRecord: its walk record too (as k_pack_records).
-template <bool kRecord>
+// Node idx with its walk record from its children l and r, each read once.
 __device__ inline void join_nodes(size_t idx, size_t l, size_t r, double4* xyzr, double* nmass, double* bmin,
-                                  double* bmax, double* quad, double ratio_sqr, nbh_walk_rec* wr = nullptr)
+                                  double* bmax, double* quad, double ratio_sqr, nbh_walk_rec* wr)
 {
 	const double4 cl = xyzr[l], cr = xyzr[r];
 	const double ml = nmass[l], mr = nmass[r];
@@ -908,38 +884,8 @@ __device__ inline void join_nodes(size_t idx, size_t l, size_t r, double4* xyzr,
 		bmax[3 * idx + d] = hi[d];
 	}
 	for(int k = 0; k < 6; ++k) { quad[6 * idx + k] = q[k]; }
-	if constexpr(kRecord)
-	{
-		for(int k = 0; k < 6; ++k) { rec.q[k] = static_cast<float>(q[k]); }
-		wr[idx] = rec;
-	}
-}
-
-// nodes [lo, hi) of one level
-__global__ void __launch_bounds__(256)
-k_level(size_t lo, size_t hi, double4* __restrict__ xyzr, double* __restrict__ nmass, double* __restrict__ bmin,
-        double* __restrict__ bmax, double* __restrict__ quad, double ratio_sqr)
-{
-	size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t idx = lo + static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; idx < hi; idx += stride)
-	{
-		join_nodes<false>(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, bmin, bmax, quad, ratio_sqr);
-	}
-}
-
-// all levels with fewer than 2 * 256 nodes in one work-group, bottom-up
-__global__ void __launch_bounds__(256)
-k_levels_top(size_t top, double4* __restrict__ xyzr, double* __restrict__ nmass, double* __restrict__ bmin,
-             double* __restrict__ bmax, double* __restrict__ quad, double ratio_sqr)
-{
-	for(size_t lo = top; lo >= 1; lo >>= 1)
-	{
-		for(size_t idx = lo + threadIdx.x; idx < 2 * lo; idx += blockDim.x)
-		{
-			join_nodes<false>(idx, 2 * idx, 2 * idx + 1, xyzr, nmass, bmin, bmax, quad, ratio_sqr);
-		}
-		__syncthreads();
-	}
+	for(int k = 0; k < 6; ++k) { rec.q[k] = static_cast<float>(q[k]); }
+	wr[idx] = rec;
 }
 
 // ---------------------------------------------------------------------------
@@ -1374,7 +1320,7 @@ __device__ inline void join_part(const double (&cc)[2], const double (&mm)[2], c
 
 // Leaves and internal nodes of each build group (a subtree of at most
 // kRadixGroup leaves), one wave per group, with their walk records.  The
-// group's leaves (as k_leaves; kBuild: the body at sorted position s is
+// group's leaves (kBuild: the body at sorted position s is
 // order[s], read from its packed record; refit: the body numbers of the build,
 // positions from y and the masses of the leaf records) and node moments are held
 // in LDS: leaf first + j in slot j, internal id k in slot k - first - 1 (the
@@ -1688,7 +1634,7 @@ k_radix_tier(const int* __restrict__ roots, int t, int n, const int2* __restrict
 		if(i < start[d + 1])
 		{
 			const int2 c = child[q[i]];
-			join_nodes<true>(q[i], c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr);
+			join_nodes(q[i], c.x, c.y, xyzr, nmass, bmin, bmax, quad, ratio_sqr, wr);
 		}
 		__syncthreads();
 	}
@@ -1743,6 +1689,144 @@ k_radix_tier(const int* __restrict__ roots, int t, int n, const int2* __restrict
 			bmax[3 * id + e] = p[kHi + e];
 		}
 		for(int e = 0; e < 6; ++e) { quad[6 * id + e] = p[kQ + e]; }
+	}
+}
+
+// Moments and walk records of the heap's nodes above the `width` (a power of two, at
+// most kHeapBase) ids from lo + blockIdx.x * width, a subtree whose root the work-group
+// ends with.  kLeaf: the ids are leaves, set here too: the body at sorted position s is
+// order[s], or with no order (refit) the leaf's body and mass of the last build.  The
+// subtree is held in LDS, four lanes a node (join_part), and the nodes go out at the
+// end, when their opening radii are known.  Bound by memory: with a launch for the
+// leaves, one for each level and one for the records, which read all of it again,
+// 100 us at 2^18 bodies and 285 at 2^20, now 55 and 153.
+constexpr int kHeapBase = 256;
+
+template <bool kLeaf>
+__global__ void __launch_bounds__(kHeapBase)
+k_heap_moments(size_t lo, int width, size_t n, const uint32_t* __restrict__ order, const double* __restrict__ y,
+               const double* __restrict__ mass, double4* __restrict__ xyzr, double* __restrict__ nmass,
+               double* __restrict__ bmin, double* __restrict__ bmax, double* __restrict__ quad,
+               int32_t* __restrict__ body_n, double ratio_sqr, nbh_walk_rec* __restrict__ wr)
+{
+	// local ids as in a heap: root 1, the given nodes [width, 2 width).  Per node mass
+	// centre, mass, box, second moments; leaves: position and mass
+	constexpr int kC = 0, kM = 3, kLo = 4, kHi = 7, kQ = 10, kPer = 17, kLeafPer = 4;
+	__shared__ double sh[kHeapBase * kPer];
+	__shared__ double base[kHeapBase * (kLeaf ? kLeafPer : kPer)];
+	const int tid = threadIdx.x;
+	const int part = tid & 3, dim = part < 3 ? part : 2;
+	const size_t first = lo + static_cast<size_t>(blockIdx.x) * width;
+	if constexpr(kLeaf)
+	{
+		if(tid < width)
+		{
+			const size_t idx = first + tid;
+			const uint32_t b = order != nullptr ? order[idx - n] : static_cast<uint32_t>(body_n[idx]);
+			nbh_walk_rec r;
+			r.c = make_double4(y[b], y[n + b], y[2 * n + b], 0.0);
+			r.m = order != nullptr ? mass[b] : nmass[idx];
+			for(int k = 0; k < 6; ++k) { r.q[k] = 0.0f; }
+			if(order != nullptr)
+			{
+				body_n[idx] = static_cast<int32_t>(b);
+				nmass[idx] = r.m;
+			}
+			xyzr[idx] = r.c;
+			bmin[3 * idx] = r.c.x; bmin[3 * idx + 1] = r.c.y; bmin[3 * idx + 2] = r.c.z;
+			bmax[3 * idx] = r.c.x; bmax[3 * idx + 1] = r.c.y; bmax[3 * idx + 2] = r.c.z;
+			wr[idx] = r;
+			double* p = base + kLeafPer * tid;
+			p[0] = r.c.x;
+			p[1] = r.c.y;
+			p[2] = r.c.z;
+			p[3] = r.m;
+		}
+	}
+	else
+	{
+		for(int i = tid >> 2; i < width; i += kHeapBase / 4)
+		{
+			const size_t idx = first + i;
+			double* p = base + kPer * i;
+			if(part < 3)
+			{
+				p[kC + part] = reinterpret_cast<const double*>(xyzr)[4 * idx + part];
+				p[kLo + part] = bmin[3 * idx + part];
+				p[kHi + part] = bmax[3 * idx + part];
+				p[kQ + part] = quad[6 * idx + part];
+				p[kQ + 3 + part] = quad[6 * idx + 3 + part];
+			}
+			else
+			{
+				p[kM] = nmass[idx];
+			}
+		}
+	}
+	__syncthreads();
+	for(int w = width >> 1; w >= 1; w >>= 1)
+	{
+		for(int i = w + (tid >> 2); i < 2 * w; i += kHeapBase / 4)
+		{
+			double cc[2], mm[2], lo2[2], hi2[2], qd[2], qo[2];
+			for(int side = 0; side < 2; ++side)
+			{
+				const int ch = 2 * i + side;
+				if(kLeaf && ch >= width)
+				{
+					const double* p = base + kLeafPer * (ch - width);
+					cc[side] = lo2[side] = hi2[side] = p[dim];
+					mm[side] = p[3];
+					qd[side] = qo[side] = 0.0;
+				}
+				else
+				{
+					const double* p = ch >= width ? base + kPer * (ch - width) : sh + kPer * ch;
+					cc[side] = p[kC + dim];
+					mm[side] = p[kM];
+					lo2[side] = p[kLo + dim];
+					hi2[side] = p[kHi + dim];
+					qd[side] = p[kQ + dim];
+					qo[side] = p[kQ + 3 + dim];
+				}
+			}
+			double c, m, l, h, qdd, qoo;
+			join_part(cc, mm, lo2, hi2, qd, qo, c, m, l, h, qdd, qoo);
+			double* p = sh + kPer * i;
+			if(part < 3)
+			{
+				p[kC + part] = c;
+				p[kLo + part] = l;
+				p[kHi + part] = h;
+				p[kQ + part] = qdd;
+				p[kQ + 3 + part] = qoo;
+			}
+			else
+			{
+				p[kM] = m;
+			}
+		}
+		__syncthreads();
+	}
+	if(tid >= 1 && tid < width)
+	{
+		const int d = 31 - __clz(tid);
+		const size_t idx = ((first / width) << d) + (tid - (1 << d));
+		const double* p = sh + kPer * tid;
+		nbh_walk_rec rec;
+		rec.c = make_double4(p[kC], p[kC + 1], p[kC + 2],
+		                     crit_radius(p[kC], p[kC + 1], p[kC + 2], p + kLo, p + kHi, ratio_sqr));
+		rec.m = p[kM];
+		for(int e = 0; e < 6; ++e) { rec.q[e] = static_cast<float>(p[kQ + e]); }
+		wr[idx] = rec;
+		xyzr[idx] = rec.c;
+		nmass[idx] = rec.m;
+		for(int e = 0; e < 3; ++e)
+		{
+			bmin[3 * idx + e] = p[kLo + e];
+			bmax[3 * idx + e] = p[kHi + e];
+		}
+		for(int e = 0; e < 6; ++e) { quad[6 * idx + e] = p[kQ + e]; }
 	}
 }
 
@@ -3880,46 +3964,21 @@ nbh_status sort_axes(nbh_ctx* ctx, nbh_tree* t, const double* y)
 	return sort_run(ctx, a, 3, n, 8, false, t->counts);
 }
 
-// Packed walk records of nodes 1 .. count-1.
-__global__ void __launch_bounds__(256)
-k_pack_records(const double4* __restrict__ xyzr, const double* __restrict__ mass, const double* __restrict__ quad,
-               nbh_walk_rec* __restrict__ wr, size_t count)
-{
-	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t i = 1 + static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += stride)
-	{
-		nbh_walk_rec r;
-		r.c = xyzr[i];
-		r.m = mass[i];
-		for(int k = 0; k < 6; ++k) { r.q[k] = static_cast<float>(quad[6 * i + k]); }
-		wr[i] = r;
-	}
-}
-
 nbh_status moments(nbh_ctx* ctx, nbh_tree* t, const double* y, const double* mass, const uint32_t* order, double ratio)
 {
 	t->ratio = ratio;
 	const size_t n = t->n;
-	hipLaunchKernelGGL(k_leaves, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, order, y, mass,
-	                   n, t->xyzr, t->mass, t->bmin, t->bmax, t->body_n, order != nullptr ? 1 : 0);
-	NBH_LAUNCHED();
-	const double ratio_sqr = ratio * ratio;
-	size_t lo = n / 2;
-	for(; lo >= 512; lo >>= 1)
+	size_t lo = n;
+	do
 	{
-		hipLaunchKernelGGL(k_level, dim3(nbh::grid_for(ctx, lo, 256)), dim3(256), 0, ctx->stream, lo, 2 * lo,
-		                   t->xyzr, t->mass, t->bmin, t->bmax, t->quad, ratio_sqr);
+		const size_t width = std::min<size_t>(lo, kHeapBase);
+		const auto kernel = lo == n ? k_heap_moments<true> : k_heap_moments<false>;
+		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(lo / width)), dim3(kHeapBase), 0, ctx->stream, lo,
+		                   static_cast<int>(width), n, order, y, mass, t->xyzr, t->mass, t->bmin, t->bmax, t->quad,
+		                   t->body_n, ratio * ratio, t->wrec);
 		NBH_LAUNCHED();
-	}
-	if(lo >= 1)
-	{
-		hipLaunchKernelGGL(k_levels_top, dim3(1), dim3(256), 0, ctx->stream, lo, t->xyzr, t->mass, t->bmin, t->bmax,
-		                   t->quad, ratio_sqr);
-		NBH_LAUNCHED();
-	}
-	hipLaunchKernelGGL(k_pack_records, dim3(nbh::grid_for(ctx, 2 * n, 256)), dim3(256), 0, ctx->stream, t->xyzr,
-	                   t->mass, t->quad, t->wrec, 2 * n);
-	NBH_LAUNCHED();
+		lo /= width;
+	} while(lo > 1);
 	return NBH_OK;
 }
 
