@@ -13,13 +13,15 @@
 //      bodies of one node; along axis a = l % 3 the first S/2 entries of the
 //      a-sorted list are exactly the count/2 smallest, i.e. std::nth_element's
 //      left part.  Each body is tagged left/right, and the two other lists are
-//      stably partitioned inside every segment (segmented scan + scatter), so
+//      stably partitioned inside every segment (counts of the tiles before + scatter), so
 //      every child segment again holds its bodies sorted along all three axes;
 //   3. after L levels entry s of any list is the body of leaf n + s;
 //   4. moments bottom-up with the operations of nbody_space_heap::update
 //      (:119-134), in FP64 with contraction off: bit-identical node records.
-// Traversal: one target per work-item, targets in heap-leaf order (spatially
-// coherent), nodes as 32-byte AoS records {cm.xyz, crit_r2} plus mass.
+// Traversal: a wave walks for consecutive leaves of the heap (spatially coherent):
+// 32 in the FP64 parity walk (k_bh_walk64), 64 in the FP32 group walks, up to 128 on the
+// Morton tree; nodes as 32-byte records {cm.xyz, crit_r2} plus mass, or packed with the
+// second moments in 64 bytes.
 #include <algorithm>
 #include <climits>
 #include <cmath>

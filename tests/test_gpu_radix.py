@@ -129,10 +129,11 @@ def _cusps(n, seed):
 
 
 @pytest.mark.parametrize("kind,n", [("plummer", 65), ("plummer", 129), ("plummer", 2049), ("plummer", 70001),
-                                    ("cusps", 1200), ("cusps", 2048), ("cusps", 30011)])
+                                    ("plummer", 150001), ("cusps", 1200), ("cusps", 2048), ("cusps", 30011)])
 def test_radix_tier_edges(ctx, kind, n):
     """Trees whose root is the smallest above a build group, a walk group and a
-    2048-leaf subtree, and of several tiers; build and refit bit for bit, and every
+    2048-leaf subtree, of several tiers, and of over 1024 walk groups (taken in runs per
+    XCD, with a remainder); build and refit bit for bit, and every
     body in one walk group, under the super-group that holds it (a lost or doubled
     body, or a wrong list, shows in the accelerations against the direct sum)."""
     y, m = _cusps(n, n) if kind == "cusps" else _state(kind, n, n)
@@ -147,7 +148,9 @@ def test_radix_tier_edges(ctx, kind, n):
             assert np.array_equal(g[k][1:2 * n], o[k][1:2 * n]), (step, k)
     idx = np.arange(0, n, max(1, n // 1000))
     a0 = _direct(y, m, idx)
-    e2, e1 = _rms(t.walk("local2"), a0, n, idx), _rms(t.walk("local"), a0, n, idx)
+    f2 = t.walk("local2")
+    assert np.array_equal(f2[:3 * n], y[3 * n:])
+    e2, e1 = _rms(f2, a0, n, idx), _rms(t.walk("local"), a0, n, idx)
     assert e2[0] < 2e-2 and e2[0] < 1.25 * e1[0] + 1e-6, (e2, e1)
     t.close()
 
