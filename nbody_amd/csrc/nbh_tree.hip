@@ -4075,6 +4075,9 @@ nbh_status nbh_tree_create(nbh_ctx* ctx, size_t n, nbh_tree** out)
 	}
 	if(e == hipSuccess) { e = hipMemsetAsync(t->xyzr, 0, 2 * n * sizeof(double4), ctx->stream); }
 	if(e == hipSuccess) { e = hipMemsetAsync(t->mass, 0, 2 * n * sizeof(double), ctx->stream); }
+	// box 0, which no node has and nbh_tree_get returns with the others
+	if(e == hipSuccess) { e = hipMemsetAsync(t->bmin, 0, 3 * sizeof(double), ctx->stream); }
+	if(e == hipSuccess) { e = hipMemsetAsync(t->bmax, 0, 3 * sizeof(double), ctx->stream); }
 	if(e == hipSuccess) { e = hipMemsetAsync(t->quad, 0, 2 * n * 6 * sizeof(double), ctx->stream); }
 	if(e == hipSuccess) { e = hipMemsetAsync(t->wrec, 0, 2 * n * sizeof(nbh_walk_rec), ctx->stream); }
 	if(e == hipSuccess) { e = hipMemsetAsync(t->body_n, 0xff, 2 * n * sizeof(int32_t), ctx->stream); }

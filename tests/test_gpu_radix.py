@@ -146,6 +146,7 @@ def test_radix_tier_edges(ctx, kind, n):
         g = t.arrays()
         for k in ("cm", "mass", "crit", "bmin", "bmax"):
             assert np.array_equal(g[k][1:2 * n], o[k][1:2 * n]), (step, k)
+        assert not g["bmin"][0].any() and not g["bmax"][0].any()      # no node: zeros, whatever the memory held
     idx = np.arange(0, n, max(1, n // 1000))
     a0 = _direct(y, m, idx)
     f2 = t.walk("local2")
