@@ -73,7 +73,8 @@ const nbh_ctx* mlp_ctx(const nbh_mlp* m);
 // Stable LSD radix sort of (key, value) pairs on the low `bits` bits of the
 // keys, 8 bits per pass, ping-ponging between (k0, v0) and (k1, v1); *sorted_vals
 // points at the buffer holding the result (the keys end in the same half).
-// counts: sort_counts_size(n) words of device scratch, 8-byte aligned.
+// counts: sort_counts_size(n) words of device scratch, 8-byte aligned, that the caller's
+// kernels have set to zero.
 size_t sort_counts_size(size_t n);
 nbh_status sort_pairs(nbh_ctx* ctx, uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n, int bits,
                       uint32_t* counts, uint32_t** sorted_vals);

@@ -1013,10 +1013,11 @@ __device__ inline uint32_t spread10(uint32_t x)
 }
 
 // 30-bit Morton keys of the positions on a 1024^3 grid over the box (values:
-// body indices).  Non-finite coordinates map to cell 0.
+// body indices).  Non-finite coordinates map to cell 0.  The sort's counts are cleared
+// on the way (a launch of its own takes 4.5 us).
 __global__ void __launch_bounds__(256)
 k_morton_keys(const double* __restrict__ y, size_t n, const double* __restrict__ box, uint64_t* __restrict__ keys,
-              uint32_t* __restrict__ vals)
+              uint32_t* __restrict__ vals, uint32_t* __restrict__ counts, size_t words)
 {
 	double lo[3], sc[3];
 	for(int d = 0; d < 3; ++d)
@@ -1037,6 +1038,7 @@ k_morton_keys(const double* __restrict__ y, size_t n, const double* __restrict__
 		keys[i] = spread10(q[0]) | (spread10(q[1]) << 1) | (spread10(q[2]) << 2);
 		vals[i] = static_cast<uint32_t>(i);
 	}
+	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < words; i += stride) { counts[i] = 0; }
 }
 
 // Launch shape and scratch layout of the FP32 path for n bodies: bodies per lane,
@@ -1117,7 +1119,8 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	NBH_LAUNCHED();
 	hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, ctx->stream, bpart, static_cast<int>(l.gbox), box);
 	NBH_LAUNCHED();
-	hipLaunchKernelGGL(k_morton_keys, dim3(l.gbox), dim3(256), 0, ctx->stream, y, n, box, keys, vals);
+	hipLaunchKernelGGL(k_morton_keys, dim3(l.gbox), dim3(256), 0, ctx->stream, y, n, box, keys, vals, counts,
+	                   nbh::sort_counts_size(n));
 	NBH_LAUNCHED();
 	uint32_t* perm = nullptr;
 	NBH_TRY(nbh::sort_pairs(ctx, keys, vals, keys + n, vals + n, n, 30, counts, &perm));

@@ -188,13 +188,6 @@ k_make_keys(const double* __restrict__ y, sort_lists a, size_t n, uint32_t* __re
 	for(size_t i = first; i < words; i += stride) { scratch[blockIdx.y * words + i] = 0; }
 }
 
-__global__ void __launch_bounds__(256)
-k_sort_clear(uint32_t* __restrict__ scratch, size_t words)
-{
-	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < words; i += stride) { scratch[i] = 0; }
-}
-
 // Counts of the digits of all passes, once over the keys (their multiset does not
 // change from pass to pass).
 __global__ void __launch_bounds__(kSortThreads)
@@ -931,7 +924,8 @@ __device__ inline uint64_t morton_cell(double x, double lo, double scale)
 __global__ void __launch_bounds__(256)
 k_morton_codes(const double* __restrict__ y, const double* __restrict__ mass, size_t n, const double* __restrict__ box,
                uint64_t* __restrict__ keys, uint32_t* __restrict__ vals, double4* __restrict__ pk,
-               uint32_t* __restrict__ marks, size_t words, int* __restrict__ parent)
+               uint32_t* __restrict__ marks, size_t words, int* __restrict__ parent, uint32_t* __restrict__ counts,
+               size_t count_words)
 {
 	const double side = fmax(fmax(box[3] - box[0], box[4] - box[1]), box[5] - box[2]);
 	const double scale = side > 0.0 ? 2097152.0 / side : 0.0;
@@ -946,7 +940,9 @@ k_morton_codes(const double* __restrict__ y, const double* __restrict__ mass, si
 		vals[i] = static_cast<uint32_t>(i);
 		pk[i] = make_double4(x, yy, z, mass[i]);
 	}
-	// what the tree's kernels count and mark in, and the parents that no node has
+	// what the sort and the tree's kernels count and mark in, and the parents that no
+	// node has
+	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < count_words; i += stride) { counts[i] = 0; }
 	for(size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < words; i += stride) { marks[i] = 0; }
 	if(blockIdx.x == 0 && threadIdx.x < 2) { parent[threadIdx.x] = 0; }
 }
@@ -3997,12 +3993,6 @@ nbh_status sort_pairs(nbh_ctx* ctx, uint64_t* k0, uint32_t* v0, uint64_t* k1, ui
 	uint32_t* out = passes % 2 == 0 ? v0 : v1;
 	sort_lists a = {};
 	a.l[0] = {{k0, k1}, {v0, v1}, out};
-	const size_t words = sort_counts_size(n);
-	if(n > static_cast<size_t>(kSortTile))
-	{
-		hipLaunchKernelGGL(k_sort_clear, dim3(grid_for(ctx, words, 256)), dim3(256), 0, ctx->stream, counts, words);
-		NBH_LAUNCHED();
-	}
 	NBH_TRY(sort_run(ctx, a, 1, n, passes, true, counts));
 	*sorted_vals = out;
 	return NBH_OK;
@@ -4186,7 +4176,8 @@ nbh_status nbh_tree_build_radix(nbh_ctx* ctx, nbh_tree* t, const double* y, cons
 	hipLaunchKernelGGL(k_box_final, dim3(1), dim3(256), 0, ctx->stream, t->box + 6, static_cast<int>(parts), t->box);
 	NBH_LAUNCHED();
 	hipLaunchKernelGGL(k_morton_codes, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, y, mass, n,
-	                   t->box, t->keys, t->vals, t->pk, t->marks, mark_words(n), t->parent);
+	                   t->box, t->keys, t->vals, t->pk, t->marks, mark_words(n), t->parent, t->counts,
+	                   nbh::sort_counts_size(n));
 	NBH_LAUNCHED();
 	uint32_t* order = nullptr;
 	// 63-bit keys: 8 passes, so the sorted keys end where they started
