@@ -390,8 +390,9 @@ k_scan_one(uint32_t* __restrict__ c, int m)
 // so every wait ends.  A pass's words carry its number: those of the passes before
 // read as not there yet.  Latency bound below some 2^19 keys: with a histogram, a
 // scan and a scatter with a work-group barrier per row of keys for every pass, list
-// by list, the heap build of 2^17 bodies took 1065 us (24 passes of 31 us), now 366
-// us, and the Morton build of 2^22 bodies 1.96 ms, now 1.70.
+// by list, the heap build of 2^17 bodies took 1065 us (24 passes of 31 us), with this
+// pass 366, and the Morton build of 2^22 bodies 1.96 ms, with this pass 1.70 (213 us
+// and 1.15 ms with the rest of the builds as they are now).
 __global__ void __launch_bounds__(kSortThreads)
 k_sort_pass(sort_lists a, size_t n, int pass, int last, int keep_keys, uint32_t* __restrict__ scratch, size_t tiles)
 {
