@@ -11,7 +11,7 @@
 // and copied once into records (x, y, z, m) in that order; blocks of consecutive
 // bodies meet pairwise, and every pair is evaluated once for both its bodies.
 // Coordinates are FP32 offsets from the FP64 position of a body close to one of the
-// two.  Per pair: 3 sub, 3 mul/fma for r^2, 1 v_rsq_f32 whose output clamp is the
+// two, the one in the denser place.  Per pair: 3 sub, 3 mul/fma for r^2, 1 v_rsq_f32 whose output clamp is the
 // reference's r^2 >= 1e-8 clamp (in scaled units), 4 mul and 6 fma.  Partial sums
 // stay in FP32 over 64 terms; a second kernel adds the blocks' sums in FP64 in a
 // fixed order and copies the velocities into f[0:3n].
@@ -600,7 +600,8 @@ k_direct_sample64(const double* __restrict__ y, const double* __restrict__ mass,
 // ---------------------------------------------------------------------------
 // FP32 tiles
 // ---------------------------------------------------------------------------
-constexpr int kF32Group = 1024;    // bodies that share an origin
+constexpr int kF32Group = 1024;    // bodies that share an origin in the pairs inside a block
+constexpr int kF32Near = 256;      // and in the pairs of two blocks
 
 // The tiles work in scaled units: offsets x' = 1e4 x and masses m' = 1e8 m (both
 // formed in FP64 and rounded once).  Then r'^2 = 1e8 r^2, and the reference's
@@ -620,17 +621,39 @@ __device__ inline float rsq_clamped(float r2)
 // The state in Morton order as one record per body: sorted[p] = (x, y, z, m) of
 // body perm[p].  Written once per force evaluation, so that the tile kernel
 // reads its targets and sources as contiguous 32-byte records instead of
-// gathering three coordinates through the permutation.
-__global__ void __launch_bounds__(256)
+// gathering three coordinates through the permutation.  spread: of each kF32Near
+// bodies (a work-group's), the mean log2 of the distances, by the largest coordinate,
+// from the first of them.
+__global__ void __launch_bounds__(kF32Near)
 k_sorted_copy(const double* __restrict__ y, const double* __restrict__ mass, const uint32_t* __restrict__ perm,
-              double4* __restrict__ sorted, size_t n)
+              double4* __restrict__ sorted, float* __restrict__ spread, size_t n)
 {
-	const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-	for(size_t p = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < n; p += stride)
+	__shared__ float part[kF32Near / 64];
+	const size_t first = static_cast<size_t>(blockIdx.x) * kF32Near;
+	const size_t p = first + threadIdx.x;
+	const size_t b0 = perm[first], b = perm[p < n ? p : first];
+	const double4 s = make_double4(y[b], y[n + b], y[2 * n + b], mass[b]);
+	if(p < n) { sorted[p] = s; }
+	const double d = fmax(fmax(fabs(s.x - y[b0]), fabs(s.y - y[n + b0])), fabs(s.z - y[2 * n + b0]));
+	float v = p < n ? __log2f(static_cast<float>(fmin(fmax(d, 1e-30), 1e30))) : 0.0f;
+	for(int off = 32; off > 0; off >>= 1) { v += __shfl_xor(v, off, 64); }
+	if((threadIdx.x & 63) == 0) { part[threadIdx.x >> 6] = v; }
+	__syncthreads();
+	if(threadIdx.x == 0)
 	{
-		const size_t b = perm[p];
-		sorted[p] = make_double4(y[b], y[n + b], y[2 * n + b], mass[b]);
+		for(int w = 1; w < kF32Near / 64; ++w) { v += part[w]; }
+		spread[blockIdx.x] = v / static_cast<float>(n - first < static_cast<size_t>(kF32Near) ? n - first : kF32Near);
 	}
+}
+
+// The one of two origins that its bodies are closer to.
+__device__ inline int nearer(const float* __restrict__ spread, int a, int b) { return spread[b] < spread[a] ? b : a; }
+
+// The origin of a wave's run of `len` bodies from `first` on in the pairs of two blocks.
+__device__ inline int run_origin(const float* __restrict__ spread, size_t first, int len, size_t n)
+{
+	const int g = static_cast<int>(first / kF32Near);
+	return len > kF32Near && first + kF32Near < n ? nearer(spread, g, g + 1) : g;
 }
 
 // A pair's offset, r^2 and v_rsq_f32 serve both bodies.  The bodies, in Morton
@@ -642,11 +665,16 @@ k_sorted_copy(const double* __restrict__ y, const double* __restrict__ mass, con
 // that body receives move with it from lane to lane (one DPP rotation per step and
 // component, folded into the addition).
 //
-// Offsets are taken from the first body of the 1024 that a lane's bodies belong
-// to: FP64 difference, scaled, rounded once.  Those 1024 are consecutive along the
-// curve, so they are close together and their offsets -- and those of the bodies
-// near them -- are small in FP32.  Sums are FP32 over 64 terms (for J over 64 sums
-// of kT), then FP64.
+// Offsets are FP64 differences from an origin, scaled and rounded once; the origin is a
+// body, so that a pair's offsets lose no more than the bits by which its two bodies lie
+// farther from that body than from each other.  Inside a block it is the first body of
+// the target's own 1024.  A pair of two blocks has one for both its bodies: the first of
+// the 256 consecutive bodies that one or the other belongs to, of the 256 that lie closer
+// to theirs (nearer).  With I's for both, a compact clump whose block is J was rounded at
+// the scale of whatever I held: bodies of a clump of 1e-3 in a ball of 10 had a median
+// error of 7.6e-5 (8192 bodies), now 5e-8, and 8e-8 with every target's own 1024.  An
+// origin costs kT record reads per 256 bodies of J, 0.4% at 2^18 bodies.  Sums are FP32
+// over 64 terms (for J over 64 sums of kT), then FP64.
 //
 // VALU issue bound: 16 instructions and one v_rsq_f32 for both bodies of a pair, at
 // the 2.4 to 2.9 clocks that e32 encodings take and 8 for the v_rsq_f32; one target
@@ -725,35 +753,43 @@ __device__ inline void sym_block(const float4* js, int lane, const float (&x)[kT
 // bodies of block J receive from block J - d (rows d >= 1 only).
 template <int kT>
 __global__ void __launch_bounds__(kSymThreads)
-k_direct_fp32_sym(const double4* __restrict__ sorted, const double* __restrict__ box, double* __restrict__ own,
-                  float* __restrict__ other, size_t n, int nb, int d0, int d1, int per)
+k_direct_fp32_sym(const double4* __restrict__ sorted, const double* __restrict__ box, const float* __restrict__ spread,
+                  double* __restrict__ own, float* __restrict__ other, size_t n, int nb, int d0, int d1, int per)
 {
 	constexpr int kB = kSymThreads * kT;
 	constexpr int kSub = kB / 64;
 	__shared__ float4 js[kSymWaves][128];
 	__shared__ float react[3][kB];
 	const int lane = threadIdx.x & 63;
-	const int wave = threadIdx.x >> 6;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int bi = blockIdx.x;
 	const size_t i0 = static_cast<size_t>(bi) * kB + static_cast<size_t>(wave) * (64 * kT) + lane;
 	bool wide = false;
 	for(int c = 0; c < 3; ++c) { wide = wide || !(box[3 + c] - box[c] < 5e7); }
-	// bodies beyond n: copies of the last one, without mass
-	const size_t g0 = i0 - lane < n ? (i0 - lane) / kF32Group * kF32Group : 0;
-	const double4 org = sorted[g0];
+	const size_t w0 = static_cast<size_t>(bi) * kB + static_cast<size_t>(wave) * (64 * kT);   // the wave's first body
+	const size_t within = w0 < n ? w0 / kF32Group * kF32Group : 0;
+	const int mine = run_origin(spread, w0 < n ? w0 : 0, 64 * kT, n);
+	size_t at = n;                  // the body that the offsets are taken from
+	int met = -1;
+	double4 org;
 	float x[kT], y[kT], z[kT], m[kT];
 	double ax[kT], ay[kT], az[kT];
+	// bodies beyond n: copies of the last one, without mass
+	auto place = [&]() {
+		org = sorted[at];
 #pragma unroll
-	for(int t = 0; t < kT; ++t)
-	{
-		const size_t i = i0 + 64 * t;
-		const double4 si = sorted[i < n ? i : n - 1];
-		x[t] = static_cast<float>((si.x - org.x) * kF32Len);
-		y[t] = static_cast<float>((si.y - org.y) * kF32Len);
-		z[t] = static_cast<float>((si.z - org.z) * kF32Len);
-		m[t] = i < n ? static_cast<float>(si.w * kF32Mass) : 0.0f;
-		ax[t] = ay[t] = az[t] = 0.0;
-	}
+		for(int t = 0; t < kT; ++t)
+		{
+			const size_t i = i0 + 64 * t;
+			const double4 si = sorted[i < n ? i : n - 1];
+			x[t] = static_cast<float>((si.x - org.x) * kF32Len);
+			y[t] = static_cast<float>((si.y - org.y) * kF32Len);
+			z[t] = static_cast<float>((si.z - org.z) * kF32Len);
+			m[t] = i < n ? static_cast<float>(si.w * kF32Mass) : 0.0f;
+		}
+	};
+#pragma unroll
+	for(int t = 0; t < kT; ++t) { ax[t] = ay[t] = az[t] = 0.0; }
 	const int first = d0 + static_cast<int>(blockIdx.y) * per;
 	const int last = first + per < d1 ? first + per : d1;
 	for(int d = first; d < last; ++d)
@@ -772,6 +808,17 @@ k_direct_fp32_sym(const double4* __restrict__ sorted, const double* __restrict__
 			const size_t j0 = static_cast<size_t>(bj) * kB + 64 * sub;
 			if(j0 < n)
 			{
+				const int gj = d > 0 ? static_cast<int>(j0 / kF32Near) : -2;
+				if(gj != met)
+				{
+					met = gj;
+					const size_t to = d > 0 ? static_cast<size_t>(nearer(spread, mine, gj)) * kF32Near : within;
+					if(to != at)
+					{
+						at = to;
+						place();
+					}
+				}
 				const size_t j = j0 + lane;
 				const double4 sj = sorted[j < n ? j : n - 1];
 				const float4 f = make_float4(static_cast<float>((sj.x - org.x) * kF32Len),
@@ -902,8 +949,8 @@ k_direct_fp32_sym_sum(const double* __restrict__ y, const uint32_t* __restrict__
 constexpr int kCorrWindow = 32;
 
 __global__ void __launch_bounds__(256)
-k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__ perm, double* __restrict__ f,
-                size_t n, int w, int kb)
+k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__ perm, const float* __restrict__ spread,
+                double* __restrict__ f, size_t n, int w, int kb)
 {
 	const size_t p = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
 	if(p >= n) { return; }
@@ -916,7 +963,12 @@ k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__
 	for(size_t q = q0; q <= q1; ++q)
 	{
 		if(q == p) { continue; }
-		const double4 org = sorted[(q / kb < p / kb ? q : p) / kF32Group * kF32Group];
+		// I's body is that of the lower block: blocks w apart or less are neighbours
+		const size_t lower = q < p ? q : p, upper = q < p ? p : q;
+		const int run = kb / kSymWaves;
+		const double4 org = sorted[q / kb == p / kb ? p / kF32Group * kF32Group :
+		                           static_cast<size_t>(nearer(spread, run_origin(spread, lower / run * run, run, n),
+		                                                      static_cast<int>(upper / kF32Near))) * kF32Near];
 		const double ox = org.x, oy = org.y, oz = org.z;
 		const double4 sj = sorted[q];
 		const double xj = sj.x, yj = sj.y, zj = sj.z, mj = sj.w;
@@ -1049,7 +1101,7 @@ k_morton_keys(const double* __restrict__ y, size_t n, const double* __restrict__
 struct fp32_layout {
 	int kt, nb, span, per;
 	unsigned gbox;
-	size_t off_other, off_acc, off_sorted, off_keys, off_vals, off_counts, off_bpart, off_box, bytes;
+	size_t off_other, off_acc, off_sorted, off_keys, off_vals, off_counts, off_bpart, off_box, off_spread, bytes;
 };
 
 // Sums of one pass take at most this much (a pass has one offset at least): 52 MiB
@@ -1096,7 +1148,8 @@ fp32_layout fp32_plan(const nbh_ctx* ctx, size_t n)
 	l.off_counts = l.off_vals + align(2 * n * sizeof(uint32_t));
 	l.off_bpart = l.off_counts + align(nbh::sort_counts_size(n) * sizeof(uint32_t));
 	l.off_box = l.off_bpart + align(6 * static_cast<size_t>(l.gbox) * sizeof(double));
-	l.bytes = l.off_box + align(6 * sizeof(double));
+	l.off_spread = l.off_box + align(6 * sizeof(double));
+	l.bytes = l.off_spread + align((n + kF32Near - 1) / kF32Near * sizeof(float));
 	return l;
 }
 
@@ -1115,6 +1168,7 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	uint32_t* counts = reinterpret_cast<uint32_t*>(base + l.off_counts);
 	double* bpart = reinterpret_cast<double*>(base + l.off_bpart);
 	double* box = reinterpret_cast<double*>(base + l.off_box);
+	float* spread = reinterpret_cast<float*>(base + l.off_spread);
 	hipLaunchKernelGGL(k_bbox_partial, dim3(l.gbox), dim3(256), 0, ctx->stream, y, n, bpart);
 	NBH_LAUNCHED();
 	hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, ctx->stream, bpart, static_cast<int>(l.gbox), box);
@@ -1124,7 +1178,8 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	NBH_LAUNCHED();
 	uint32_t* perm = nullptr;
 	NBH_TRY(nbh::sort_pairs(ctx, keys, vals, keys + n, vals + n, n, 30, counts, &perm));
-	hipLaunchKernelGGL(k_sorted_copy, dim3(l.gbox), dim3(256), 0, ctx->stream, y, mass, perm, sorted, n);
+	hipLaunchKernelGGL(k_sorted_copy, dim3(static_cast<unsigned>((n + kF32Near - 1) / kF32Near)), dim3(kF32Near), 0,
+	                   ctx->stream, y, mass, perm, sorted, spread, n);
 	NBH_LAUNCHED();
 	const int kb = kSymThreads * l.kt;
 	const int offsets = l.nb / 2 + 1;
@@ -1137,7 +1192,7 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 			hipLaunchKernelGGL(l.kt == 8 ? k_direct_fp32_sym<8> : l.kt == 4 ? k_direct_fp32_sym<4> :
 			                   l.kt == 2 ? k_direct_fp32_sym<2> : k_direct_fp32_sym<1>,
 			                   dim3(static_cast<unsigned>(l.nb), static_cast<unsigned>(rows)), dim3(kSymThreads), 0,
-			                   ctx->stream, sorted, box, own, other, n, l.nb, d0, d1, l.per);
+			                   ctx->stream, sorted, box, spread, own, other, n, l.nb, d0, d1, l.per);
 			NBH_LAUNCHED();
 			hipLaunchKernelGGL(k_direct_fp32_sym_sum, dim3(nbh::grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, y, perm,
 			                   own, other, acc, f, n, kb, l.nb, d0, d1, rows, d0 == 0 ? 1 : 0, d1 == offsets ? 1 : 0);
@@ -1147,7 +1202,7 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	if(precision == NBH_FP32_CORR)
 	{
 		hipLaunchKernelGGL(k_direct_window, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, ctx->stream,
-		                   sorted, perm, f, n, kCorrWindow, kb);
+		                   sorted, perm, spread, f, n, kCorrWindow, kb);
 		NBH_LAUNCHED();
 	}
 	return NBH_OK;

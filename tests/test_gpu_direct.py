@@ -171,6 +171,38 @@ def test_fp32_far_apart_and_clamped(ctx, scale):
     assert np.sqrt(np.mean(rel ** 2)) < FP32_RMS_REL and rel.max() < FP32_MAX_REL
 
 
+# sizes with blocks of 256, 512, 1024 and 2048 bodies
+@pytest.mark.parametrize("n,halo,clump", [(8192, 10.0, 1e-3), (40000, 100.0, 1e-2), (100000, 10.0, 1e-3),
+                                          (200000, 100.0, 1e-2)])
+@pytest.mark.parametrize("prec", [NBH_FP32, NBH_FP32_CORR])
+def test_fp32_clump_in_a_wide_state(ctx, n, halo, clump, prec):
+    """Half the bodies in a clump 10^4 times smaller than the ball around it.  Offsets
+    taken close to the clump leave its pairs a few FP32 roundings (8 x 2^-24 bounds
+    those of offsets, r^2, rsq, products and sums in the median); offsets taken in the ball
+    round at 10^4 x 2^-24 = 6e-4 of the clump's size, and the median of the clump's bodies
+    is then 4e-6 to 2e-4.  The few bodies that share their 1024 with the ball keep such
+    errors, whichever origin the others have: one in a hundred may, no bound on the
+    maximum."""
+    rng = np.random.default_rng(n)
+
+    def ball(k, r):
+        u = rng.standard_normal((3, k))
+        return u * (r * rng.random(k) ** (1 / 3) / np.linalg.norm(u, axis=0))
+
+    k = n // 2
+    pos = np.concatenate([ball(n - k, halo), ball(k, clump) + 1.0], axis=1)
+    order = rng.permutation(n)
+    y = np.concatenate([pos[:, order].reshape(-1), np.zeros(3 * n)])
+    m = rng.uniform(0.5, 1.5, n) / n
+    rel = _rel_err(_run(ctx, y, m, prec), _run(ctx, y, m, NBH_FP64), n)
+    inside = rel[order >= n - k]
+    print(f"\n[fp32] n={n} clump median {np.median(inside):.2e} p99 {np.percentile(inside, 99):.2e}, "
+          f"ball median {np.median(rel[order < n - k]):.2e}")
+    assert np.median(inside) < 8 * 2.0 ** -24
+    assert np.percentile(inside, 99) < halo / clump * 2.0 ** -24
+    assert np.median(rel[order < n - k]) < 8 * 2.0 ** -24
+
+
 def test_fp32_matches_fp64_kernel_large(ctx):
     """At 2^17 bodies (no CPU reference needed) the FP32 tiles agree with the
     FP64 kernel, which is bit-exact with the oracle at every smaller size."""
