@@ -687,9 +687,24 @@ __device__ inline float rot_left(float v)     // lane l gets lane l + 1 (mod 64)
 	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x134, 0xf, 0xf, false));
 }
 
+// Whether coordinates are so large that (1/r)^3 could leave the FP32 range.
+__device__ inline bool box_wide(const double* __restrict__ box)
+{
+	bool wide = false;
+	for(int c = 0; c < 3; ++c) { wide = wide || !(box[3 + c] - box[c] < 5e7); }
+	return wide;
+}
+
+// m / r^3 from q = 1/r.
+template <bool kWide>
+__device__ inline float pair_weight(float m, float q)
+{
+	const float q2 = q * q;
+	return kWide ? (m * q) * q2 : m * (q2 * q);
+}
+
 // 64 bodies of J (js[l], js[l + 64] = body l) against kT bodies per lane: p += what
 // the lane's bodies receive; kReact: r = what body `lane` of J receives.
-// kWide: coordinates so large that (1/r)^3 could leave the FP32 range.
 // kFine: each product goes to the FP64 sums ax by itself.
 template <int kT, bool kReact, bool kWide, bool kFine>
 __device__ inline void sym_block(const float4* js, int lane, const float (&x)[kT], const float (&y)[kT],
@@ -710,9 +725,7 @@ __device__ inline void sym_block(const float4* js, int lane, const float (&x)[kT
 			const float dy = s.y - y[t];
 			const float dz = s.z - z[t];
 			const float q = rsq_clamped(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
-			const float q2 = q * q;
-			const float q3 = q2 * q;
-			const float wj = kWide ? (s.w * q) * q2 : s.w * q3;
+			const float wj = pair_weight<kWide>(s.w, q);
 			if(kFine)
 			{
 				ax[t] += static_cast<double>(dx * wj);
@@ -727,7 +740,7 @@ __device__ inline void sym_block(const float4* js, int lane, const float (&x)[kT
 			}
 			if(kReact)
 			{
-				const float wi = kWide ? (m[t] * q) * q2 : m[t] * q3;
+				const float wi = pair_weight<kWide>(m[t], q);
 				ux = t == 0 ? dx * wi : fmaf(dx, wi, ux);
 				uy = t == 0 ? dy * wi : fmaf(dy, wi, uy);
 				uz = t == 0 ? dz * wi : fmaf(dz, wi, uz);
@@ -764,8 +777,7 @@ k_direct_fp32_sym(const double4* __restrict__ sorted, const double* __restrict__
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int bi = blockIdx.x;
 	const size_t i0 = static_cast<size_t>(bi) * kB + static_cast<size_t>(wave) * (64 * kT) + lane;
-	bool wide = false;
-	for(int c = 0; c < 3; ++c) { wide = wide || !(box[3 + c] - box[c] < 5e7); }
+	const bool wide = box_wide(box);
 	const size_t w0 = static_cast<size_t>(bi) * kB + static_cast<size_t>(wave) * (64 * kT);   // the wave's first body
 	const size_t within = w0 < n ? w0 / kF32Group * kF32Group : 0;
 	const int mine = run_origin(spread, w0 < n ? w0 : 0, 64 * kT, n);
@@ -942,31 +954,32 @@ k_direct_fp32_sym_sum(const double* __restrict__ y, const uint32_t* __restrict__
 // the sources at positions p - w .. p + w (its neighbours along the curve, where
 // the FP32 rounding of the offsets weighs most) are recomputed in FP64 (force
 // law of nbody/nbody_data.cpp:35-44) and in the FP32 tiles' own arithmetic (same
-// origin, scaled units and clamped rsq), and f gets the difference.  kb: bodies
-// per block of the tiles; a pair's origin is that of the body in the lower block,
-// and the target's own inside a block (blocks w apart or less are neighbours, and
-// of two neighbours the lower one is I).
+// origin, scaled units, clamped rsq and form of the weight), and f gets the
+// difference: the term of a pair that stands alone cancels to the last bit.  kb: bodies
+// per block of the tiles; blocks w apart or less are neighbours, and of two neighbours
+// the lower one is I.
 constexpr int kCorrWindow = 32;
 
 __global__ void __launch_bounds__(256)
 k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__ perm, const float* __restrict__ spread,
-                double* __restrict__ f, size_t n, int w, int kb)
+                const double* __restrict__ box, double* __restrict__ f, size_t n, int w, int kb)
 {
 	const size_t p = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
 	if(p >= n) { return; }
 	const uint32_t i = perm[p];
 	const double4 me = sorted[p];
 	const double xi = me.x, yi = me.y, zi = me.z;
+	const bool wide = box_wide(box);
 	double cx = 0.0, cy = 0.0, cz = 0.0;
 	const size_t q0 = p > static_cast<size_t>(w) ? p - w : 0;
 	const size_t q1 = p + w < n - 1 ? p + w : n - 1;
 	for(size_t q = q0; q <= q1; ++q)
 	{
 		if(q == p) { continue; }
-		// I's body is that of the lower block: blocks w apart or less are neighbours
 		const size_t lower = q < p ? q : p, upper = q < p ? p : q;
 		const int run = kb / kSymWaves;
-		const double4 org = sorted[q / kb == p / kb ? p / kF32Group * kF32Group :
+		const bool inside = q / kb == p / kb;
+		const double4 org = sorted[inside ? p / kF32Group * kF32Group :
 		                           static_cast<size_t>(nearer(spread, run_origin(spread, lower / run * run, run, n),
 		                                                      static_cast<int>(upper / kF32Near))) * kF32Near];
 		const double ox = org.x, oy = org.y, oz = org.z;
@@ -980,7 +993,8 @@ k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__
 		const float fy = static_cast<float>((yj - oy) * kF32Len) - static_cast<float>((yi - oy) * kF32Len);
 		const float fz = static_cast<float>((zj - oz) * kF32Len) - static_cast<float>((zi - oz) * kF32Len);
 		const float qf = rsq_clamped(fmaf(fz, fz, fmaf(fy, fy, fx * fx)));
-		const float wf = (static_cast<float>(mj * kF32Mass) * qf) * (qf * qf);
+		const float mf = static_cast<float>(mj * kF32Mass);
+		const float wf = inside || wide ? pair_weight<true>(mf, qf) : pair_weight<false>(mf, qf);
 		cx += dx * c - static_cast<double>(fx * wf);
 		cy += dy * c - static_cast<double>(fy * wf);
 		cz += dz * c - static_cast<double>(fz * wf);
@@ -1202,7 +1216,7 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	if(precision == NBH_FP32_CORR)
 	{
 		hipLaunchKernelGGL(k_direct_window, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, ctx->stream,
-		                   sorted, perm, spread, f, n, kCorrWindow, kb);
+		                   sorted, perm, spread, box, f, n, kCorrWindow, kb);
 		NBH_LAUNCHED();
 	}
 	return NBH_OK;

@@ -239,6 +239,30 @@ def test_fp32_corr_close_pair_far_from_origin(ctx):
     assert ec.max() < 1e-6
 
 
+# blocks of 256, 512, 1024 and 2048 bodies
+@pytest.mark.parametrize("n,kb", [(1024, 256), (24576, 512), (49152, 1024), (163840, 2048)])
+def test_fp32_corr_takes_out_the_tiles_own_terms(ctx, n, kb):
+    """All bodies but two without mass, so that each of the two receives one term: the
+    correction pass must find the tiles' FP32 term to the last bit, for neighbours in one
+    block and in two, and leave the FP64 term (a few roundings of 2^-53; an FP32 term that
+    differs in its last bit leaves 3e-8)."""
+    rng = np.random.default_rng(n)
+    # order along the curve: x, as y and z stay in the first of 1024 cells (the last body
+    # alone sets the box)
+    x = (np.arange(n) + 0.6 * rng.random(n)) / n
+    pos = np.stack([x, 9e-4 * rng.random(n), 9e-4 * rng.random(n)])
+    pos[:, -1] = 1.0
+    y = np.concatenate([pos.reshape(-1), np.zeros(3 * n)])
+    for a, b in [(kb - 1, kb), (2 * kb - 3, 2 * kb + 5), (3 * kb - 1, 3 * kb + 1), (kb + 7, kb + 9), (kb + 63, kb + 64)]:
+        m = np.zeros(n)
+        m[[a, b]] = rng.uniform(0.5, 1.5, 2)
+        f = _run(ctx, y, m, NBH_FP32_CORR)[3 * n:].reshape(3, n)
+        d = pos[:, b] - pos[:, a]
+        w = d / max(d @ d, 1e-8) ** 1.5
+        for got, want in ((f[:, a], m[b] * w), (f[:, b], -m[a] * w)):
+            assert np.linalg.norm(got - want) < 1e-14 * np.linalg.norm(want), (a, b)
+
+
 @pytest.mark.parametrize("kind,n", [("plummer", 32768), ("cube", 16384)])
 def test_fp32_corr_accuracy(ctx, kind, n):
     """With the correction pass the force error against the FP64 kernel drops
