@@ -92,6 +92,69 @@ def test_fp64_large_matches_sampled_targets(ctx, n):
     assert np.array_equal(f[:3 * n], y[3 * n:])
 
 
+def _odd_roots(c, bits):
+    """The odd M with M^2 = c (mod 2^bits), c = 1 (mod 8)."""
+    m = 1
+    for k in range(4, bits + 1):            # M^2 = c (mod 2^(k - 1)) -> (mod 2^k)
+        if (m * m - c) % (1 << k):
+            m += 1 << (k - 2)
+    half = 1 << (bits - 1)
+    return {r % (1 << bits) for r in (m, -m, m + half, half - m)}
+
+
+def _hard_operands(count):
+    """(r^2, -a) whose root and whose quotient a / (r^2 sqrt(r^2)) lie next to the middle
+    of two doubles: r^2 = (M^2 - c) / 2^s with M odd of 54 bits, and a = (Q B - r) / 2^54
+    with Q odd of 54 bits and B the denominator's significand, small odd c and r.  The
+    root's last step multiplies by 1 / (2 sqrt(x)) (1 + d), |d| <= 1.5 (2^-24.18)^2 =
+    2^-47.8 from v_rsq_f64's error, so a root M - c / (2 M) is sure to round right where
+    |c| / 2^54 > |d|: |c| > 75."""
+    rng = np.random.default_rng(1)
+    r2 = []
+    for k in [k for k in range(-1000, 1000) if abs(8 * k + 1) > 75]:
+        for s in (54, 55):
+            for m in _odd_roots(8 * k + 1, s):
+                t = m * m - (8 * k + 1) >> s
+                if m >> 53 == 1 and t >> 52 == 1:
+                    # t 2^s has the root M: an even power of two leaves it as hard
+                    r2.append(np.ldexp(float(t), s % 2 - 52 + 2 * int(rng.integers(-10, 20))))
+    r2 = np.array(r2[:count // 2])
+    r2 = np.concatenate([r2, 10.0 ** rng.uniform(-7, 12, count - len(r2))])
+    a = np.empty(count)
+    for i, b in enumerate(r2 * np.sqrt(r2)):
+        b = int(np.ldexp(np.frexp(b)[0], 53))
+        while b % 2 == 0:
+            b >>= 1
+        inv = pow(b, -1, 1 << 54)
+        for r in range(1, 100, 2):
+            q = (r if i % 2 else -r) * inv % (1 << 54)
+            if q >> 53 == 1:
+                break
+        a[i] = np.ldexp(float(q * b - (r if i % 2 else -r) >> 54), -52)
+    return r2, a
+
+
+# terms through LDS, in turns and a target per work-item
+@pytest.mark.parametrize("n", [4001, 20011, 1 << 18])
+def test_fp64_quotients_next_to_midpoints(ctx, n):
+    """The bare root and quotient round as IEEE's where that is hardest.  Body 0 is so
+    heavy that every other body's sum is the one term it receives from it."""
+    r2, a = (v[np.arange(n - 1) % len(v)] for v in _hard_operands(min(n - 1, 20010)))
+    # RN(dx^2) + RN(dy^2) = r^2: dx from below, dy^2 the few ulps that are missing
+    dx = np.sqrt(r2) * (1 - 2.0 ** -51)
+    dy = np.sqrt(r2 - dx * dx)
+    keep = dx * dx + dy * dy == r2
+    assert keep.mean() > 0.99
+    heavy = 2.0 ** 190
+    y = np.zeros((6, n))
+    y[0, 1:], y[1, 1:] = dx, dy
+    m = np.concatenate([[heavy], a * 2.0 ** -150])
+    f = _run(ctx, y.reshape(-1), m, NBH_FP64)[3 * n:].reshape(3, n)[:, 1:]
+    coeff = (-m[1:] * heavy) / (r2 * np.sqrt(r2))
+    for got, d in ((f[0], dx), (f[1], dy)):
+        assert np.array_equal(got[keep], ((d * coeff) / m[1:])[keep])
+
+
 def test_fp64_clamp_and_coincident(ctx):
     """Pairs closer than 1e-4 use r^2 = 1e-8; coincident bodies contribute 0."""
     pos = np.array([[0, 0, 0], [1e-5, 0, 0], [1e-5, 0, 0], [1, 2, 3]], dtype=np.float64)
