@@ -2043,9 +2043,9 @@ k_bh_walk64(const double4* __restrict__ xyzr, const double* __restrict__ nmass, 
 	const double gm8 = 8.0 * gm1;
 	const bool all_safe =
 	    __ballot(!(coord_in_range(me.x) && coord_in_range(me.y) && coord_in_range(me.z) && mass_in_range(gm1))) == 0;
-	// box of the bodies (lanes without one repeat the first); it says nothing of a
-	// body that is not a number
-	const bool box_holds = __ballot(!(me.x == me.x && me.y == me.y && me.z == me.z)) == 0;
+	// box of the bodies (lanes without one repeat the first); it says nothing of a body
+	// that is not a number or infinite, whose offset from a node may be no number
+	const bool box_holds = __ballot(!(isfinite(me.x) && isfinite(me.y) && isfinite(me.z))) == 0;
 	double3 lo = make_double3(me.x, me.y, me.z), hi = lo;
 	for(int off = 16; off > 0; off >>= 1)
 	{

@@ -189,6 +189,25 @@ def test_traverse_fp64_edges_bit_exact(ctx, n, ratio):
     t.close()
 
 
+@pytest.mark.parametrize("n", [64, 2048])
+@pytest.mark.parametrize("ratio", [0.5, 2.0])
+def test_traverse_fp64_infinite_coordinates(ctx, n, ratio):
+    """Bodies that have run away: differences of infinities are no numbers, which pass no
+    test, so that a body's finite components and its NaNs are the oracle's."""
+    y, m = _state("ball", n, 60 + n)
+    y[[5, 9, n // 2]] = np.inf
+    y[n + 21] = -np.inf
+    dy, dm = ctx.put(y), ctx.put(m)
+    t = GpuTree(ctx, n)
+    t.build(dy, dm, ratio)
+    h = oracle_lib.Heap(n)
+    h.build(y, m, ratio)
+    f0 = h.fcompute(y, m, LAYOUT["heap_stackless"], 1)
+    assert np.isfinite(f0.reshape(6, n)[5]).all()
+    assert np.array_equal(t.fcompute(dy, dm, LAYOUT["heap_stackless"]), f0, equal_nan=True)
+    t.close()
+
+
 def test_traverse_fp64_coincident_bodies(ctx):
     """No node is ever taken: every body's walk reaches every leaf, and f is 0."""
     n = 128
