@@ -125,8 +125,9 @@ nbh_status nbh_clamp(nbh_ctx* ctx, double* y, size_t nbodies, double b);
    (nbody_engine_cuda_impl.cu:10-124; host nbody/nbody_engine_cuda.cpp:202-247).
    NBH_FP64 reproduces nbody_engine_simple::fcompute (nbody_engine_simple.cpp:116-173)
    operation for operation.  block_size: work-group size of the FP64 kernel
-   that gives every target a work-item (2^18 bodies and more on 256 CUs;
-   64..1024, multiple of 64), 0 = default. */
+   that gives every target a work-item (above 2^18 bodies on 256 CUs, and below,
+   down to 2^16, where its waves fill the SIMDs evenly; 64..1024, multiple of 64),
+   0 = default. */
 nbh_status nbh_fcompute_direct(nbh_ctx* ctx, const double* y, const double* mass, double* f,
                                size_t n, nbh_precision precision, int block_size);
 

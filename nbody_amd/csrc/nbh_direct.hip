@@ -1222,6 +1222,22 @@ nbh_status fp32_run(nbh_ctx* ctx, const double* y, const double* mass, double* f
 	return NBH_OK;
 }
 
+// Whether n bodies (more than the split form takes) get a target per lane rather than
+// turns.  A target per lane takes a whole pass over the sources for every wave that the
+// busiest SIMD has, so it wins where those waves are nearly all there: 20.3 ms against
+// 22.3 at 2^17 bodies (two waves per SIMD on 256 CUs), 45.1 against 50.2 at 196608 and 77.3
+// against 88.2 at 2^18; just above, 30.8 against 26.3, 58.3 against 53.9 and 95.6 against
+// 93.5.  The two meet at 0.82 to 0.89 of the targets that the waves could hold (108000 to
+// 116000, 168000 to 175000 and 224000 to 230000 bodies; work-groups of 256 and 64).  With one wave per SIMD turns are never slower (65536: 5.7 ms
+// both), and beyond four a target per lane loses 2% at most.
+bool fp64_lane_targets(size_t n, size_t bs, size_t cus)
+{
+	const size_t per_wave = 4 * 64 * cus;                             // targets of one wave on every SIMD
+	const size_t groups = ((n + bs - 1) / bs + cus - 1) / cus;        // of the busiest CU
+	const size_t waves = (groups * bs + 255) / 256;                   // of its busiest SIMD
+	return n > 4 * per_wave || (n > per_wave && 8 * n >= 7 * waves * per_wave);
+}
+
 }  // namespace
 
 extern "C" nbh_status nbh_direct_sample(nbh_ctx* ctx, const double* y, const double* mass, size_t n,
@@ -1252,18 +1268,15 @@ extern "C" nbh_status nbh_fcompute_direct(nbh_ctx* ctx, const double* y, const d
 		          "block_size %d: must be a multiple of 64 in [64, 1024]", block_size);
 		const bool simple = precision == NBH_FP64;
 		nbh::scoped_timer timer(ctx, simple ? "direct_fp64" : "direct_fp64_block");
-		// split terms while every work-group gets a CU of its own; a target per lane
-		// once that gives every SIMD four waves (turns and a target per lane: 21.7 and
-		// 20.6 ms at 2^17, 33.2 and 36.9 at 150000, 57.7 and 63.3 at 200000, 95.8 and
-		// 84.8 at 2^18); turns between
 		const size_t cus = static_cast<size_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
+		// split terms while every work-group gets a CU of its own
 		if(n <= kSplitTgt * cus)
 		{
 			hipLaunchKernelGGL(simple ? k_direct_fp64_split<kLawSimple> : k_direct_fp64_split<kLawBlock>,
 			                   dim3(static_cast<unsigned>((n + kSplitTgt - 1) / kSplitTgt)), dim3(kSplitThreads), 0,
 			                   ctx->stream, y, mass, f, n);
 		}
-		else if(n < 4 * 4 * 64 * cus)
+		else if(!fp64_lane_targets(n, static_cast<size_t>(bs), cus))
 		{
 			hipLaunchKernelGGL(simple ? k_direct_fp64_turns<kLawSimple> : k_direct_fp64_turns<kLawBlock>,
 			                   dim3(static_cast<unsigned>((n + kTurnTgt - 1) / kTurnTgt)), dim3(kTurnThreads), 0,

@@ -78,10 +78,11 @@ def test_fp64_bit_exact_at_tile_edges(ctx, n, law):
     assert np.array_equal(f, f0)
 
 
-@pytest.mark.parametrize("n", [131071, 262143, 262144])
+@pytest.mark.parametrize("n", [114687, 114689, 131071, 131073, 172032, 229375, 229376, 262143, 262144])
 def test_fp64_large_matches_sampled_targets(ctx, n):
-    """On both sides of the last switch (2^18 bodies on 256 CUs) against the
-    per-target sums of nbh_direct_sample, which keeps the same order."""
+    """On both sides of the switches between turns and a target per work-item (7/8 of two,
+    three and four waves per SIMD, and above, on 256 CUs) against the per-target sums of
+    nbh_direct_sample, which keeps the same order."""
     y, m = _state("plummer", n, 9)
     idx = np.unique(np.concatenate([np.arange(0, n, 4099), [n - 2, n - 1]])).astype(np.uint32)
     dy, dm, df, di, da = ctx.put(y), ctx.put(m), ctx.alloc(6 * n), ctx.put_raw(idx), ctx.alloc(3 * len(idx))
