@@ -89,10 +89,11 @@ def test_build_bit_exact(ctx, kind, n):
 
 
 @pytest.mark.parametrize("ties", [False, True])
-@pytest.mark.parametrize("n", [4, 8, 2048, 8192, 16384, 1 << 23])
+@pytest.mark.parametrize("n", [4, 8, 2048, 8192, 16384, 1 << 23, 1 << 24])
 def test_build_split_edges(ctx, n, ties):
     """Segments split in LDS alone, one and two levels above it, and segments of more
-    tiles than a tile sums itself (2^23): every level's segments hold their lower half
+    tiles than a tile sums itself, whose counts one work-group scans (2^23) or several do
+    (2^24): every level's segments hold their lower half
     first along its axis, equal coordinates by body index, and each body once."""
     rng = np.random.default_rng(n)
     pos = rng.integers(0, 50, size=(3, n)).astype(np.float64) if ties else rng.random((3, n))

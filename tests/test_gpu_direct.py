@@ -49,6 +49,7 @@ def _run(ctx, y, m, prec, bs=0):
     return df.read()
 
 
+# (up to 4096 bodies on 256 CUs the work-group size is checked and chooses nothing)
 @pytest.mark.parametrize("n,bs", [(1, 0), (7, 64), (100, 128), (1000, 256), (1024, 64), (1500, 1024)])
 def test_fp64_bit_exact(ctx, n, bs):
     y, m = _state("ball", n, 11 + n)
@@ -156,6 +157,40 @@ def test_fp64_quotients_next_to_midpoints(ctx, n):
         assert np.array_equal(got[keep], ((d * coeff) / m[1:])[keep])
 
 
+def _sampled_sums(y, m, idx, law):
+    """Accelerations of bodies idx, terms added in index order (cumsum adds in order)."""
+    n = len(m)
+    pos = y[:3 * n].reshape(3, n)
+    out = np.empty((3, len(idx)))
+    for k, i in enumerate(idx):
+        d = pos[:, i, None] - pos
+        r2 = np.maximum(d[0] * d[0] + d[1] * d[1] + d[2] * d[2], 1e-8)
+        if law == NBH_FP64:
+            c = (-1.0 * m[i] * m) / (r2 * np.sqrt(r2))
+            c[i] = 0.0                                     # the self pair is left out: its term is a zero
+            out[:, k] = [np.cumsum(np.concatenate([[0.0], d[a] * c]))[-1] / m[i] for a in range(3)]
+        else:
+            c = m / (np.sqrt(r2) * r2)
+            out[:, k] = [np.cumsum(np.concatenate([[0.0], -(d[a] * c)]))[-1] for a in range(3)]
+    return out
+
+
+# a target per work-item: two waves on every SIMD of 256 CUs nearly full (work-groups of
+# 64, 128, 256: 118011 bodies), and more than four (every work-group size: above 2^18)
+@pytest.mark.parametrize("n,bs", [(118011, 0), (118011, 64), (118011, 128), (131072, 256), (262144 + 77, 512),
+                                  (262144 + 77, 1024), (262144 + 1, 64), (262144 + 3, 192)])
+@pytest.mark.parametrize("law", [NBH_FP64, NBH_FP64_BLOCK])
+def test_fp64_target_per_lane_bit_exact(ctx, n, bs, law):
+    """Ragged last work-groups and tiles of every size, both laws, and bodies and tiles
+    with operands out of the bare sequences' range."""
+    y, m = _edge_state(n)
+    m[n // 5] = 1e70
+    idx = np.array([0, 1, 63, 64, n // 3, n // 2, n // 5, n // 5 + 1, n - 3, n - 2, n - 1, 255, 256, 1023, 1024, 77777])
+    f = _run(ctx, y, m, law, bs)
+    assert np.array_equal(f[:3 * n], y[3 * n:])
+    assert np.array_equal(f[3 * n:].reshape(3, n)[:, idx], _sampled_sums(y, m, idx, law))
+
+
 def test_fp64_clamp_and_coincident(ctx):
     """Pairs closer than 1e-4 use r^2 = 1e-8; coincident bodies contribute 0."""
     pos = np.array([[0, 0, 0], [1e-5, 0, 0], [1e-5, 0, 0], [1, 2, 3]], dtype=np.float64)
@@ -219,7 +254,10 @@ def test_fp32_block_edges(ctx, n):
     assert np.array_equal(f, _run(ctx, y, m, NBH_FP32))      # the same bits again
     fc = _run(ctx, y, m, NBH_FP32_CORR)
     if n > 1:
-        assert _rel_err(fc, f64, n).mean() <= 1.5 * _rel_err(f, f64, n).mean()
+        e, ec = _rel_err(f, f64, n), _rel_err(fc, f64, n)
+        assert ec.mean() <= 1.5 * e.mean()
+        if n > 64:                 # beyond the window of 32 on either side
+            assert np.sqrt(np.mean(ec ** 2)) < np.sqrt(np.mean(e ** 2)) and ec.max() <= e.max()
 
 
 @pytest.mark.parametrize("scale", [1e-3, 1e9])
@@ -327,7 +365,8 @@ def test_fp32_corr_takes_out_the_tiles_own_terms(ctx, n, kb):
             assert np.linalg.norm(got - want) < 1e-14 * np.linalg.norm(want), (a, b)
 
 
-@pytest.mark.parametrize("kind,n", [("plummer", 32768), ("cube", 16384)])
+# blocks of 512, 256, 1024 and 2048 bodies
+@pytest.mark.parametrize("kind,n", [("plummer", 32768), ("cube", 16384), ("cube", 65537), ("plummer", 200003)])
 def test_fp32_corr_accuracy(ctx, kind, n):
     """With the correction pass the force error against the FP64 kernel drops
     below that of the FP32 tiles alone (largest and RMS relative error)."""

@@ -34,6 +34,8 @@ def _state(kind, n, seed):
     return oracle_lib.state_from_data(_data(kind, n, seed))
 
 
+# (up to 4096 bodies on 256 CUs the work-group size is checked and chooses nothing; the
+# form that uses it is tested in test_gpu_direct.py)
 @pytest.mark.parametrize("n,bs", [(1, 0), (64, 64), (100, 128), (1000, 256), (1536, 1024), (4096, 0)])
 def test_block_bit_exact(ctx, n, bs):
     y, m = _state("plummer", n, 21 + n)
