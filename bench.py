@@ -3,7 +3,7 @@
 
 Workload (the direct-sum configuration the metric is quoted on): N = 262144
 bodies of a Plummer sphere (scale radius 1, total mass 1, seed 2), FP64 state,
-FP32 force tiles with compensated accumulation, driven by the Dormand-Prince
+FP32 force tiles summed block by block in FP64, driven by the Dormand-Prince
 5(4) solver (rkdp) with error_threshold 1e-9 and dt = 1e-3.  A step is one
 rkdp advise(); the adaptive rule may split it into 8 substeps (one level, so a
 step costs 7 or 63 force evaluations).  value = N^2 pair interactions per
@@ -727,6 +727,28 @@ def copy_probe() -> int:
     return 0
 
 
+# What the printed line keeps of a Barnes-Hut run, and what it leaves out elsewhere;
+# --details has all of it.
+RUN_KEYS = ("variant", "steps_per_s", "walk_ms", "rms_max_over_seeds")
+LEFT_OUT = ("rms", "p99", "plain_rms", "plain_p99", "rms_by_seed", "p99_max_over_seeds",
+            "plain_theta_0.5_p99_max_over_seeds")
+LINE_BYTES = 9000       # a record of a run may hold only the last 10 kB of its output
+
+
+def bench_line(out: dict) -> str:
+    """`out` as the one line to print: five significant digits below the top level,
+    and of the Barnes-Hut runs the main figures."""
+    def short(v):
+        if isinstance(v, float):
+            return float(f"{v:.5g}")
+        if isinstance(v, dict):
+            keep = RUN_KEYS if "ms_per_step" in v else [k for k in v if k not in LEFT_OUT]
+            return {k: short(v[k]) for k in keep if k in v}
+        return [short(w) for w in v] if isinstance(v, list) else v
+
+    return json.dumps({k: v if isinstance(v, float) else short(v) for k, v in out.items()}, separators=(",", ":"))
+
+
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("--gpus", type=int, default=1)
@@ -752,6 +774,8 @@ def main(argv=None) -> int:
                     help="split-precision force precisions (default: all three)")
     ap.add_argument("--split-stream", default="", metavar="BASE",
                     help="run the split-precision workload in chunks through frame streams BASE_<solver>_<prec>")
+    ap.add_argument("--details", default="", metavar="FILE",
+                    help="also write everything that was measured, unrounded, as JSON")
     ap.add_argument("--pmc-probe", action="store_true",
                     help="only launch the kernels measured by the hardware-counter runs, then exit")
     ap.add_argument("--bh-probe", metavar="VARIANT",
@@ -920,7 +944,9 @@ def main(argv=None) -> int:
         out["split_precision"] = split_precision_run(
             1 << 16, a.split_precision, tuple(a.split_solver or ("rkfeagin10", "bs")),
             tuple(a.split_prec or ("fp64", "fp32", "fp32_corr")), a.split_stream)
-    print(json.dumps(out), flush=True)
+    if a.details:
+        Path(a.details).write_text(json.dumps(out) + "\n")
+    print(bench_line(out), flush=True)
     return 0
 
 
