@@ -2842,7 +2842,7 @@ constexpr float kSuperNearMin = 5.0f;
 // The tree a group walk runs on.  Heap (child == nullptr): children of node k
 // are 2k and 2k + 1, and the walk groups and super-groups are the heap nodes
 // of 64 and 1024 bodies.  Morton tree: the children of internal id k are
-// child[k]; group g is grp[g] = (node id, first sorted leaf, leaves (<= 64),
+// child[k]; group g is grp[g] = (node id, first sorted leaf, leaves (<= kRadixWalk),
 // super-group or -1) and super-group s is sup[s] = (node id, first leaf).  In
 // both, a group's or super-group's box is its node's box.
 struct WalkTree {
