@@ -35,8 +35,8 @@ __device__ inline void keep_order()
 // 1 / (2 sqrt(x)) to 2^-46, so h^3 is the reciprocal of b8 = 8 x sqrt(x) to 2^-44
 // and one Newton step (error squared, 2^-88) leaves the same rounded reciprocal
 // as two from v_rcp_f64's 2^-24 (2^-96); the quotient and its correction are the
-// general ones.  Measured on 2.5e10 random and hard operands: the bits of the
-// general sequences; 106 clocks at four waves per SIMD against 114 with the
+// general ones.  In a throw-away kernel 2.5e10 random and hard operands gave the bits
+// of the general sequences; 106 clocks at four waves per SIMD against 114 with the
 // reciprocal.  Every step runs for all N before the next: an FP64 result is ready
 // about 16 clocks after its issue and an FP64 instruction issues every 4.5, but
 // left alone the scheduler runs one chain after the other.

@@ -1916,10 +1916,10 @@ __device__ inline void write_f(const double* __restrict__ y, const double* __res
 // A body per lane, each on its own way through the tree, spent its time on gathers,
 // divergent branches and the general quotient and root: 252 us at 1024 bodies, 1.56
 // ms at 16384, 3.8 at 65536, 7.6 at 2^17 and 313 at 2^20 (ratio 2) against 90 us,
-// 0.44, 1.49, 3.9 and 72 ms.  At 2^17 bodies the VALU is then busy 62% of the time,
-// three quarters of that with the terms.  Without the box test it took 5.0 ms;
-// four terms in flight at two or three waves per SIMD 4.1 and 4.8 (spills), four
-// entries per half 4.0.
+// 0.44, 1.49, 3.9 and 72 ms.  At 2^17 bodies a SIMD then issues 0.155 VALU
+// instructions a clock (0.22 is the most for FP64), some 60% of them the terms'.
+// Without the box test it took 5.0 ms; four terms in flight at two or three waves per
+// SIMD 4.1 and 4.8 (spills), four entries per half 4.0.
 constexpr int kWalkTgt = 32;
 constexpr int kWalkEntries = 64;
 constexpr int kWalkPer = 8;
