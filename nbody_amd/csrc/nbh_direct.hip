@@ -965,6 +965,7 @@ k_direct_fp32_sym_sum(const double* __restrict__ y, const uint32_t* __restrict__
 // per block of the tiles; blocks w apart or less are neighbours, and of two neighbours
 // the lower one is I.
 constexpr int kCorrWindow = 32;
+static_assert(kCorrWindow <= 64, "a window reaches into one run of a block");
 
 __global__ void __launch_bounds__(256)
 k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__ perm, const float* __restrict__ spread,
@@ -976,19 +977,32 @@ k_direct_window(const double4* __restrict__ sorted, const uint32_t* __restrict__
 	const double4 me = sorted[p];
 	const double xi = me.x, yi = me.y, zi = me.z;
 	const bool wide = box_wide(box);
-	double cx = 0.0, cy = 0.0, cz = 0.0;
 	const size_t q0 = p > static_cast<size_t>(w) ? p - w : 0;
 	const size_t q1 = p + w < n - 1 ? p + w : n - 1;
+	// The window reaches into one run and one 256 of the block below, where it is J, and of
+	// the block above, where it is I: an origin for each.
+	const size_t b0 = p / kb * kb, b1 = b0 + kb;
+	const int run = kb / kSymWaves;
+	const double4 own = sorted[p / kF32Group * kF32Group];
+	double4 below = own, above = own;
+	if(q0 < b0)
+	{
+		below = sorted[static_cast<size_t>(nearer(spread, run_origin(spread, (b0 - 1) / run * run, run, n),
+		                                          static_cast<int>(b0 / kF32Near))) * kF32Near];
+	}
+	if(q1 >= b1)
+	{
+		above = sorted[static_cast<size_t>(nearer(spread, run_origin(spread, p / run * run, run, n),
+		                                          static_cast<int>(b1 / kF32Near))) * kF32Near];
+	}
+	double cx = 0.0, cy = 0.0, cz = 0.0;
 	for(size_t q = q0; q <= q1; ++q)
 	{
 		if(q == p) { continue; }
-		const size_t lower = q < p ? q : p, upper = q < p ? p : q;
-		const int run = kb / kSymWaves;
-		const bool inside = q / kb == p / kb;
-		const double4 org = sorted[inside ? p / kF32Group * kF32Group :
-		                           static_cast<size_t>(nearer(spread, run_origin(spread, lower / run * run, run, n),
-		                                                      static_cast<int>(upper / kF32Near))) * kF32Near];
-		const double ox = org.x, oy = org.y, oz = org.z;
+		const bool lower = q < b0, upper = q >= b1, inside = !lower && !upper;
+		const double ox = lower ? below.x : upper ? above.x : own.x;
+		const double oy = lower ? below.y : upper ? above.y : own.y;
+		const double oz = lower ? below.z : upper ? above.z : own.z;
 		const double4 sj = sorted[q];
 		const double xj = sj.x, yj = sj.y, zj = sj.z, mj = sj.w;
 		const double dx = xj - xi, dy = yj - yi, dz = zj - zi;
